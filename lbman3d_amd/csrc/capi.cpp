@@ -391,22 +391,22 @@ int run_qtensor(lbm_solver* s, KernelRecorder* rec) {
     hipStream_t st = s->stream;
     if (s->fp64) {
         if (rec) rec->begin("qstep_f64");
-        launch_qstep(s->d64, s->bc64, s->k64, s->V, st);
+        launch_qstep(s->d64, s->bc64, s->k64, st);
         if (rec) rec->end();
         swap_q(s->d64);
         if (s->k64.force_full) {
             if (rec) rec->begin("force_f64");
-            launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, s->V, FL_FORCE | FL_STORE_F, 0, st);
+            launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, FL_FORCE | FL_STORE_F, 0, st);
             if (rec) rec->end();
         }
     } else {
         if (rec) rec->begin("qstep_f32");
-        launch_qstep(s->d32, s->bc32, s->k32, s->V, st);
+        launch_qstep(s->d32, s->bc32, s->k32, st);
         if (rec) rec->end();
         swap_q(s->d32);
         if (s->k32.force_full) {
             if (rec) rec->begin("force_f32");
-            launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, s->V, FL_FORCE | FL_STORE_F, 0, st);
+            launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, FL_FORCE | FL_STORE_F, 0, st);
             if (rec) rec->end();
         }
     }
@@ -418,12 +418,12 @@ int run_lbm(lbm_solver* s, KernelRecorder* rec) {
     hipStream_t st = s->stream;
     if (s->fp64) {
         if (rec) rec->begin("lbm_f64");
-        launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, s->V, FL_LBM | FL_STORE_RHO, s->pulled, st);
+        launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, FL_LBM | FL_STORE_RHO, s->pulled, st);
         if (rec) rec->end();
         swap_g(s->d64);
     } else {
         if (rec) rec->begin("lbm_f32");
-        launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, s->V, FL_LBM | FL_STORE_RHO, s->pulled, st);
+        launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, FL_LBM | FL_STORE_RHO, s->pulled, st);
         if (rec) rec->end();
         swap_g(s->d32);
     }
@@ -457,12 +457,14 @@ int run_step(lbm_solver* s, bool last, KernelRecorder* rec) {
         swap_u(s->d64);
     } else if (s->fp64) {
         if (rec) rec->begin("qstep_f64");
-        launch_qstep(s->d64, s->bc64, s->k64, s->V, st);
+        launch_qstep(s->d64, s->bc64, s->k64, st);
         if (rec) rec->end();
         swap_q(s->d64);
         if (rec) rec->begin("force_lbm_f64");
-        launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, s->V, FL_FORCE | FL_LBM | FL_STORE_F | FL_STORE_RHO,
-                                        s->pulled, st);
+        // Steps between downloads keep the force and (without a moving wall,
+        // whose slots read it) the density to themselves: 4 of 80 values.
+        const int flags = FL_FORCE | FL_LBM | (last ? FL_STORE_F : 0) | (last || s->moving ? FL_STORE_RHO : 0);
+        launch_force_lbm<double, false>(s->d64, s->bc64, s->k64, flags, s->pulled, st);
         if (rec) rec->end();
         swap_g(s->d64);
     } else {
@@ -477,12 +479,12 @@ int run_step(lbm_solver* s, bool last, KernelRecorder* rec) {
             swap_u(s->d32);
         } else {
             if (rec) rec->begin("qstep_f32");
-            launch_qstep(s->d32, s->bc32, s->k32, s->V, st);
+            launch_qstep(s->d32, s->bc32, s->k32, st);
             if (rec) rec->end();
             swap_q(s->d32);
             const int flags = FL_FORCE | FL_LBM | (aux ? (FL_STORE_F | FL_STORE_RHO) : 0);
             if (rec) rec->begin("force_lbm_f32");
-            launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, s->V, flags, s->pulled, st);
+            launch_force_lbm<float, true>(s->d32, s->bc32, s->k32, flags, s->pulled, st);
             if (rec) rec->end();
             swap_g(s->d32);
         }
@@ -590,14 +592,31 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
     int r = s->fp64 ? alloc_fields(s, s->d64) : alloc_fields(s, s->d32);
     if (r) return cleanup(r);
     void* p = nullptr;
-    if (hipMalloc(&p, table.size() * sizeof(uint16_t)) != hipSuccess)
+    // Slot rows padded to kSlotRow entries, then (moving walls) e_j . u_wall
+    // per face and slot in the handle's type.
+    const size_t slot_bytes = kClasses * kSlotRow * sizeof(uint16_t);
+    std::vector<char> wall_tables(slot_bytes + 6 * kSlotRow * s->esize(), 0);
+    for (int cls = 0; cls < kClasses; ++cls)
+        std::memcpy(&wall_tables[cls * kSlotRow * sizeof(uint16_t)], &table[cls * kQ], kQ * sizeof(uint16_t));
+    s->bc64 = make_bc<double>(*cfg);
+    s->bc32 = make_bc<float>(*cfg);
+    auto fill_dots = [&](auto* dot, const auto& bc) {
+        for (int face = 0; face < 6; ++face)
+            for (int j = 0; j < kQ; ++j)
+                dot[face * kSlotRow + j] = cx(j) * bc.wall_u[face][0] + cy(j) * bc.wall_u[face][1] + cz(j) * bc.wall_u[face][2];
+    };
+    if (s->fp64) fill_dots((double*)&wall_tables[slot_bytes], s->bc64);
+    else fill_dots((float*)&wall_tables[slot_bytes], s->bc32);
+    if (hipMalloc(&p, wall_tables.size()) != hipSuccess)
         return cleanup(fail(LBM_ERR_HIP, "hipMalloc(slot table) failed"));
     s->allocs.push_back(p);
-    s->slots = (uint16_t*)p;
-    if (hipMemcpy(p, table.data(), table.size() * sizeof(uint16_t), hipMemcpyHostToDevice) != hipSuccess)
+    if (hipMemcpy(p, wall_tables.data(), wall_tables.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(LBM_ERR_HIP, "slot table upload failed"));
-    s->d64.slots = s->slots;
-    s->d32.slots = s->slots;
+    s->d64.slots = s->d32.slots = (const uint16_t*)p;
+    if (s->moving) {
+        s->d64.wdot = (const double*)((char*)p + slot_bytes);
+        s->d32.wdot = (const float*)((char*)p + slot_bytes);
+    }
     if (hipMalloc(&p, 3 * s->V * sizeof(double)) != hipSuccess) return cleanup(fail(LBM_ERR_HIP, "hipMalloc failed"));
     s->allocs.push_back(p);
     s->uprev = (double*)p;
@@ -608,8 +627,6 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
     s->allocs.push_back(p);
     s->partials = (double*)p;
     s->diag_out = s->partials + s->diag_blocks * 10;
-    s->bc64 = make_bc<double>(*cfg);
-    s->bc32 = make_bc<float>(*cfg);
     s->bc32.slots_xy = s->bc64.slots_xy = slots_independent_of_z(*cfg, table) ? 1 : 0;
     s->k64 = make_phys<double>(*cfg);
     s->k32 = make_phys<float>(*cfg);
@@ -754,8 +771,8 @@ int lbm_download_populations(lbm_handle s, double* f) {
     const long V = s->V;
     void* tmp = nullptr;
     HIPCHK(hipMalloc(&tmp, kQ * s->vs * s->esize()));
-    if (s->fp64) launch_stream_only(s->d64, s->bc64, V, s->pulled, (double*)tmp, s->stream);
-    else launch_stream_only(s->d32, s->bc32, V, s->pulled, (float*)tmp, s->stream);
+    if (s->fp64) launch_stream_only(s->d64, s->bc64, s->pulled, (double*)tmp, s->stream);
+    else launch_stream_only(s->d32, s->bc32, s->pulled, (float*)tmp, s->stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         (void)hipFree(tmp);

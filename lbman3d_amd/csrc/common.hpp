@@ -49,6 +49,7 @@ enum : int { UB_PERIODIC = 0, UB_NOSLIP = 1, UB_MOVING = 2, UB_SPECULAR = 3 };
 // Entry bits: [1:0] kind, [5:2] source direction, [8:6] face.
 enum : int { SLOT_STREAM = 0, SLOT_BOUNCE = 1, SLOT_MIRROR = 2 };
 constexpr int kClasses = 64;
+constexpr int kSlotRow = 16;   // entries per class in device memory (32 bytes: two vector loads)
 __host__ __device__ inline int slot_kind(uint16_t e) { return e & 3; }
 __host__ __device__ inline int slot_src(uint16_t e) { return (e >> 2) & 15; }
 __host__ __device__ inline int slot_face(uint16_t e) { return (e >> 6) & 7; }
@@ -60,6 +61,20 @@ __host__ __device__ inline int node_class(int x, int y, int z, int nx, int ny, i
     const int b = (y == 0 ? 1 : 0) | (y == ny - 1 ? 2 : 0);
     const int c = (z == 0 ? 1 : 0) | (z == nz - 1 ? 2 : 0);
     return a | (b << 2) | (c << 4);
+}
+
+// Quotient of n < 2^31 by a fixed divisor as a multiply and a shift: with
+// l = ceil(log2 d) and m = ceil(2^(31 + l) / d) the error of n m / 2^(31 + l)
+// stays below 1 / d.
+struct FastDiv {
+    uint32_t mul, shift, one;
+    __device__ __forceinline__ unsigned div(unsigned n) const { return one ? n : __umulhi(n, mul) >> shift; }
+};
+inline FastDiv fast_div(unsigned d) {
+    if (d <= 1) return {0, 0, 1};
+    unsigned l = 1;
+    while ((1ull << l) < d) ++l;
+    return {(uint32_t)(((1ull << (31 + l)) + d - 1) / d), l - 1, 0};
 }
 
 // Boundary description handed to every kernel by value.
@@ -99,7 +114,8 @@ struct Fields {
     T* rho;         // density, stored as rho - BCDesc::rho_base
     T* g;           // populations, source buffer   [15][vs]
     T* gn;          // populations, destination     [15][vs]
-    const uint16_t* slots;  // [kClasses][15] pull-slot table
+    const uint16_t* slots;  // [kClasses][kSlotRow] pull-slot table
+    const T* wdot;          // [6 faces][kSlotRow] e_j . u_wall; null without a moving wall
     long vs;        // population stride (>= V, multiple of 64)
 };
 

@@ -32,20 +32,6 @@
 
 namespace lbm {
 
-// Global access as uniform base + 32-bit byte offset, so the compiler can use
-// the scalar-base addressing form (one VGPR per address instead of two).
-__device__ __forceinline__ float ldo(const float* base, unsigned boff) {
-    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + boff);
-}
-__device__ __forceinline__ void sto(float* base, unsigned boff, float v) {
-    *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + boff) = v;
-}
-__device__ __forceinline__ double ldo(const double* base, unsigned boff) {
-    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + boff);
-}
-__device__ __forceinline__ void sto(double* base, unsigned boff, double v) {
-    *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + boff) = v;
-}
 // Store with an optional non-temporal hint (streaming output read back only
 // next step, so it need not displace the halo rows held in L2).
 template <bool NT>
@@ -82,7 +68,7 @@ __device__ __forceinline__ void gather32(const Fields<T>& f, const BCDesc<T>& bc
         }
         return;
     }
-    const uint16_t* row = f.slots + cls * kQ;
+    const uint16_t* row = f.slots + cls * kSlotRow;
     T rho_prev = T(0);
     bool have_rho = false;
 #pragma unroll
@@ -731,6 +717,9 @@ fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int n
 }
 
 // ---- wall shells of a single simulation, one thread per cell ------------------
+__device__ __forceinline__ Node<unsigned> shell_node(const int q[3], const int n[3]) {
+    return {q[0], q[1], q[2], ((unsigned)q[2] * n[1] + q[1]) * n[0] + q[0]};
+}
 #ifndef LBM_FUSED_BODY_ONLY
 // Q update over the shell and its one-cell halo (w = 3). Every cell stores
 // Sigma and Tau for the force pass; only shell cells store Q^{n+1} and the
@@ -741,9 +730,7 @@ shell_qstep_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRegion
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    const Pos p{q[0], q[1], q[2]};
-    const long c = cell_of(p.x, p.y, p.z, bc.n[0], bc.n[1]);
-    qstep_cell(f, bc, k, c, p, !cell_mask(bc, 1, p.x, p.y).writes(p.z));
+    qstep_cell<true>(f, bc, k, shell_node(q, bc.n), !cell_mask(bc, 1, q[0], q[1]).writes(q[2]));
 }
 
 // Body force and collide-stream of the shell cells (w = 2); f.q points at
@@ -754,8 +741,7 @@ shell_force_lbm_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRe
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    const Pos p{q[0], q[1], q[2]};
-    force_lbm_cell<float, true, true>(f, bc, k, cell_of(p.x, p.y, p.z, bc.n[0], bc.n[1]), p, flags, pull);
+    force_lbm_cell<float, true, true, true>(f, bc, k, shell_node(q, bc.n), flags, pull);
 }
 #endif  // LBM_FUSED_BODY_ONLY
 
@@ -1133,7 +1119,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
         __shared__ uint32_t sSlot[16][8];
         if (t < 16 * 8) {
             const int cl = t >> 3, w = t & 7;
-            const uint16_t* row = f.slots + cl * kQ;
+            const uint16_t* row = f.slots + cl * kSlotRow;
             const uint32_t lo = row[2 * w], hi = 2 * w + 1 < kQ ? row[2 * w + 1] : 0u;
             sSlot[cl][w] = lo | (hi << 16);
         }

@@ -6,12 +6,9 @@
 #include "fused_step.hpp"
 
 namespace lbm {
-template void launch_qstep<double>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&, long,
-                                   hipStream_t);
-template void launch_force_lbm<double, false>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&,
-                                              long, int, int, hipStream_t);
-template void launch_stream_only<double>(const Fields<double>&, const BCDesc<double>&, long, int, double*,
-                                         hipStream_t);
+template void launch_qstep<double>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&, hipStream_t);
+template void launch_force_lbm<double, false>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&, int, int, hipStream_t);
+template void launch_stream_only<double>(const Fields<double>&, const BCDesc<double>&, int, double*, hipStream_t);
 template void launch_diagnostics<double>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&, long,
                                          double*, double*, int, double*, hipStream_t);
 template void launch_order_director<double>(const Fields<double>&, long, double*, double*, hipStream_t);

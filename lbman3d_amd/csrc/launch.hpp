@@ -12,19 +12,18 @@ enum : int { FL_FORCE = 1, FL_LBM = 2, FL_STORE_F = 4, FL_STORE_RHO = 8 };
 
 // Q update: Q^n, u^{n-1} -> Q^{n+1}, Sigma^n, Tau^n, F = Ericksen force.
 template <typename T>
-void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long V, hipStream_t s);
+void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, hipStream_t s);
 
 // Body force and/or collide-stream. pull = 0 reads the node's own slots
 // (populations uploaded as post-streaming values), pull = 1 gathers from the
 // upwind neighbours / walls (post-collision storage).
 template <typename T, bool SHIFTED>
-void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long V, int flags,
-                      int pull, hipStream_t s);
+void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, int flags, int pull,
+                      hipStream_t s);
 
 // Post-streaming populations f(x, j) of the stored state into out[15][vs].
 template <typename T>
-void launch_stream_only(const Fields<T>& f, const BCDesc<T>& bc, long V, int pull, T* out,
-                        hipStream_t s);
+void launch_stream_only(const Fields<T>& f, const BCDesc<T>& bc, int pull, T* out, hipStream_t s);
 
 // FP64 reductions: per-block partials of mass, px, py, pz, kinetic, du2, u2,
 // umax^2, free energy, nonfinite count; then a single-block final pass.

@@ -32,14 +32,15 @@ __device__ __forceinline__ int nb_index(int i, int s, int n, bool lo_per, bool h
 // Ghost-substituted (minus, plus) pair of Q component c along axis a
 // (QAxisGhostPair / QGhost, src/boundary_handler.h:257-282): only the low
 // face's tag selects the periodic short-cut.
+// Selects, not branches: a branch here would hold back the loads that follow.
 template <typename T>
 __device__ __forceinline__ void q_pair(const BCDesc<T>& bc, int a, int c, int i, T qm, T q0, T qp,
                                        T& m, T& p) {
-    m = qm;
-    p = qp;
-    if (bc.qkind[2 * a] == QB_PERIODIC) return;
-    if (i == 0) m = (bc.qkind[2 * a] == QB_ANCHOR) ? T(2.0) * bc.anchor[2 * a][c] - q0 : q0;
-    if (i == bc.n[a] - 1) p = (bc.qkind[2 * a + 1] == QB_ANCHOR) ? T(2.0) * bc.anchor[2 * a + 1][c] - q0 : q0;
+    const bool walls = bc.qkind[2 * a] != QB_PERIODIC;
+    const T tm = T(2.0) * bc.anchor[2 * a][c] - q0, tp = T(2.0) * bc.anchor[2 * a + 1][c] - q0;
+    const T gm = bc.qkind[2 * a] == QB_ANCHOR ? tm : q0, gp = bc.qkind[2 * a + 1] == QB_ANCHOR ? tp : q0;
+    m = (walls & (i == 0)) ? gm : qm;
+    p = (walls & (i == bc.n[a] - 1)) ? gp : qp;
 }
 
 // QGradientAndLaplacian for one component from its seven stencil values
@@ -66,21 +67,21 @@ __device__ __forceinline__ Deriv<T> q_deriv(const BCDesc<T>& bc, int c, const in
 }
 
 // Velocity ghost pair for component comp along axis a
-// (VelocityGhost / VelocityAxisGhostPair, src/boundary_handler.h:121-146).
+// (VelocityGhost / VelocityAxisGhostPair, src/boundary_handler.h:121-146);
+// wall_u is zero on walls that do not move.
 template <typename T>
 __device__ __forceinline__ T u_ghost(const BCDesc<T>& bc, int face, int comp, bool normal, T vb) {
-    const int k = bc.ukind[face];
-    const T wv = (k == UB_MOVING) ? bc.wall_u[face][comp] : T(0.0);
-    if (k == UB_SPECULAR) return normal ? (T(2.0) * wv - vb) : vb;
-    return T(2.0) * wv - vb;
+    const T reflected = T(2.0) * bc.wall_u[face][comp] - vb;
+    return (bc.ukind[face] == UB_SPECULAR && !normal) ? vb : reflected;
 }
 template <typename T, bool NOGHOST = false>
 __device__ __forceinline__ T u_grad(const BCDesc<T>& bc, int a, int comp, int i, T vm, T v0, T vp) {
     T m = vm, p = vp;
-    if (!NOGHOST && bc.ukind[2 * a] != UB_PERIODIC) {
-        const bool normal = (comp == a);
-        if (i == 0) m = u_ghost(bc, 2 * a, comp, normal, v0);
-        if (i == bc.n[a] - 1) p = u_ghost(bc, 2 * a + 1, comp, normal, v0);
+    if (!NOGHOST) {
+        const bool walls = bc.ukind[2 * a] != UB_PERIODIC, normal = comp == a;
+        const T gm = u_ghost(bc, 2 * a, comp, normal, v0), gp = u_ghost(bc, 2 * a + 1, comp, normal, v0);
+        m = (walls & (i == 0)) ? gm : vm;
+        p = (walls & (i == bc.n[a] - 1)) ? gp : vp;
     }
     return (p - m) / T(2.0);
 }

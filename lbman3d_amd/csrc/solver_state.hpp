@@ -26,7 +26,6 @@ struct lbm_solver {
     BCDesc<float> bc32{};
     Phys<double> k64{};
     Phys<float> k32{};
-    uint16_t* slots = nullptr;
     double* uprev = nullptr;
     double* partials = nullptr;
     double* diag_out = nullptr;

@@ -3,6 +3,8 @@
 // access of a wavefront is a contiguous, coalesced run.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "physics.hpp"
@@ -27,50 +29,118 @@ __device__ __forceinline__ long cell_of(int x, int y, int z, int nx, int ny) {
     return ((long)z * ny + y) * nx + x;
 }
 
-// Gather the 15 incoming populations of node (x, y, z) from the
-// post-collision buffer g: upwind neighbour, or the node's own reflected
-// population at a wall (push semantics of src/lbm_solver.tpp:144-192 and
-// HandleBoundaryPoint, src/boundary_handler.h:403-426, restated as pull
-// through the host-built slot table). rho_prev is the density this node had
-// when those populations were produced (moving walls).
-template <typename T, bool SHIFTED>
-__device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, int x, int y, int z, long c,
-                                       int pull, T out[kQ]) {
-    const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
+// Global access as uniform base + 32-bit byte offset, so the compiler can use
+// the scalar-base addressing form (one VGPR per address instead of two).
+template <typename T>
+__device__ __forceinline__ T ldo(const T* base, unsigned boff) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + boff);
+}
+template <typename T>
+__device__ __forceinline__ void sto(T* base, unsigned boff, T v) {
+    *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + boff) = v;
+}
+
+// A cell by position and index. Off is 32 bits while an array stays below
+// 4 GiB (an index is then one register next to the array's scalar base).
+template <typename Off>
+struct Node {
+    int x, y, z;
+    Off c;   // (z * ny + y) * nx + x
+};
+template <typename Off, typename T>
+__device__ __forceinline__ T ldn(const T* base, Off o) {
+    if constexpr (sizeof(Off) == 4) return ldo(base, o * (unsigned)sizeof(T));
+    else return base[o];
+}
+template <typename Off, typename T>
+__device__ __forceinline__ void stn(T* base, Off o, T v) {
+    if constexpr (sizeof(Off) == 4) sto(base, o * (unsigned)sizeof(T), v);
+    else base[o] = v;
+}
+
+// The node and its six stencil neighbours (xm, xp, ym, yp, zm, zp) under one
+// set of tags (kind[face], 0 = periodic): a periodic side wraps, any other
+// side clamps to the node itself (nb_index).
+template <bool WALLS, typename Off>
+__device__ __forceinline__ void stencil(const Node<Off>& p, const int n[3], const int kind[6], Off nb[7]) {
+    const Off sx = 1, sy = (Off)(unsigned)n[0], sz = sy * (Off)(unsigned)n[1];
+    const Off stride[3] = {sx, sy, sz};
+    const int pos[3] = {p.x, p.y, p.z};
+    nb[0] = p.c;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const Off span = stride[a] * (Off)(unsigned)(n[a] - 1);
+        const bool lo = WALLS && kind[2 * a] != 0, hi = WALLS && kind[2 * a + 1] != 0;
+        nb[1 + 2 * a] = pos[a] > 0 ? p.c - stride[a] : p.c + (lo ? (Off)0 : span);
+        nb[2 + 2 * a] = pos[a] < n[a] - 1 ? p.c + stride[a] : p.c - (hi ? (Off)0 : span);
+    }
+}
+
+// Gather the 15 incoming populations of a node from the post-collision buffer
+// g: upwind neighbour, or the node's own reflected population at a wall (push
+// semantics of src/lbm_solver.tpp:144-192 and HandleBoundaryPoint,
+// src/boundary_handler.h:403-426, restated as pull through the host-built slot
+// table). rho_prev is the density this node had when those populations were
+// produced (moving walls; Fields::wdot holds e_j . u_wall per face and slot).
+// WALLS false: every velocity face periodic.
+//
+// No load waits for another, the slot row's aside: a wavefront without a wall
+// cell reads the 15 wrapped upwind neighbours, and one with a wall cell
+// selects, per lane and slot, the neighbour or the node's own population.
+// (A branch per slot made a wall wavefront a chain of 15 dependent loads.)
+template <typename T, bool WALLS, typename Off>
+__device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, const Node<Off>& p, int pull,
+                                       T out[kQ]) {
     const T* g = f.g;
     const long vs = f.vs;
     if (!pull) {
 #pragma unroll
-        for (int j = 0; j < kQ; ++j) out[j] = g[j * vs + c];
+        for (int j = 0; j < kQ; ++j) out[j] = ldn(g + j * vs, p.c);
         return;
     }
-    const int cls = node_class(x, y, z, nx, ny, nz);
-    if (cls == 0) {
+    // Index c + 1 of each axis is the wrapped neighbour at -c.
+    const int n[3] = {bc.n[0], bc.n[1], bc.n[2]};
+    Off d[3][3];
+    {
+        Off stride = 1;
+        const int pos[3] = {p.x, p.y, p.z};
 #pragma unroll
-        for (int j = 0; j < kQ; ++j) out[j] = g[j * vs + c - cx(j) - (long)cy(j) * nx - (long)cz(j) * nx * ny];
+        for (int a = 0; a < 3; ++a) {
+            const Off span = stride * (Off)(unsigned)(n[a] - 1);
+            d[a][0] = pos[a] < n[a] - 1 ? stride : (Off)0 - span;
+            d[a][1] = 0;
+            d[a][2] = pos[a] > 0 ? (Off)0 - stride : span;
+            stride *= (Off)(unsigned)n[a];
+        }
+    }
+    const int cls = WALLS ? node_class(p.x, p.y, p.z, n[0], n[1], n[2]) : 0;
+    if (!WALLS || __builtin_amdgcn_ballot_w64(cls != 0) == 0) {
+#pragma unroll
+        for (int j = 0; j < kQ; ++j)
+            out[j] = ldn(g + j * vs, (Off)(p.c + d[0][cx(j) + 1] + d[1][cy(j) + 1] + d[2][cz(j) + 1]));
         return;
     }
-    const uint16_t* row = f.slots + cls * kQ;
-    T rho_prev = T(0);
-    bool have_rho = false;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4* rp = reinterpret_cast<const u32x4*>(f.slots + cls * kSlotRow);
+    const u32x4 r0 = rp[0], r1 = rp[1];
+    const uint32_t words[8] = {r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]};
+    uint16_t e[kQ];
 #pragma unroll
     for (int j = 0; j < kQ; ++j) {
-        const uint16_t e = row[j];
-        const int kind = slot_kind(e);
-        if (kind == SLOT_STREAM) {
-            int xs = x - cx(j), ys = y - cy(j), zs = z - cz(j);
-            xs = xs < 0 ? xs + nx : (xs >= nx ? xs - nx : xs);
-            ys = ys < 0 ? ys + ny : (ys >= ny ? ys - ny : ys);
-            zs = zs < 0 ? zs + nz : (zs >= nz ? zs - nz : zs);
-            out[j] = g[j * vs + cell_of(xs, ys, zs, nx, ny)];
-        } else if (kind == SLOT_MIRROR) {
-            out[j] = g[slot_src(e) * vs + c];
-        } else {
-            const int face = slot_face(e);
-            if (!have_rho) { rho_prev = bc.rho_base + f.rho[c]; have_rho = true; }
-            const T dot = T(cx(j)) * bc.wall_u[face][0] + T(cy(j)) * bc.wall_u[face][1]
-                        + T(cz(j)) * bc.wall_u[face][2];
-            out[j] = g[slot_src(e) * vs + c] + T(6.0) * rho_prev * T(wgt(j)) * dot;
+        e[j] = (uint16_t)(words[j >> 1] >> (16 * (j & 1)));
+        const Off nb = p.c + d[0][cx(j) + 1] + d[1][cy(j) + 1] + d[2][cz(j) + 1];
+        const bool stream = slot_kind(e[j]) == SLOT_STREAM;
+        out[j] = g[(size_t)(stream ? j : slot_src(e[j])) * (size_t)vs + (stream ? nb : p.c)];
+    }
+    if (f.wdot) {
+        const T rho_prev = bc.rho_base + ldn(f.rho, p.c);
+        T dot[kQ];
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) dot[j] = f.wdot[slot_face(e[j]) * kSlotRow + j];
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+            const T moved = out[j] + T(6.0) * rho_prev * T(wgt(j)) * dot[j];
+            out[j] = slot_kind(e[j]) == SLOT_BOUNCE ? moved : out[j];
         }
     }
 }
@@ -79,67 +149,81 @@ __device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, 
 // QTensorSolver::StepAndSetupBodyForce (src/qtensor_solver.tpp:50-147).
 // One cell. `own` false stores Sigma and Tau only (a halo cell of a region
 // pass whose Q^{n+1} and Ericksen force belong to another launch).
-template <typename T>
-__device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long c, Pos p,
-                                           bool own) {
-    const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
+//
+// Every load is issued before the first use, and the ghosts are selects: with
+// a branch per component and axis (uniform, but a branch) the loads of each
+// component waited for the arithmetic of the one before, eight memory
+// latencies in a row. Bound by latency on small grids and by the caches on
+// large ones. With force_lbm_cell, a step of the two kernels went from 23.7
+// to 14.4 us at 32^3 FP64, 48.6 to 36.4 us (FP64) and 30.7 to 19.0 us (FP32)
+// on a 20x100x100 channel, and 2.82 to 2.56 ms at 256^3 FP64.
+template <bool WALLS, typename T, typename Off>
+__device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
+                                           const Node<Off>& p, bool own) {
     const int pos[3] = {p.x, p.y, p.z};
-
     // Q stencil neighbours (Q tags), velocity neighbours (velocity tags).
-    const int qxm = nb_index(p.x, -1, nx, bc.qkind[0] == QB_PERIODIC, bc.qkind[1] == QB_PERIODIC);
-    const int qxp = nb_index(p.x, +1, nx, bc.qkind[0] == QB_PERIODIC, bc.qkind[1] == QB_PERIODIC);
-    const int qym = nb_index(p.y, -1, ny, bc.qkind[2] == QB_PERIODIC, bc.qkind[3] == QB_PERIODIC);
-    const int qyp = nb_index(p.y, +1, ny, bc.qkind[2] == QB_PERIODIC, bc.qkind[3] == QB_PERIODIC);
-    const int qzm = nb_index(p.z, -1, nz, bc.qkind[4] == QB_PERIODIC, bc.qkind[5] == QB_PERIODIC);
-    const int qzp = nb_index(p.z, +1, nz, bc.qkind[4] == QB_PERIODIC, bc.qkind[5] == QB_PERIODIC);
-    const long q_nb[6] = {cell_of(qxm, p.y, p.z, nx, ny), cell_of(qxp, p.y, p.z, nx, ny),
-                          cell_of(p.x, qym, p.z, nx, ny), cell_of(p.x, qyp, p.z, nx, ny),
-                          cell_of(p.x, p.y, qzm, nx, ny), cell_of(p.x, p.y, qzp, nx, ny)};
+    Off qs[7], us[7];
+    stencil<WALLS>(p, bc.n, bc.qkind, qs);
+    stencil<WALLS>(p, bc.n, bc.ukind, us);
+    T v[8][7];
+#pragma unroll
+    for (int m = 0; m < 5; ++m)
+#pragma unroll
+        for (int i = 0; i < 7; ++i) v[m][i] = ldn(f.q[m], qs[i]);
+#pragma unroll
+    for (int A = 0; A < 3; ++A)
+#pragma unroll
+        for (int i = 0; i < 7; ++i) v[5 + A][i] = ldn(f.u[A], us[i]);
     T Q[5];
     Deriv<T> dq[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
-        const T* q = f.q[m];
-        Q[m] = q[c];
-        dq[m] = q_deriv(bc, m, pos, Q[m], q[q_nb[0]], q[q_nb[1]], q[q_nb[2]], q[q_nb[3]], q[q_nb[4]], q[q_nb[5]]);
+        Q[m] = v[m][0];
+        dq[m] = q_deriv<T, !WALLS>(bc, m, pos, Q[m], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
     }
-    const int uxm = nb_index(p.x, -1, nx, bc.ukind[0] == UB_PERIODIC, bc.ukind[1] == UB_PERIODIC);
-    const int uxp = nb_index(p.x, +1, nx, bc.ukind[0] == UB_PERIODIC, bc.ukind[1] == UB_PERIODIC);
-    const int uym = nb_index(p.y, -1, ny, bc.ukind[2] == UB_PERIODIC, bc.ukind[3] == UB_PERIODIC);
-    const int uyp = nb_index(p.y, +1, ny, bc.ukind[2] == UB_PERIODIC, bc.ukind[3] == UB_PERIODIC);
-    const int uzm = nb_index(p.z, -1, nz, bc.ukind[4] == UB_PERIODIC, bc.ukind[5] == UB_PERIODIC);
-    const int uzp = nb_index(p.z, +1, nz, bc.ukind[4] == UB_PERIODIC, bc.ukind[5] == UB_PERIODIC);
-    const long u_nb[6] = {cell_of(uxm, p.y, p.z, nx, ny), cell_of(uxp, p.y, p.z, nx, ny),
-                          cell_of(p.x, uym, p.z, nx, ny), cell_of(p.x, uyp, p.z, nx, ny),
-                          cell_of(p.x, p.y, uzm, nx, ny), cell_of(p.x, p.y, uzp, nx, ny)};
     T u[3], g[3][3];
 #pragma unroll
     for (int A = 0; A < 3; ++A) {
-        const T* v = f.u[A];
-        const T v0 = v[c];
-        u[A] = v0;
+        u[A] = v[5 + A][0];
 #pragma unroll
-        for (int B = 0; B < 3; ++B) g[A][B] = u_grad(bc, B, A, pos[B], v[u_nb[2 * B]], v0, v[u_nb[2 * B + 1]]);
+        for (int B = 0; B < 3; ++B)
+            g[A][B] = u_grad<T, !WALLS>(bc, B, A, pos[B], v[5 + A][1 + 2 * B], u[A], v[5 + A][2 + 2 * B]);
     }
     T qn[5], sg[5], ta[3], fe[3];
     q_pointwise(k, Q, u, dq, g, qn, sg, ta, fe);
 #pragma unroll
-    for (int m = 0; m < 5; ++m) f.sig[m][c] = sg[m];
+    for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, sg[m]);
 #pragma unroll
-    for (int m = 0; m < 3; ++m) f.tau[m][c] = ta[m];
+    for (int m = 0; m < 3; ++m) stn(f.tau[m], p.c, ta[m]);
     if (own) {
 #pragma unroll
-        for (int m = 0; m < 5; ++m) f.qn[m][c] = qn[m];
+        for (int m = 0; m < 5; ++m) stn(f.qn[m], p.c, qn[m]);
 #pragma unroll
-        for (int m = 0; m < 3; ++m) f.F[m][c] = fe[m];
+        for (int m = 0; m < 3; ++m) stn(f.F[m], p.c, fe[m]);
     }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, long V) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= V) return;
-    qstep_cell(f, bc, k, c, cell_pos(c, bc.n[0], bc.n[1]), true);
+// One thread per cell, cells linear; positions by multiplication (the
+// compiler's 64-bit division is some 150 instructions, three times a cell).
+struct CellGrid {
+    FastDiv by_plane, by_nx;
+    unsigned plane, nx, cells;
+};
+inline CellGrid cell_grid(const int n[3]) {
+    const unsigned plane = (unsigned)n[0] * (unsigned)n[1];
+    return {fast_div(plane), fast_div((unsigned)n[0]), plane, (unsigned)n[0], plane * (unsigned)n[2]};
+}
+template <typename Off>
+__device__ __forceinline__ Node<Off> node_at(const CellGrid& g, unsigned c) {
+    const unsigned z = g.by_plane.div(c), r = c - z * g.plane, y = g.by_nx.div(r);
+    return {(int)(r - y * g.nx), (int)y, (int)z, (Off)c};
+}
+
+template <typename T, bool WALLS, typename Off>
+__global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg) {
+    const unsigned c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= cg.cells) return;
+    qstep_cell<WALLS>(f, bc, k, node_at<Off>(cg, c), true);
 }
 
 // ---- body force and collide-stream ----------------------------------------
@@ -148,92 +232,81 @@ __global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc
 // is the merge the reference documents as valid (src/qtensor_solver.tpp:219-247):
 // the force at a node feeds only that node's collision.
 // One cell. UN: the velocity goes to un (fused-step buffers, where u still
-// holds u^{n-1} for other cells) instead of replacing u in place.
-template <typename T, bool SHIFTED, bool UN>
-__device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long c,
-                                               Pos p, int flags, int pull) {
-    const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
-    T F[3];
+// holds u^{n-1} for other cells) instead of replacing u in place. Loads first,
+// as in qstep_cell.
+template <typename T, bool SHIFTED, bool UN, bool WALLS, typename Off>
+__device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
+                                               const Node<Off>& p, int flags, int pull) {
+    T pop[kQ], F[3];
+    if (flags & FL_LBM) gather<T, WALLS>(f, bc, p, pull, pop);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) F[m] = ldn(f.F[m], p.c);   // the Ericksen force, or the whole force
     if (flags & FL_FORCE) {
-        const T fe[3] = {f.F[0][c], f.F[1][c], f.F[2][c]};
         if (k.force_full) {
             const int pos[3] = {p.x, p.y, p.z};
-            const int xm = nb_index(p.x, -1, nx, bc.qkind[0] == QB_PERIODIC, bc.qkind[1] == QB_PERIODIC);
-            const int xp = nb_index(p.x, +1, nx, bc.qkind[0] == QB_PERIODIC, bc.qkind[1] == QB_PERIODIC);
-            const int ym = nb_index(p.y, -1, ny, bc.qkind[2] == QB_PERIODIC, bc.qkind[3] == QB_PERIODIC);
-            const int yp = nb_index(p.y, +1, ny, bc.qkind[2] == QB_PERIODIC, bc.qkind[3] == QB_PERIODIC);
-            const int zm = nb_index(p.z, -1, nz, bc.qkind[4] == QB_PERIODIC, bc.qkind[5] == QB_PERIODIC);
-            const int zp = nb_index(p.z, +1, nz, bc.qkind[4] == QB_PERIODIC, bc.qkind[5] == QB_PERIODIC);
-            const long nb[6] = {cell_of(xm, p.y, p.z, nx, ny), cell_of(xp, p.y, p.z, nx, ny),
-                                cell_of(p.x, ym, p.z, nx, ny), cell_of(p.x, yp, p.z, nx, ny),
-                                cell_of(p.x, p.y, zm, nx, ny), cell_of(p.x, p.y, zp, nx, ny)};
-            T dQ[5][3];
+            Off nb[7];
+            stencil<WALLS>(p, bc.n, bc.qkind, nb);
+            T v[13][7];
+#pragma unroll
+            for (int m = 0; m < 13; ++m) {
+                const T* a = m < 5 ? f.q[m] : (m < 10 ? f.sig[m - 5] : f.tau[m - 10]);
+#pragma unroll
+                for (int i = 0; i < 7; ++i) v[m][i] = ldn(a, nb[i]);
+            }
+            const T u[3] = {ldn(f.u[0], p.c), ldn(f.u[1], p.c), ldn(f.u[2], p.c)};
+            T dQ[5][3], dS[8][3];
 #pragma unroll
             for (int m = 0; m < 5; ++m) {
-                const T* q = f.q[m];
-                const Deriv<T> d = q_deriv(bc, m, pos, q[c], q[nb[0]], q[nb[1]], q[nb[2]], q[nb[3]], q[nb[4]], q[nb[5]]);
-                dQ[m][0] = d.d[0];
-                dQ[m][1] = d.d[1];
-                dQ[m][2] = d.d[2];
-            }
-            T dS[8][3];
+                const Deriv<T> d =
+                    q_deriv<T, !WALLS>(bc, m, pos, v[m][0], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
 #pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const T* s = m < 5 ? f.sig[m] : f.tau[m - 5];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) dS[m][a] = (s[nb[2 * a + 1]] - s[nb[2 * a]]) / T(2.0);
+                for (int a = 0; a < 3; ++a) dQ[m][a] = d.d[a];
             }
-            const T u[3] = {f.u[0][c], f.u[1][c], f.u[2][c]};
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+#pragma unroll
+                for (int a = 0; a < 3; ++a) dS[m][a] = (v[5 + m][2 + 2 * a] - v[5 + m][1 + 2 * a]) / T(2.0);
+            const T fe[3] = {F[0], F[1], F[2]};
             body_force(k, dQ, dS, u, fe, F);
-        } else {
-            F[0] = fe[0];
-            F[1] = fe[1];
-            F[2] = fe[2];
         }
         if (flags & FL_STORE_F) {
-            f.F[0][c] = F[0];
-            f.F[1][c] = F[1];
-            f.F[2][c] = F[2];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) stn(f.F[m], p.c, F[m]);
         }
-    } else {
-        F[0] = f.F[0][c];
-        F[1] = f.F[1][c];
-        F[2] = f.F[2][c];
     }
     if (!(flags & FL_LBM)) return;
 
-    T pop[kQ];
-    gather<T, SHIFTED>(f, bc, p.x, p.y, p.z, c, pull, pop);
     T rho_st, u[3];   // the density in its stored form (rho - BCDesc::rho_base)
     if constexpr (SHIFTED) collide_shifted(k, pop, F, rho_st, u);
     else collide_plain(k, pop, F, rho_st, u);
-    if (flags & FL_STORE_RHO) f.rho[c] = rho_st;
+    if (flags & FL_STORE_RHO) stn(f.rho, p.c, rho_st);
     T* const* uo = UN ? f.un : f.u;
-    uo[0][c] = u[0];
-    uo[1][c] = u[1];
-    uo[2][c] = u[2];
 #pragma unroll
-    for (int j = 0; j < kQ; ++j) f.gn[j * f.vs + c] = pop[j];
+    for (int m = 0; m < 3; ++m) stn(uo[m], p.c, u[m]);
+#pragma unroll
+    for (int j = 0; j < kQ; ++j) stn(f.gn + j * f.vs, p.c, pop[j]);
 }
 
-template <typename T, bool SHIFTED>
+// FLAGS is a template argument so that the step's own combination is one
+// straight run from the loads to the stores.
+template <typename T, bool SHIFTED, bool WALLS, int FLAGS, typename Off>
 __global__ void __launch_bounds__(kBlock)
-force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, long V, int flags, int pull) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= V) return;
-    force_lbm_cell<T, SHIFTED, false>(f, bc, k, c, cell_pos(c, bc.n[0], bc.n[1]), flags, pull);
+force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg, int store, int pull) {
+    const unsigned c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= cg.cells) return;
+    force_lbm_cell<T, SHIFTED, false, WALLS>(f, bc, k, node_at<Off>(cg, c), FLAGS | store, pull);
 }
 
-template <typename T>
+template <typename T, bool WALLS, typename Off>
 __global__ void __launch_bounds__(kBlock)
-stream_only_kernel(Fields<T> f, BCDesc<T> bc, long V, int pull, T* out) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= V) return;
-    const Pos p = cell_pos(c, bc.n[0], bc.n[1]);
+stream_only_kernel(Fields<T> f, BCDesc<T> bc, CellGrid cg, int pull, T* out) {
+    const unsigned c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= cg.cells) return;
+    const Node<Off> p = node_at<Off>(cg, c);
     T pop[kQ];
-    gather<T, false>(f, bc, p.x, p.y, p.z, c, pull, pop);
+    gather<T, WALLS>(f, bc, p, pull, pop);
 #pragma unroll
-    for (int j = 0; j < kQ; ++j) out[j * f.vs + c] = pop[j];
+    for (int j = 0; j < kQ; ++j) stn(out + j * f.vs, p.c, pop[j]);
 }
 
 // ---- FP64 diagnostics ---------------------------------------------------------
@@ -354,21 +427,55 @@ order_director_kernel(Fields<T> f, long V, double* order, double* director) {
 // ---- launchers ---------------------------------------------------------------
 inline unsigned grid_for(long V) { return (unsigned)((V + kBlock - 1) / kBlock); }
 
+// fn(walls, offset) with the kernels' template arguments: whether any face has
+// a wall, and 32-bit indices while an array stays below 4 GiB.
+template <typename T, typename F>
+void with_step_form(const BCDesc<T>& bc, const CellGrid& cg, F&& fn) {
+    bool walls = false;
+    for (int face = 0; face < 6; ++face)
+        walls = walls || bc.qkind[face] != QB_PERIODIC || bc.ukind[face] != UB_PERIODIC;
+    auto with_offset = [&](auto w) {
+        if ((size_t)cg.cells * sizeof(T) < (1ull << 32)) fn(w, 0u);
+        else fn(w, (size_t)0);
+    };
+    if (walls) with_offset(std::true_type{});
+    else with_offset(std::false_type{});
+}
+
 template <typename T>
-void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long V, hipStream_t s) {
-    hipLaunchKernelGGL(qstep_kernel<T>, dim3(grid_for(V)), dim3(kBlock), 0, s, f, bc, k, V);
+void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, hipStream_t s) {
+    const CellGrid cg = cell_grid(bc.n);
+    with_step_form(bc, cg, [&](auto w, auto off) {
+        hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, decltype(off)>), dim3(grid_for(cg.cells)),
+                           dim3(kBlock), 0, s, f, bc, k, cg);
+    });
 }
 
 template <typename T, bool SHIFTED>
-void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, long V, int flags, int pull,
+void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, int flags, int pull,
                       hipStream_t s) {
-    hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED>), dim3(grid_for(V)), dim3(kBlock), 0, s, f, bc, k, V, flags,
-                       pull);
+    const CellGrid cg = cell_grid(bc.n);
+    const int store = flags & (FL_STORE_F | FL_STORE_RHO);
+    with_step_form(bc, cg, [&](auto w, auto off) {
+        auto go = [&](auto parts) {
+            hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED, decltype(w)::value, decltype(parts)::value, decltype(off)>),
+                               dim3(grid_for(cg.cells)), dim3(kBlock), 0, s, f, bc, k, cg, store, pull);
+        };
+        switch (flags & (FL_FORCE | FL_LBM)) {
+            case FL_FORCE: go(std::integral_constant<int, FL_FORCE>{}); break;
+            case FL_LBM: go(std::integral_constant<int, FL_LBM>{}); break;
+            default: go(std::integral_constant<int, FL_FORCE | FL_LBM>{}); break;
+        }
+    });
 }
 
 template <typename T>
-void launch_stream_only(const Fields<T>& f, const BCDesc<T>& bc, long V, int pull, T* out, hipStream_t s) {
-    hipLaunchKernelGGL(stream_only_kernel<T>, dim3(grid_for(V)), dim3(kBlock), 0, s, f, bc, V, pull, out);
+void launch_stream_only(const Fields<T>& f, const BCDesc<T>& bc, int pull, T* out, hipStream_t s) {
+    const CellGrid cg = cell_grid(bc.n);
+    with_step_form(bc, cg, [&](auto w, auto off) {
+        hipLaunchKernelGGL((stream_only_kernel<T, decltype(w)::value, decltype(off)>), dim3(grid_for(cg.cells)),
+                           dim3(kBlock), 0, s, f, bc, cg, pull, out);
+    });
 }
 
 template <typename T>
