@@ -202,6 +202,10 @@ BCDesc<T> make_bc(const lbm_config& c) {
         for (int k = 0; k < 5; ++k) b.anchor[f][k] = (T)a[k];
         for (int k = 0; k < 3; ++k) b.wall_u[f][k] = (T)(c.walls[f].ubc == LBM_U_MOVING ? c.walls[f].wall_u[k] : 0.0);
     }
+    for (int a = 0; a < 3; ++a) {
+        const int lo = c.walls[2 * a].qbc, hi = c.walls[2 * a + 1].qbc;
+        if (lo != LBM_Q_PERIODIC && (lo == LBM_Q_ANCHORING || hi != LBM_Q_NEUMANN)) b.q_ghosts = 1;
+    }
     return b;
 }
 template BCDesc<double> make_bc<double>(const lbm_config&);

@@ -86,6 +86,8 @@ struct BCDesc {
     T anchor[6][5];      // strong-anchoring Q per face (xx, xy, xz, yy, yz)
     T wall_u[6][3];      // wall velocity per face (MovingWall; zero otherwise)
     int all_periodic_u;  // every velocity face periodic: no wall slots anywhere
+    int q_ghosts;        // some axis has a wall whose ghost Q differs from what the stress stencil
+                         // reads beyond it: anchoring, or a periodic high face opposite a wall
     int slots_xy;        // every reachable class has the slot row of its x, y
                          // bits alone (the z bits change nothing)
     T rho_base;          // the density array holds rho - rho_base (rho0 for the
@@ -106,8 +108,8 @@ template <typename T>
 struct Fields {
     T* q[5];        // Q^n            (xx, xy, xz, yy, yz)
     T* qn[5];       // Q^{n+1}
-    T* sig[5];      // Sigma^n
-    T* tau[3];      // Tau^n (xy, xz, yz)
+    T* sig[5];      // Sigma^n                 } FP64; in FP32 the stress components
+    T* tau[3];      // Tau^n (xy, xz, yz)      } that qstep_cell describes
     T* F[3];        // body force
     T* u[3];        // velocity u^{n-1} (unfused kernels update it in place)
     T* un[3];       // velocity u^n written by the fused kernel

@@ -976,29 +976,6 @@ fused_step_kernel_pf(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull,
     }
 }
 
-// Divergence form of the body force. With P = -alpha Q^{n+1} + (Sigma +/- Tau)
-// in the sign pattern of body_force (src/qtensor_solver.tpp:154-217,
-// src/boundary_handler.h:335-392), F_a = d_b P_ab - mu u_a + F_E,a, and a
-// neighbour along axis b contributes only the column (P_xb, P_yb, P_zb):
-//   X set (x neighbours): -aQxx + Sxx, -aQxy + Sxy - Txy, -aQxz + Sxz - Txz;
-//   Y set (y neighbours): -aQxy + Sxy + Txy, -aQyy + Syy, -aQyz + Syz - Tyz;
-//   Z set (z neighbours): -aQxz + Sxz + Txz, -aQyz + Syz + Tyz, a(Qxx + Qyy) - Sxx - Syy.
-// (Szz = -Sxx - Syy and Qzz = -Qxx - Qyy.)
-__device__ __forceinline__ void p_sets(float alpha, const StageA& a, float pxy[6], float pz[3]) {
-    const float* q = a.qn;
-    const float* sg = a.sg;
-    const float* ta = a.ta;
-    pxy[0] = sg[0] - alpha * q[0];
-    pxy[1] = (sg[1] - ta[0]) - alpha * q[1];
-    pxy[2] = (sg[2] - ta[1]) - alpha * q[2];
-    pxy[3] = (sg[1] + ta[0]) - alpha * q[1];
-    pxy[4] = sg[3] - alpha * q[3];
-    pxy[5] = (sg[4] - ta[2]) - alpha * q[4];
-    pz[0] = (sg[2] + ta[1]) - alpha * q[2];
-    pz[1] = (sg[4] + ta[2]) - alpha * q[4];
-    pz[2] = alpha * (q[0] + q[3]) - (sg[0] + sg[3]);
-}
-
 // Boundary tags the third pipeline's WALLS mode computes exactly: z faces
 // periodic (and a slot table whose rows do not depend on the z position:
 // BCDesc::slots_xy), x and y faces with a periodic or Neumann Q tag and a periodic,
@@ -1231,7 +1208,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
             const int qpos[3] = {qpos_i[0], qpos_i[1], zq};
             stage_a_lean<TX, TY, WALLS ? 2 : 1, UPWIND>(bc, k, sIn[bi], ia + 1, ib + 1, hin[0], hin[1], hin[2], qpos,
                                                         qpos, ai, fe_new);
-            p_sets(k.alpha, ai, pxy_new, z_new);
+            p_sets(k.alpha, ai.qn, ai.sg, ai.ta, pxy_new, z_new);
         }
         float pr_new[6] = {0, 0, 0, 0, 0, 0};
         if (has_ring) {
@@ -1245,7 +1222,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
             }
             StageA ar;
             stage_a_lean<TX, TY, WALLS ? 2 : 1, UPWIND>(bc, k, sIn[bi], ra + 1, rb + 1, zm, c, zp, qpos, qpos, ar, fer);
-            p_sets(k.alpha, ar, pr_new, zr);
+            p_sets(k.alpha, ar.qn, ar.sg, ar.ta, pr_new, zr);
         }
 
         // ---- force + collide-stream at plane pb (sP[bi ^ 1] holds plane pb) ----

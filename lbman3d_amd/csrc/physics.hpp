@@ -240,6 +240,27 @@ __device__ __forceinline__ void body_force(const Phys<T>& k, const T dQ[5][3], c
     F[2] = fe[2] + fz;
 }
 
+// Divergence form of the body force. With P = -alpha Q^{n+1} + (Sigma +/- Tau)
+// in the sign pattern of body_force (src/qtensor_solver.tpp:154-217,
+// src/boundary_handler.h:335-392), F_a = d_b P_ab - mu u_a + F_E,a, and a
+// neighbour along axis b contributes only the column (P_xb, P_yb, P_zb):
+//   X set (x neighbours): -aQxx + Sxx, -aQxy + Sxy - Txy, -aQxz + Sxz - Txz;
+//   Y set (y neighbours): -aQxy + Sxy + Txy, -aQyy + Syy, -aQyz + Syz - Tyz;
+//   Z set (z neighbours): -aQxz + Sxz + Txz, -aQyz + Syz + Tyz, a(Qxx + Qyy) - Sxx - Syy.
+// (Szz = -Sxx - Syy and Qzz = -Qxx - Qyy.)
+template <typename T>
+__device__ __forceinline__ void p_sets(T alpha, const T q[5], const T sg[5], const T ta[3], T pxy[6], T pz[3]) {
+    pxy[0] = sg[0] - alpha * q[0];
+    pxy[1] = (sg[1] - ta[0]) - alpha * q[1];
+    pxy[2] = (sg[2] - ta[1]) - alpha * q[2];
+    pxy[3] = (sg[1] + ta[0]) - alpha * q[1];
+    pxy[4] = sg[3] - alpha * q[3];
+    pxy[5] = (sg[4] - ta[2]) - alpha * q[4];
+    pz[0] = (sg[2] + ta[1]) - alpha * q[2];
+    pz[1] = (sg[4] + ta[2]) - alpha * q[4];
+    pz[2] = alpha * (q[0] + q[3]) - (sg[0] + sg[3]);
+}
+
 // Plain populations: moments with the half-force correction, then Feq + Guo
 // forcing + BGK for every direction (ComputeMoments / ComputeFeqAndForcing /
 // PointwiseBGKCollide, src/physics_helpers.h:69-129). f[] in, f[] out.

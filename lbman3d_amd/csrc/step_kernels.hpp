@@ -147,8 +147,14 @@ __device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, 
 
 // ---- Q update ----------------------------------------------------------------
 // QTensorSolver::StepAndSetupBodyForce (src/qtensor_solver.tpp:50-147).
-// One cell. `own` false stores Sigma and Tau only (a halo cell of a region
+// One cell. `own` false stores the stresses only (a halo cell of a region
 // pass whose Q^{n+1} and Ericksen force belong to another launch).
+//
+// The stresses handed to the force kernel are Sigma and Tau in FP64. FP32
+// stores the eight independent components of the divergence form instead
+// (p_sets; zz = -xx - yy), in the same arrays: the force then needs 20
+// neighbour values rather than 52 and no Q^{n+1} (force kernel at 97x75x113:
+// 31.1 -> 26.3 us, at 256^3: 727 -> 557 us; FP64 keeps the reference's bits).
 //
 // Every load is issued before the first use, and the ghosts are selects: with
 // a branch per component and axis (uniform, but a branch) the loads of each
@@ -191,10 +197,20 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
     }
     T qn[5], sg[5], ta[3], fe[3];
     q_pointwise(k, Q, u, dq, g, qn, sg, ta, fe);
+    if constexpr (sizeof(T) == 4) {
+        T pxy[6], pz[3];
+        p_sets(k.alpha, qn, sg, ta, pxy, pz);
 #pragma unroll
-    for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, sg[m]);
+        for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, pxy[m]);
+        stn(f.tau[0], p.c, pxy[5]);
+        stn(f.tau[1], p.c, pz[0]);
+        stn(f.tau[2], p.c, pz[1]);
+    } else {
 #pragma unroll
-    for (int m = 0; m < 3; ++m) stn(f.tau[m], p.c, ta[m]);
+        for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, sg[m]);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) stn(f.tau[m], p.c, ta[m]);
+    }
     if (own) {
 #pragma unroll
         for (int m = 0; m < 5; ++m) stn(f.qn[m], p.c, qn[m]);
@@ -258,6 +274,97 @@ __global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc
 }
 
 // ---- body force and collide-stream ----------------------------------------
+// Both forms add the active and passive force to the Ericksen force in F.
+// FP64: differences of Q^{n+1}, Sigma and Tau in the reference's order.
+template <bool WALLS, typename T, typename Off>
+__device__ __forceinline__ void force_differences(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
+                                                  const Node<Off>& p, T F[3]) {
+    const int pos[3] = {p.x, p.y, p.z};
+    Off nb[7];
+    stencil<WALLS>(p, bc.n, bc.qkind, nb);
+    T v[13][7];
+#pragma unroll
+    for (int m = 0; m < 13; ++m) {
+        const T* a = m < 5 ? f.q[m] : (m < 10 ? f.sig[m - 5] : f.tau[m - 10]);
+#pragma unroll
+        for (int i = 0; i < 7; ++i) v[m][i] = ldn(a, nb[i]);
+    }
+    const T u[3] = {ldn(f.u[0], p.c), ldn(f.u[1], p.c), ldn(f.u[2], p.c)};
+    T dQ[5][3], dS[8][3];
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+        const Deriv<T> d =
+            q_deriv<T, !WALLS>(bc, m, pos, v[m][0], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) dQ[m][a] = d.d[a];
+    }
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) dS[m][a] = (v[5 + m][2 + 2 * a] - v[5 + m][1 + 2 * a]) / T(2.0);
+    const T fe[3] = {F[0], F[1], F[2]};
+    body_force(k, dQ, dS, u, fe, F);
+}
+
+// FP32: the divergence form, from the components qstep_cell stored.
+template <bool WALLS, typename T, typename Off>
+__device__ __forceinline__ void force_divergence(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
+                                                 const Node<Off>& p, T F[3]) {
+    Off nb[7];
+    stencil<WALLS>(p, bc.n, bc.qkind, nb);
+    // Array of component b of axis a's set: x (xx, yx, zx), y (xy, yy, zy), z (xz, yz, then zz = -xx - yy).
+    const T* const sets[3][4] = {{f.sig[0], f.sig[1], f.sig[2], nullptr},
+                                 {f.sig[3], f.sig[4], f.tau[0], nullptr},
+                                 {f.tau[1], f.tau[2], f.sig[0], f.sig[4]}};
+    T v[3][4][2];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < (a < 2 ? 3 : 4); ++b)
+#pragma unroll
+            for (int side = 0; side < 2; ++side) v[a][b][side] = ldn(sets[a][b], nb[1 + 2 * a + side]);
+    T d[3][3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        d[0][b] = v[0][b][1] - v[0][b][0];
+        d[1][b] = v[1][b][1] - v[1][b][0];
+    }
+    d[2][0] = v[2][0][1] - v[2][0][0];
+    d[2][1] = v[2][1][1] - v[2][1][0];
+    d[2][2] = (v[2][2][0] - v[2][2][1]) + (v[2][3][0] - v[2][3][1]);
+    if (WALLS && bc.q_ghosts) {
+        // Where the ghost of Q is not the value beyond the face that the
+        // stresses use (anchoring; a periodic high face opposite a wall), the
+        // set there holds -alpha times the wrong Q. The sets' Q components:
+        constexpr int qc[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, -1}};
+        const int pos[3] = {p.x, p.y, p.z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (bc.qkind[2 * a] == QB_PERIODIC) continue;
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                if (pos[a] != (side ? bc.n[a] - 1 : 0)) continue;
+                const int face = 2 * a + side;
+                const T sign = side ? -k.alpha : k.alpha;   // -alpha, and minus at the low side
+                auto off_by = [&](int c) {
+                    const T q0 = ldn(f.q[c], p.c);
+                    return (bc.qkind[face] == QB_ANCHOR ? T(2.0) * bc.anchor[face][c] - q0 : q0) - ldn(f.q[c], nb[1 + face]);
+                };
+#pragma unroll
+                for (int b = 0; b < 3; ++b)
+                    d[a][b] += sign * (qc[a][b] >= 0 ? off_by(qc[a][b]) : -(off_by(0) + off_by(3)));
+            }
+        }
+    }
+    T u[3] = {T(0), T(0), T(0)};
+    if (k.mu != T(0)) {
+#pragma unroll
+        for (int b = 0; b < 3; ++b) u[b] = ldn(f.u[b], p.c);
+    }
+#pragma unroll
+    for (int b = 0; b < 3; ++b) F[b] += T(0.5) * ((d[0][b] + d[1][b]) + d[2][b]) - k.mu * u[b];
+}
+
 // SetActiveStressAndComputeBodyForce (src/qtensor_solver.tpp:154-217) and
 // LatticeBoltzmannStep (src/lbm_solver.tpp:89-224) at one node. Fusing the two
 // is the merge the reference documents as valid (src/qtensor_solver.tpp:219-247):
@@ -274,31 +381,8 @@ __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<
     for (int m = 0; m < 3; ++m) F[m] = ldn(f.F[m], p.c);   // the Ericksen force, or the whole force
     if (flags & FL_FORCE) {
         if (k.force_full) {
-            const int pos[3] = {p.x, p.y, p.z};
-            Off nb[7];
-            stencil<WALLS>(p, bc.n, bc.qkind, nb);
-            T v[13][7];
-#pragma unroll
-            for (int m = 0; m < 13; ++m) {
-                const T* a = m < 5 ? f.q[m] : (m < 10 ? f.sig[m - 5] : f.tau[m - 10]);
-#pragma unroll
-                for (int i = 0; i < 7; ++i) v[m][i] = ldn(a, nb[i]);
-            }
-            const T u[3] = {ldn(f.u[0], p.c), ldn(f.u[1], p.c), ldn(f.u[2], p.c)};
-            T dQ[5][3], dS[8][3];
-#pragma unroll
-            for (int m = 0; m < 5; ++m) {
-                const Deriv<T> d =
-                    q_deriv<T, !WALLS>(bc, m, pos, v[m][0], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
-#pragma unroll
-                for (int a = 0; a < 3; ++a) dQ[m][a] = d.d[a];
-            }
-#pragma unroll
-            for (int m = 0; m < 8; ++m)
-#pragma unroll
-                for (int a = 0; a < 3; ++a) dS[m][a] = (v[5 + m][2 + 2 * a] - v[5 + m][1 + 2 * a]) / T(2.0);
-            const T fe[3] = {F[0], F[1], F[2]};
-            body_force(k, dQ, dS, u, fe, F);
+            if constexpr (sizeof(T) == 4) force_divergence<WALLS>(f, bc, k, p, F);
+            else force_differences<WALLS>(f, bc, k, p, F);
         }
         if (flags & FL_STORE_F) {
 #pragma unroll
@@ -325,7 +409,8 @@ __global__ void __launch_bounds__(kBlock)
 force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg, int store, int pull) {
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
-    force_lbm_cell<T, SHIFTED, false, WALLS>(f, bc, k, node_at<Off>(cg, c), FLAGS | store, pull);
+    force_lbm_cell<T, SHIFTED, false, WALLS>(f, bc, k, node_at<Off>(cg, c),
+                                               FLAGS | (store & (FL_STORE_F | FL_STORE_RHO)), pull);
 }
 
 template <typename T, bool WALLS, typename Off>

@@ -28,10 +28,13 @@ MIXED = abi.BCConfig(_W(abi.Neumann(), abi.Periodic()), _W(abi.Neumann(), abi.Pe
 LID = abi.BCConfig(_W(abi.Anchoring(0.4, 0.3, 1.1), abi.NoSlip()), _W(abi.Neumann(), abi.MovingWall(0.0, 0.02, -0.01)),
                    _W(abi.Periodic(), abi.Periodic()), _W(abi.Periodic(), abi.Periodic()),
                    _W(abi.Periodic(), abi.Periodic()), _W(abi.Periodic(), abi.Periodic()), "LidX")
+ONE_SIDED = abi.BCConfig(_W(abi.Neumann(), abi.NoSlip()), _W(abi.Periodic(), abi.NoSlip()),
+                         _W(abi.Periodic(), abi.NoSlip()), _W(abi.Anchoring(0.5, 0.9, 0.4), abi.NoSlip()),
+                         _W(abi.Anchoring(0.5, 0.9, 0.4), abi.Periodic()), _W(abi.Periodic(), abi.Periodic()), "OneSided")
 CASES = [(abi.FullyPeriodicConfig, (1, 1, 1)), (abi.FullyPeriodicConfig, (2, 1, 3)), (abi.FullyPeriodicConfig, (16, 16, 1)),
          (abi.FullyPeriodicConfig, (17, 5, 3)), (abi.FullyPeriodicConfig, (129, 2, 1)), (abi.ChannelConfig, (20, 13, 5)),
          (abi.SlitConfig, (64, 4, 2)), (abi.SlitNoSlipConfig, (65, 3, 4)), (BOX, (5, 7, 9)), (BOX, (3, 2, 2)),
-         (MIXED, (9, 6, 5)), (LID, (7, 11, 6)), (BC_BY_NAME["MovingLidZ"], (33, 4, 8)),
+         (MIXED, (9, 6, 5)), (ONE_SIDED, (8, 7, 6)), (ONE_SIDED, (2, 1, 1)), (LID, (7, 11, 6)), (BC_BY_NAME["MovingLidZ"], (33, 4, 8)),
          (BC_BY_NAME["AnchoredZ"], (10, 9, 2))]
 
 
