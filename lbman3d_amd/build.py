@@ -25,6 +25,7 @@ SOURCES = {
     "batch.hip": ["-ffp-contract=fast", "-x", "hip"],
     "closure.hip": ["-ffp-contract=fast"],
     "defects.hip": ["-ffp-contract=off"],
+    "transfer.hip": ["-ffp-contract=off"],
 }
 EXTRA: list[str] = []
 

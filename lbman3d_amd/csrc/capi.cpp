@@ -24,6 +24,7 @@
 #include "tile_map.hpp"
 #include "runtime.hpp"
 #include "solver_state.hpp"
+#include "transfer.hpp"
 
 using namespace lbm;
 
@@ -245,16 +246,6 @@ bool has_moving_wall(const lbm_config& c) {
     return false;
 }
 
-// Feq(rho, u) for one node in the reference's operand order
-// (Feq, src/physics_helpers.h:69-71; LbmSolver::Initialize, src/lbm_solver.tpp:59-87).
-void feq_host(double rho, double ux, double uy, double uz, double out[kQ]) {
-    const double u2 = ux * ux + uy * uy + uz * uz;
-    for (int i = 0; i < kQ; ++i) {
-        const double ue = ux * (double)cx(i) + uy * (double)cy(i) + uz * (double)cz(i);
-        out[i] = wgt(i) * rho * (1.0 + 3.0 * ue + 4.5 * ue * ue - 1.5 * u2);
-    }
-}
-
 }  // namespace lbm
 
 
@@ -317,42 +308,6 @@ int alloc_fields(lbm_solver* s, Fields<T>& f) {
 
 // What the density array is stored relative to (rho0 for FP32, 0 for FP64).
 double rho_base(const lbm_solver* s) { return s->fp64 ? 0.0 : s->cfg.p.density; }
-
-int fill_value(lbm_solver* s, void* dst, double v) {
-    std::vector<char> host(s->V * s->esize());
-    if (s->fp64) std::fill((double*)host.data(), (double*)host.data() + s->V, v);
-    else std::fill((float*)host.data(), (float*)host.data() + s->V, (float)v);
-    HIPCHK(hipMemcpyAsync(dst, host.data(), host.size(), hipMemcpyHostToDevice, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
-    return LBM_OK;
-}
-
-// Copy an FP64 host block of n values into a device field of the handle's
-// type; an FP32 field stores src - base (the density keeps rho - rho0).
-int put_field(lbm_solver* s, void* dst, const double* src, long n, double base = 0.0) {
-    if (s->fp64) {
-        HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    } else {
-        std::vector<float> tmp(n);
-        for (long i = 0; i < n; ++i) tmp[i] = (float)(src[i] - base);
-        HIPCHK(hipMemcpyAsync(dst, tmp.data(), n * sizeof(float), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    }
-    return LBM_OK;
-}
-int get_field(lbm_solver* s, double* dst, const void* src, long n, double base = 0.0) {
-    if (s->fp64) {
-        HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    } else {
-        std::vector<float> tmp(n);
-        HIPCHK(hipMemcpyAsync(tmp.data(), src, n * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-        for (long i = 0; i < n; ++i) dst[i] = base + (double)tmp[i];
-    }
-    return LBM_OK;
-}
 
 void* field_ptr(lbm_solver* s, int which, int comp) {
     // which: 0 rho, 1 u, 2 q, 3 F
@@ -573,6 +528,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
     if (ndev < 1) return fail(LBM_ERR_HIP, "no HIP device");
 
     lbm_solver* s = new lbm_solver();
+    staging_open();
     s->cfg = *cfg;
     s->V = (long)cfg->nx * cfg->ny * cfg->nz;
     s->vs = (s->V + 63) / 64 * 64 + kStagger;   // population planes staggered like the arrays
@@ -636,9 +592,7 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
     s->k32 = make_phys<float>(*cfg);
     // FluidFields constructor state (src/fluid_fields.cc:6-17): rho = kDensity,
     // u = F = 0, populations Feq(rho0, 0).
-    if ((r = fill_value(s, field_ptr(s, 0, 0), cfg->p.density - rho_base(s)))) return cleanup(r);
-    std::vector<double> rho(s->V, cfg->p.density);
-    if ((r = lbm_upload_state(s, rho.data(), nullptr, nullptr, nullptr, nullptr))) return cleanup(r);
+    if ((r = put_rest(s))) return cleanup(r);
     *out = s;
     return LBM_OK;
 }
@@ -648,6 +602,7 @@ int lbm_destroy(lbm_handle s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     for (void* p : s->allocs) (void)hipFree(p);
     if (s->stream) (void)hipStreamDestroy(s->stream);
+    staging_close();
     delete s;
     return LBM_OK;
 }
@@ -675,65 +630,23 @@ int lbm_device_info(char* buf, size_t len) {
 int lbm_upload_state(lbm_handle s, const double* rho, const double* ux, const double* uy, const double* uz,
                      const double* q) {
     if (!s) return fail(LBM_ERR_INVALID, "null handle");
-    const long V = s->V;
-    int r;
-    if (rho && (r = put_field(s, field_ptr(s, 0, 0), rho, V, rho_base(s)))) return r;
-    const double* uu[3] = {ux, uy, uz};
-    for (int a = 0; a < 3; ++a)
-        if (uu[a] && (r = put_field(s, field_ptr(s, 1, a), uu[a], V))) return r;
-    if (q)
-        for (int m = 0; m < 5; ++m)
-            if ((r = put_field(s, field_ptr(s, 2, m), q + m * V, V))) return r;
-    // Populations = Feq(rho, u) of the (now current) device state.
-    std::vector<double> hr(V), hu[3];
-    if ((r = get_field(s, hr.data(), field_ptr(s, 0, 0), V, rho_base(s)))) return r;
-    for (int a = 0; a < 3; ++a) {
-        hu[a].resize(V);
-        if ((r = get_field(s, hu[a].data(), field_ptr(s, 1, a), V))) return r;
-    }
-    // For FP32 the device copy of rho/u is rounded; Feq is formed from the
-    // FP64 inputs where given so the shifted populations carry full precision.
-    const double* src_r = rho ? rho : hr.data();
-    const double* src_u[3] = {ux ? ux : hu[0].data(), uy ? uy : hu[1].data(), uz ? uz : hu[2].data()};
-    if (s->fp64) {
-        std::vector<double> g(kQ * s->vs, 0.0);
-        double fe[kQ];
-        for (long c = 0; c < V; ++c) {
-            feq_host(src_r[c], src_u[0][c], src_u[1][c], src_u[2][c], fe);
-            for (int i = 0; i < kQ; ++i) g[i * s->vs + c] = fe[i];
-        }
-        HIPCHK(hipMemcpyAsync(s->d64.g, g.data(), g.size() * sizeof(double), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    } else {
-        std::vector<float> g(kQ * s->vs, 0.0f);
-        double fe[kQ];
-        const double r0 = s->cfg.p.density;
-        for (long c = 0; c < V; ++c) {
-            feq_host(src_r[c], src_u[0][c], src_u[1][c], src_u[2][c], fe);
-            for (int i = 0; i < kQ; ++i) g[i * s->vs + c] = (float)(fe[i] - wgt(i) * r0);
-        }
-        HIPCHK(hipMemcpyAsync(s->d32.g, g.data(), g.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
-        HIPCHK(hipStreamSynchronize(s->stream));
-    }
+    // Feq is formed from the FP64 inputs where given (the device's copy of an
+    // FP32 run is rounded), so the shifted populations carry full precision.
+    const double* const u[3] = {ux, uy, uz};
+    if (int r = put_state(s, rho, u, q)) return r;
     s->pulled = 0;
     return LBM_OK;
 }
 
+// Population i of the handle's stored form is f_i less this.
+static double pop_base(const lbm_solver* s, int i) { return s->fp64 ? 0.0 : wgt(i) * s->cfg.p.density; }
+
 int lbm_upload_populations(lbm_handle s, const double* f) {
     if (!s || !f) return fail(LBM_ERR_INVALID, "null argument");
-    const long V = s->V;
-    if (s->fp64) {
-        std::vector<double> g(kQ * s->vs, 0.0);
-        for (int i = 0; i < kQ; ++i) std::memcpy(&g[i * s->vs], f + i * V, V * sizeof(double));
-        HIPCHK(hipMemcpyAsync(s->d64.g, g.data(), g.size() * sizeof(double), hipMemcpyHostToDevice, s->stream));
-    } else {
-        std::vector<float> g(kQ * s->vs, 0.0f);
-        const double r0 = s->cfg.p.density;
-        for (int i = 0; i < kQ; ++i)
-            for (long c = 0; c < V; ++c) g[i * s->vs + c] = (float)(f[i * V + c] - wgt(i) * r0);
-        HIPCHK(hipMemcpyAsync(s->d32.g, g.data(), g.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    }
-    HIPCHK(hipStreamSynchronize(s->stream));
+    PutItem items[kQ];
+    for (int i = 0; i < kQ; ++i)
+        items[i] = {(char*)s->gptr() + i * s->vs * s->esize(), f + i * s->V, pop_base(s, i)};
+    if (int r = put_fields(s, items, kQ)) return r;
     s->pulled = 0;
     return LBM_OK;
 }
@@ -741,68 +654,47 @@ int lbm_upload_populations(lbm_handle s, const double* f) {
 int lbm_upload_force(lbm_handle s, const double* fx, const double* fy, const double* fz) {
     if (!s) return fail(LBM_ERR_INVALID, "null handle");
     const double* ff[3] = {fx, fy, fz};
+    PutItem items[3];
+    int n = 0;
     for (int a = 0; a < 3; ++a)
-        if (ff[a])
-            if (int r = put_field(s, field_ptr(s, 3, a), ff[a], s->V)) return r;
-    return LBM_OK;
+        if (ff[a]) items[n++] = {field_ptr(s, 3, a), ff[a], 0.0};
+    return put_fields(s, items, n);
 }
 
 int lbm_download_state(lbm_handle s, double* rho, double* ux, double* uy, double* uz, double* q) {
     if (!s) return fail(LBM_ERR_INVALID, "null handle");
-    const long V = s->V;
-    int r;
-    if (rho && (r = get_field(s, rho, field_ptr(s, 0, 0), V, rho_base(s)))) return r;
+    FetchItem items[9];
+    int n = 0;
+    if (rho) items[n++] = {field_ptr(s, 0, 0), rho, rho_base(s)};
     double* uu[3] = {ux, uy, uz};
     for (int a = 0; a < 3; ++a)
-        if (uu[a] && (r = get_field(s, uu[a], field_ptr(s, 1, a), V))) return r;
+        if (uu[a]) items[n++] = {field_ptr(s, 1, a), uu[a], 0.0};
     if (q)
-        for (int m = 0; m < 5; ++m)
-            if ((r = get_field(s, q + m * V, field_ptr(s, 2, m), V))) return r;
-    return LBM_OK;
+        for (int m = 0; m < 5; ++m) items[n++] = {field_ptr(s, 2, m), q + m * s->V, 0.0};
+    return fetch_fields(s, items, n);
 }
 
 int lbm_download_force(lbm_handle s, double* fx, double* fy, double* fz) {
     if (!s) return fail(LBM_ERR_INVALID, "null handle");
     double* ff[3] = {fx, fy, fz};
+    FetchItem items[3];
+    int n = 0;
     for (int a = 0; a < 3; ++a)
-        if (ff[a])
-            if (int r = get_field(s, ff[a], field_ptr(s, 3, a), s->V)) return r;
-    return LBM_OK;
+        if (ff[a]) items[n++] = {field_ptr(s, 3, a), ff[a], 0.0};
+    return fetch_fields(s, items, n);
 }
 
 int lbm_download_populations(lbm_handle s, double* f) {
     if (!s || !f) return fail(LBM_ERR_INVALID, "null argument");
-    const long V = s->V;
     void* tmp = nullptr;
     HIPCHK(hipMalloc(&tmp, kQ * s->vs * s->esize()));
+    auto release = scope_exit([&] { (void)hipFree(tmp); });
     if (s->fp64) launch_stream_only(s->d64, s->bc64, s->pulled, (double*)tmp, s->stream);
     else launch_stream_only(s->d32, s->bc32, s->pulled, (float*)tmp, s->stream);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) {
-        (void)hipFree(tmp);
-        return fail(LBM_ERR_HIP, std::string("stream_only launch: ") + hipGetErrorString(e));
-    }
-    int r = LBM_OK;
-    if (s->fp64) {
-        std::vector<double> g(kQ * s->vs);
-        if (hipMemcpyAsync(g.data(), tmp, g.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-            hipStreamSynchronize(s->stream) != hipSuccess)
-            r = fail(LBM_ERR_HIP, "population download failed");
-        else
-            for (int i = 0; i < kQ; ++i) std::memcpy(f + i * V, &g[i * s->vs], V * sizeof(double));
-    } else {
-        std::vector<float> g(kQ * s->vs);
-        if (hipMemcpyAsync(g.data(), tmp, g.size() * sizeof(float), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-            hipStreamSynchronize(s->stream) != hipSuccess)
-            r = fail(LBM_ERR_HIP, "population download failed");
-        else {
-            const double r0 = s->cfg.p.density;
-            for (int i = 0; i < kQ; ++i)
-                for (long c = 0; c < V; ++c) f[i * V + c] = (double)g[i * s->vs + c] + wgt(i) * r0;
-        }
-    }
-    (void)hipFree(tmp);
-    return r;
+    HIPCHK(hipGetLastError());
+    FetchItem items[kQ];
+    for (int i = 0; i < kQ; ++i) items[i] = {(char*)tmp + i * s->vs * s->esize(), f + i * s->V, pop_base(s, i)};
+    return fetch_fields(s, items, kQ);
 }
 
 int lbm_qtensor_step(lbm_handle s) {
@@ -874,20 +766,7 @@ int lbm_diagnostics(lbm_handle s, lbm_diag* out) {
 
 int lbm_order_director(lbm_handle s, double* order, double* director) {
     if (!s || !order || !director) return fail(LBM_ERR_INVALID, "null argument");
-    void* tmp = nullptr;
-    HIPCHK(hipMalloc(&tmp, 4 * s->V * sizeof(double)));
-    double* o = (double*)tmp;
-    double* d = o + s->V;
-    if (s->fp64) launch_order_director(s->d64, s->V, o, d, s->stream);
-    else launch_order_director(s->d32, s->V, o, d, s->stream);
-    int r = LBM_OK;
-    if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(order, o, s->V * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-        hipMemcpyAsync(director, d, 3 * s->V * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-        hipStreamSynchronize(s->stream) != hipSuccess)
-        r = fail(LBM_ERR_HIP, "order/director failed");
-    (void)hipFree(tmp);
-    return r;
+    return fetch_order_director(s, order, director);
 }
 
 // ---- order/director without device allocation --------------------------------
@@ -932,8 +811,8 @@ int lbm_order_director_noalloc(lbm_handle s, double* order, double* director) {
     if (int r = scratch_for_current_device(&base)) return r;
     double* o = base;
     double* d = base + s->V;
-    if (s->fp64) launch_order_director(s->d64, s->V, o, d, s->stream);
-    else launch_order_director(s->d32, s->V, o, d, s->stream);
+    if (s->fp64) launch_order_director(s->d64, 0, s->V, o, d, s->stream);
+    else launch_order_director(s->d32, 0, s->V, o, d, s->stream);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(order, o, s->V * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
         hipMemcpyAsync(director, d, 3 * s->V * sizeof(double), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||

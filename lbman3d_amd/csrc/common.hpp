@@ -63,6 +63,16 @@ __host__ __device__ inline int node_class(int x, int y, int z, int nx, int ny, i
     return a | (b << 2) | (c << 4);
 }
 
+// Feq(rho, u) of one node in the reference's operand order (Feq,
+// src/physics_helpers.h:69-71; LbmSolver::Initialize, src/lbm_solver.tpp:59-87).
+__host__ __device__ inline void feq_node(double rho, double ux, double uy, double uz, double out[kQ]) {
+    const double u2 = ux * ux + uy * uy + uz * uz;
+    for (int i = 0; i < kQ; ++i) {
+        const double ue = ux * (double)cx(i) + uy * (double)cy(i) + uz * (double)cz(i);
+        out[i] = wgt(i) * rho * (1.0 + 3.0 * ue + 4.5 * ue * ue - 1.5 * u2);
+    }
+}
+
 // Quotient of n < 2^31 by a fixed divisor as a multiply and a shift: with
 // l = ceil(log2 d) and m = ceil(2^(31 + l) / d) the error of n m / 2^(31 + l)
 // stays below 1 / d.

@@ -66,8 +66,8 @@ extern "C" int lbm_defect_faces(lbm_handle s, uint8_t* def_x, uint8_t* def_y, ui
     double* order = (double*)tmp;
     double* dir = order + V;
     uint8_t* faces = (uint8_t*)(dir + 3 * V);
-    if (s->fp64) launch_order_director(s->d64, V, order, dir, s->stream);
-    else launch_order_director(s->d32, V, order, dir, s->stream);
+    if (s->fp64) launch_order_director(s->d64, 0, V, order, dir, s->stream);
+    else launch_order_director(s->d32, 0, V, order, dir, s->stream);
     uint8_t* host[3] = {def_x, def_y, def_z};
     long o = 0;
     for (int fam = 0; fam < 3; ++fam) {

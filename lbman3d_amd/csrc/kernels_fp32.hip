@@ -9,5 +9,5 @@ template void launch_force_lbm<float, true>(const Fields<float>&, const BCDesc<f
 template void launch_stream_only<float>(const Fields<float>&, const BCDesc<float>&, int, float*, hipStream_t);
 template void launch_diagnostics<float>(const Fields<float>&, const BCDesc<float>&, const Phys<double>&, long,
                                         double*, double*, int, double*, hipStream_t);
-template void launch_order_director<float>(const Fields<float>&, long, double*, double*, hipStream_t);
+template void launch_order_director<float>(const Fields<float>&, long, long, double*, double*, hipStream_t);
 }  // namespace lbm

@@ -11,7 +11,7 @@ template void launch_force_lbm<double, false>(const Fields<double>&, const BCDes
 template void launch_stream_only<double>(const Fields<double>&, const BCDesc<double>&, int, double*, hipStream_t);
 template void launch_diagnostics<double>(const Fields<double>&, const BCDesc<double>&, const Phys<double>&, long,
                                          double*, double*, int, double*, hipStream_t);
-template void launch_order_director<double>(const Fields<double>&, long, double*, double*, hipStream_t);
+template void launch_order_director<double>(const Fields<double>&, long, long, double*, double*, hipStream_t);
 
 // FP64 tile catalogue of the fused step (first pipeline, periodic
 // specialisation). Rows of 16 doubles are one 128-byte line.

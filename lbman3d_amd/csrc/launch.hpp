@@ -31,9 +31,10 @@ template <typename T>
 void launch_diagnostics(const Fields<T>& f, const BCDesc<T>& bc, const Phys<double>& k, long V,
                         double* uprev, double* partials, int nblocks, double* out, hipStream_t s);
 
-// Order parameter and director per cell in FP64.
+// Order parameter and director in FP64 of n cells from c0 on, into order[n] and
+// director[n][3] (device or pinned host memory).
 template <typename T>
-void launch_order_director(const Fields<T>& f, long V, double* order, double* director, hipStream_t s);
+void launch_order_director(const Fields<T>& f, long c0, long n, double* order, double* director, hipStream_t s);
 
 // Fused single-kernel FP32 step (Q update + body force + collide-stream).
 // tile: index of the tile shape (see fused_tile_count()).

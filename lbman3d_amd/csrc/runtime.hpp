@@ -27,7 +27,6 @@ BCDesc<T> make_bc(const lbm_config& c);
 template <typename T>
 Phys<T> make_phys(const lbm_config& c);
 bool has_moving_wall(const lbm_config& c);
-void feq_host(double rho, double ux, double uy, double uz, double out[kQ]);
 
 // splitmix64 finaliser (Steele, Lea, Flood; "Fast splittable pseudorandom
 // number generators", OOPSLA 2014).

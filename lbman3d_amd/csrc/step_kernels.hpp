@@ -520,9 +520,13 @@ __global__ void __launch_bounds__(64) diag_final_kernel(const double* partials, 
 // QtensorToOrderDirector (src/analysis_fields.cc:59-93) in FP64.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-order_director_kernel(Fields<T> f, long V, double* order, double* director) {
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= V) return;
+order_director_kernel(Fields<T> f, long c0, long n, double* order, double* director) {
+    // The directors leave through LDS, so that a wavefront writes whole lines
+    // (the target may be host memory).
+    __shared__ double out[3 * kBlock];
+    const long first = (long)blockIdx.x * kBlock;
+    const int t = threadIdx.x, cells = (int)min((long)kBlock, n - first);
+    const long c = c0 + first + min(t, cells - 1);
     const double Qxx = f.q[0][c], Qxy = f.q[1][c], Qxz = f.q[2][c], Qyy = f.q[3][c], Qyz = f.q[4][c];
     const double pp = Qxx * Qxx + Qxx * Qyy + Qyy * Qyy + Qxy * Qxy + Qxz * Qxz + Qyz * Qyz;
     const double qd = -(Qxx + Qyy) * (Qxx * Qyy - Qxy * Qxy) - Qyy * Qxz * Qxz - Qxx * Qyz * Qyz + 2 * Qxy * Qxz * Qyz;
@@ -534,10 +538,12 @@ order_director_kernel(Fields<T> f, long V, double* order, double* director) {
     double nyv = Qyz * (Qxx - S) - Qxy * Qxz;
     double nzv = Qxy * Qxy - (Qxx - S) * (Qyy - S);
     const double inv = 1.0 / sqrt(nxv * nxv + nyv * nyv + nzv * nzv);
-    order[c] = S;
-    director[3 * c + 0] = nxv * inv;
-    director[3 * c + 1] = nyv * inv;
-    director[3 * c + 2] = nzv * inv;
+    if (t < cells) order[first + t] = S;
+    out[3 * t + 0] = nxv * inv;
+    out[3 * t + 1] = nyv * inv;
+    out[3 * t + 2] = nzv * inv;
+    __syncthreads();
+    for (int i = t; i < 3 * cells; i += kBlock) director[3 * first + i] = out[i];
 }
 
 // ---- launchers ---------------------------------------------------------------
@@ -602,8 +608,8 @@ void launch_diagnostics(const Fields<T>& f, const BCDesc<T>& bc, const Phys<doub
 }
 
 template <typename T>
-void launch_order_director(const Fields<T>& f, long V, double* order, double* director, hipStream_t s) {
-    hipLaunchKernelGGL(order_director_kernel<T>, dim3(grid_for(V)), dim3(kBlock), 0, s, f, V, order, director);
+void launch_order_director(const Fields<T>& f, long c0, long n, double* order, double* director, hipStream_t s) {
+    hipLaunchKernelGGL(order_director_kernel<T>, dim3(grid_for(n)), dim3(kBlock), 0, s, f, c0, n, order, director);
 }
 
 }  // namespace lbm

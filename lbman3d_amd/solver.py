@@ -206,15 +206,14 @@ class DeviceSolver:
 
     def state(self):
         V = self.V
-        rho, ux, uy, uz = (np.empty(V) for _ in range(4))
-        q = np.empty(5 * V)
-        check(lib().lbm_download_state(self.h, _p(rho), _p(ux), _p(uy), _p(uz), _p(q)))
-        return {"rho": rho, "u": np.stack([ux, uy, uz]), "q": q.reshape(5, V)}
+        rho, u, q = np.empty(V), np.empty((3, V)), np.empty((5, V))
+        check(lib().lbm_download_state(self.h, _p(rho), _p(u[0]), _p(u[1]), _p(u[2]), _p(q)))
+        return {"rho": rho, "u": u, "q": q}
 
     def force(self):
-        F = [np.empty(self.V) for _ in range(3)]
+        F = np.empty((3, self.V))
         check(lib().lbm_download_force(self.h, *[_p(x) for x in F]))
-        return np.stack(F)
+        return F
 
     def populations(self):
         f = np.empty(15 * self.V)
@@ -343,10 +342,9 @@ class BatchSolver:
 
     def state(self, i):
         V = self._V(i)
-        rho, ux, uy, uz = (np.empty(V) for _ in range(4))
-        q = np.empty(5 * V)
-        check(lib().lbm_batch_download_state(self.h, i, _p(rho), _p(ux), _p(uy), _p(uz), _p(q)))
-        return {"rho": rho, "u": np.stack([ux, uy, uz]), "q": q.reshape(5, V)}
+        rho, u, q = np.empty(V), np.empty((3, V)), np.empty((5, V))
+        check(lib().lbm_batch_download_state(self.h, i, _p(rho), _p(u[0]), _p(u[1]), _p(u[2]), _p(q)))
+        return {"rho": rho, "u": u, "q": q}
 
     def diagnostics(self, i) -> dict:
         d = LbmDiag()
