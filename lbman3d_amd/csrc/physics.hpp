@@ -74,15 +74,17 @@ __device__ __forceinline__ T u_ghost(const BCDesc<T>& bc, int face, int comp, bo
     const T reflected = T(2.0) * bc.wall_u[face][comp] - vb;
     return (bc.ukind[face] == UB_SPECULAR && !normal) ? vb : reflected;
 }
+template <typename T>
+__device__ __forceinline__ void u_pair(const BCDesc<T>& bc, int a, int comp, int i, T vm, T v0, T vp, T& m, T& p) {
+    const bool walls = bc.ukind[2 * a] != UB_PERIODIC, normal = comp == a;
+    const T gm = u_ghost(bc, 2 * a, comp, normal, v0), gp = u_ghost(bc, 2 * a + 1, comp, normal, v0);
+    m = (walls & (i == 0)) ? gm : vm;
+    p = (walls & (i == bc.n[a] - 1)) ? gp : vp;
+}
 template <typename T, bool NOGHOST = false>
 __device__ __forceinline__ T u_grad(const BCDesc<T>& bc, int a, int comp, int i, T vm, T v0, T vp) {
     T m = vm, p = vp;
-    if (!NOGHOST) {
-        const bool walls = bc.ukind[2 * a] != UB_PERIODIC, normal = comp == a;
-        const T gm = u_ghost(bc, 2 * a, comp, normal, v0), gp = u_ghost(bc, 2 * a + 1, comp, normal, v0);
-        m = (walls & (i == 0)) ? gm : vm;
-        p = (walls & (i == bc.n[a] - 1)) ? gp : vp;
-    }
+    if (!NOGHOST) u_pair(bc, a, comp, i, vm, v0, vp, m, p);
     return (p - m) / T(2.0);
 }
 

@@ -145,6 +145,32 @@ __device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, 
     }
 }
 
+// Ghosts of a node's stencil values, v[i] as `stencil` numbers them: the values
+// beyond a wall replace what the stencil read there. Called under a branch
+// that only wavefronts with a cell on a wall take, after every load is issued:
+// with the selects in line, the wall constants and lane masks of all components
+// spilled 90 scalar registers and the FP64 Q kernel held 202 vector registers.
+template <typename T>
+__device__ __forceinline__ void q_ghosts(const BCDesc<T>& bc, const int pos[3], int c, T v[7]) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) q_pair(bc, a, c, pos[a], v[1 + 2 * a], v[0], v[2 + 2 * a], v[1 + 2 * a], v[2 + 2 * a]);
+}
+template <typename T>
+__device__ __forceinline__ void u_ghosts(const BCDesc<T>& bc, const int pos[3], int comp, T v[7]) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) u_pair(bc, a, comp, pos[a], v[1 + 2 * a], v[0], v[2 + 2 * a], v[1 + 2 * a], v[2 + 2 * a]);
+}
+// Whether a cell lies on the first or last plane of an axis with a wall.
+__device__ __forceinline__ bool on_wall(const int pos[3], const int n[3], const int qkind[6], const int ukind[6]) {
+    bool on = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool walls = (qkind[2 * a] | qkind[2 * a + 1] | ukind[2 * a] | ukind[2 * a + 1]) != 0;
+        on |= walls & ((pos[a] == 0) | (pos[a] == n[a] - 1));
+    }
+    return on;
+}
+
 // ---- Q update ----------------------------------------------------------------
 // QTensorSolver::StepAndSetupBodyForce (src/qtensor_solver.tpp:50-147).
 // One cell. `own` false stores the stresses only (a halo cell of a region
@@ -180,12 +206,18 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
     for (int A = 0; A < 3; ++A)
 #pragma unroll
         for (int i = 0; i < 7; ++i) v[5 + A][i] = ldn(f.u[A], us[i]);
+    if (WALLS && __builtin_amdgcn_ballot_w64(on_wall(pos, bc.n, bc.qkind, bc.ukind)) != 0) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) q_ghosts(bc, pos, m, v[m]);
+#pragma unroll
+        for (int A = 0; A < 3; ++A) u_ghosts(bc, pos, A, v[5 + A]);
+    }
     T Q[5];
     Deriv<T> dq[5];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         Q[m] = v[m][0];
-        dq[m] = q_deriv<T, !WALLS>(bc, m, pos, Q[m], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
+        dq[m] = q_deriv<T, true>(bc, m, pos, Q[m], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
     }
     T u[3], g[3][3];
 #pragma unroll
@@ -193,7 +225,7 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
         u[A] = v[5 + A][0];
 #pragma unroll
         for (int B = 0; B < 3; ++B)
-            g[A][B] = u_grad<T, !WALLS>(bc, B, A, pos[B], v[5 + A][1 + 2 * B], u[A], v[5 + A][2 + 2 * B]);
+            g[A][B] = u_grad<T, true>(bc, B, A, pos[B], v[5 + A][1 + 2 * B], u[A], v[5 + A][2 + 2 * B]);
     }
     T qn[5], sg[5], ta[3], fe[3];
     q_pointwise(k, Q, u, dq, g, qn, sg, ta, fe);
