@@ -741,7 +741,7 @@ shell_force_lbm_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRe
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    force_lbm_cell<float, true, true, true>(f, bc, k, shell_node(q, bc.n), flags, pull);
+    force_lbm_cell<float, true, true, true, true>(f, bc, k, shell_node(q, bc.n), flags, pull);
 }
 #endif  // LBM_FUSED_BODY_ONLY
 

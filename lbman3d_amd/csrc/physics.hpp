@@ -138,85 +138,115 @@ __device__ __forceinline__ T adv_axis(int upwind, T u, T dq, T d2q) {
 }
 
 // Beris-Edwards pointwise update, stresses and Ericksen force
-// (PointwiseStepAndSetupBodyForce, src/model.h:102-342).
+// (PointwiseStepAndSetupBodyForce, src/model.h:102-342), in three parts so that
+// a kernel can take the five components one after another: q_rates from the
+// velocity gradient, q_component for each component in the order xx, xy, xz,
+// yy, yz, then q_finish.
+template <typename T>
+struct QRates {
+    T TrQ2, Q2[5], ld;        // tr Q^2, Q^2 - I tr Q^2 / 3, A + C tr Q^2
+    T E[5], W[3];             // strain rate (xx, xy, xz, yy, yz), vorticity (xy, xz, yz)
+    T H[5], advc[5], hd[3];   // molecular field, advection, partial sums of H : grad Q
+    T d0[3], d3[3];           // grad Qxx and grad Qyy
+};
 // g[A][B] = d u_A / d x_B with g[2][2] unused.
 template <typename T>
-__device__ __forceinline__ void q_pointwise(const Phys<T>& k, const T Q[5], const T u[3],
-                                            const Deriv<T> dq[5], const T g[3][3],
-                                            T qn[5], T sg[5], T ta[3], T fe[3]) {
+__device__ __forceinline__ void q_rates(const Phys<T>& k, const T Q[5], const T g[3][3], QRates<T>& r) {
     const T Qxx = Q[0], Qxy = Q[1], Qxz = Q[2], Qyy = Q[3], Qyz = Q[4];
-    const T TrQ2 = T(2.0) * (Qxx * Qxx + Qyy * Qyy + Qxx * Qyy + Qxy * Qxy + Qxz * Qxz + Qyz * Qyz);
+    r.TrQ2 = T(2.0) * (Qxx * Qxx + Qyy * Qyy + Qxx * Qyy + Qxy * Qxy + Qxz * Qxz + Qyz * Qyz);
     const T third = T(1.0 / 3.0);
-    const T Q2xx = Qxx * Qxx + Qxy * Qxy + Qxz * Qxz - third * TrQ2;
-    const T Q2xy = Qxx * Qxy + Qxy * Qyy + Qxz * Qyz;
-    const T Q2xz = Qxy * Qyz - Qxz * Qyy;
-    const T Q2yy = Qxy * Qxy + Qyy * Qyy + Qyz * Qyz - third * TrQ2;
-    const T Q2yz = Qxy * Qxz - Qyz * Qxx;
-    const T Q2[5] = {Q2xx, Q2xy, Q2xz, Q2yy, Q2yz};
-
-    const T Exx = g[0][0];
-    const T Exy = T(0.5) * (g[0][1] + g[1][0]);
-    const T Exz = T(0.5) * (g[0][2] + g[2][0]);
-    const T Eyy = g[1][1];
-    const T Eyz = T(0.5) * (g[1][2] + g[2][1]);
-    const T Wxy = T(0.5) * (g[0][1] - g[1][0]);
-    const T Wxz = T(0.5) * (g[0][2] - g[2][0]);
-    const T Wyz = T(0.5) * (g[1][2] - g[2][1]);
-    const T E[5] = {Exx, Exy, Exz, Eyy, Eyz};
-
-    T advc[5];
+    r.Q2[0] = Qxx * Qxx + Qxy * Qxy + Qxz * Qxz - third * r.TrQ2;
+    r.Q2[1] = Qxx * Qxy + Qxy * Qyy + Qxz * Qyz;
+    r.Q2[2] = Qxy * Qyz - Qxz * Qyy;
+    r.Q2[3] = Qxy * Qxy + Qyy * Qyy + Qyz * Qyz - third * r.TrQ2;
+    r.Q2[4] = Qxy * Qxz - Qyz * Qxx;
+    r.ld = k.A + k.C * r.TrQ2;
+    r.E[0] = g[0][0];
+    r.E[1] = T(0.5) * (g[0][1] + g[1][0]);
+    r.E[2] = T(0.5) * (g[0][2] + g[2][0]);
+    r.E[3] = g[1][1];
+    r.E[4] = T(0.5) * (g[1][2] + g[2][1]);
+    r.W[0] = T(0.5) * (g[0][1] - g[1][0]);
+    r.W[1] = T(0.5) * (g[0][2] - g[2][0]);
+    r.W[2] = T(0.5) * (g[1][2] - g[2][1]);
+}
+template <typename T>
+__device__ __forceinline__ void q_component(const Phys<T>& k, int c, T Qc, const T u[3], const Deriv<T>& dq,
+                                            QRates<T>& r) {
+    r.advc[c] = -(adv_axis(k.advection, u[0], dq.d[0], dq.d2[0]) + adv_axis(k.advection, u[1], dq.d[1], dq.d2[1])
+                  + adv_axis(k.advection, u[2], dq.d[2], dq.d2[2]));
+    r.H[c] = k.L * dq.lap - r.ld * Qc - k.B * r.Q2[c];
 #pragma unroll
-    for (int c = 0; c < 5; ++c)
-        advc[c] = -(adv_axis(k.advection, u[0], dq[c].d[0], dq[c].d2[0])
-                    + adv_axis(k.advection, u[1], dq[c].d[1], dq[c].d2[1])
-                    + adv_axis(k.advection, u[2], dq[c].d[2], dq[c].d2[2]));
-
-    const T cor[5] = {T(2.0) * (Qxy * Wxy + Qxz * Wxz),
-                      -Qxx * Wxy + Qxz * Wyz + Qyy * Wxy + Qyz * Wxz,
-                      T(-2.0) * Qxx * Wxz - Qxy * Wyz - Qyy * Wxz + Qyz * Wxy,
-                      T(2.0) * (-Qxy * Wxy + Qyz * Wyz),
-                      -Qxx * Wyz - Qxy * Wxz - Qxz * Wxy - T(2.0) * Qyy * Wyz};
-
-    const T two3 = T(2.0 / 3.0);
-    const T trQE = (T(2.0) * Exx + Eyy) * Qxx + (T(2.0) * Exy) * Qxy + (T(2.0) * Exz) * Qxz
-                 + (Exx + T(2.0) * Eyy) * Qyy + T(2.0) * Eyz * Qyz;
-    const T aln2[5] = {
-        T(2.0) * (Exx * Qxx + Exy * Qxy + Exz * Qxz) - two3 * trQE,
-        Exy * Qxx + Eyy * Qxy + Eyz * Qxz + Qxy * Exx + Qyy * Exy + Qyz * Exz,
-        Exz * Qxx + Eyz * Qxy + (-Exx - Eyy) * Qxz + Qxz * Exx + Qyz * Exy + (-Qxx - Qyy) * Exz,
-        T(2.0) * (Exy * Qxy + Eyy * Qyy + Eyz * Qyz) - two3 * trQE,
-        Exz * Qxy + Eyz * Qyy + (-Exx - Eyy) * Qyz + Qxz * Exy + Qyz * Eyy + (-Qxx - Qyy) * Eyz};
-
-    const T ld = k.A + k.C * TrQ2;
-    T H[5];
+    for (int a = 0; a < 3; ++a) {
+        r.hd[a] = c == 0 ? r.H[c] * dq.d[a] : r.hd[a] + r.H[c] * dq.d[a];
+        if (c == 0) r.d0[a] = dq.d[a];
+        if (c == 3) r.d3[a] = dq.d[a];
+    }
+}
+// Results of component c go to emit(c, Q^{n+1}, Sigma).
+template <typename T, typename F>
+__device__ __forceinline__ void q_finish(const Phys<T>& k, const T Q[5], const QRates<T>& r, T ta[3], T fe[3],
+                                         F&& emit) {
+    const T Qxx = Q[0], Qxy = Q[1], Qxz = Q[2], Qyy = Q[3], Qyz = Q[4];
+    const T Exx = r.E[0], Exy = r.E[1], Exz = r.E[2], Eyy = r.E[3], Eyz = r.E[4];
+    const T Wxy = r.W[0], Wxz = r.W[1], Wyz = r.W[2];
+    const T Hxx = r.H[0], Hxy = r.H[1], Hxz = r.H[2], Hyy = r.H[3], Hyz = r.H[4];
 #pragma unroll
-    for (int c = 0; c < 5; ++c) H[c] = k.L * dq[c].lap - ld * Q[c] - k.B * Q2[c];
-    const T Hxx = H[0], Hxy = H[1], Hxz = H[2], Hyy = H[3], Hyz = H[4];
-
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-        fe[a] = T(-2.0) * (Hxx * dq[0].d[a] + Hxy * dq[1].d[a] + Hxz * dq[2].d[a] + Hyy * dq[3].d[a]
-                           + Hyz * dq[4].d[a])
-              - Hxx * dq[3].d[a] - Hyy * dq[0].d[a];
-
-    const T trQH = (T(2.0) * Hxx + Hyy) * Qxx + (T(2.0) * Hxy) * Qxy + (T(2.0) * Hxz) * Qxz
-                 + (Hxx + T(2.0) * Hyy) * Qyy + T(2.0) * Hyz * Qyz;
-    const T QH[5] = {
-        T(2.0) * (Hxx * Qxx + Hxy * Qxy + Hxz * Qxz) - two3 * trQH,
-        Hxy * Qxx + Hyy * Qxy + Hyz * Qxz + Qxy * Hxx + Qyy * Hxy + Qyz * Hxz,
-        Hxz * Qxx + Hyz * Qxy + (-Hxx - Hyy) * Qxz + Qxz * Hxx + Qyz * Hxy + (-Qxx - Qyy) * Hxz,
-        T(2.0) * (Hxy * Qxy + Hyy * Qyy + Hyz * Qyz) - two3 * trQH,
-        Hxz * Qxy + Hyz * Qyy + (-Hxx - Hyy) * Qyz + Qxz * Hxy + Qyz * Hyy + (-Qxx - Qyy) * Hyz};
+    for (int a = 0; a < 3; ++a) fe[a] = T(-2.0) * r.hd[a] - Hxx * r.d3[a] - Hyy * r.d0[a];
     ta[0] = (Hxy * Qxx + Hyy * Qxy + Hyz * Qxz) - (Qxy * Hxx + Qyy * Hxy + Qyz * Hxz);
     ta[1] = (Hxz * Qxx + Hyz * Qxy + (-Hxx - Hyy) * Qxz) - (Qxz * Hxx + Qyz * Hxy + (-Qxx - Qyy) * Hxz);
     ta[2] = (Hxz * Qxy + Hyz * Qyy + (-Hxx - Hyy) * Qyz) - (Qxz * Hxy + Qyz * Hyy + (-Qxx - Qyy) * Hyz);
-
+    const T two3 = T(2.0 / 3.0);
+    const T trQE = (T(2.0) * Exx + Eyy) * Qxx + (T(2.0) * Exy) * Qxy + (T(2.0) * Exz) * Qxz
+                 + (Exx + T(2.0) * Eyy) * Qyy + T(2.0) * Eyz * Qyz;
+    const T trQH = (T(2.0) * Hxx + Hyy) * Qxx + (T(2.0) * Hxy) * Qxy + (T(2.0) * Hxz) * Qxz
+                 + (Hxx + T(2.0) * Hyy) * Qyy + T(2.0) * Hyz * Qyz;
 #pragma unroll
     for (int c = 0; c < 5; ++c) {
+        T cor, aln2, QH;
+        switch (c) {
+            case 0:
+                cor = T(2.0) * (Qxy * Wxy + Qxz * Wxz);
+                aln2 = T(2.0) * (Exx * Qxx + Exy * Qxy + Exz * Qxz) - two3 * trQE;
+                QH = T(2.0) * (Hxx * Qxx + Hxy * Qxy + Hxz * Qxz) - two3 * trQH;
+                break;
+            case 1:
+                cor = -Qxx * Wxy + Qxz * Wyz + Qyy * Wxy + Qyz * Wxz;
+                aln2 = Exy * Qxx + Eyy * Qxy + Eyz * Qxz + Qxy * Exx + Qyy * Exy + Qyz * Exz;
+                QH = Hxy * Qxx + Hyy * Qxy + Hyz * Qxz + Qxy * Hxx + Qyy * Hxy + Qyz * Hxz;
+                break;
+            case 2:
+                cor = T(-2.0) * Qxx * Wxz - Qxy * Wyz - Qyy * Wxz + Qyz * Wxy;
+                aln2 = Exz * Qxx + Eyz * Qxy + (-Exx - Eyy) * Qxz + Qxz * Exx + Qyz * Exy + (-Qxx - Qyy) * Exz;
+                QH = Hxz * Qxx + Hyz * Qxy + (-Hxx - Hyy) * Qxz + Qxz * Hxx + Qyz * Hxy + (-Qxx - Qyy) * Hxz;
+                break;
+            case 3:
+                cor = T(2.0) * (-Qxy * Wxy + Qyz * Wyz);
+                aln2 = T(2.0) * (Exy * Qxy + Eyy * Qyy + Eyz * Qyz) - two3 * trQE;
+                QH = T(2.0) * (Hxy * Qxy + Hyy * Qyy + Hyz * Qyz) - two3 * trQH;
+                break;
+            default:
+                cor = -Qxx * Wyz - Qxy * Wxz - Qxz * Wxy - T(2.0) * Qyy * Wyz;
+                aln2 = Exz * Qxy + Eyz * Qyy + (-Exx - Eyy) * Qyz + Qxz * Exy + Qyz * Eyy + (-Qxx - Qyy) * Eyz;
+                QH = Hxz * Qxy + Hyz * Qyy + (-Hxx - Hyy) * Qyz + Qxz * Hxy + Qyz * Hyy + (-Qxx - Qyy) * Hyz;
+                break;
+        }
         const T aln3 = T(-2.0) * trQE * Q[c];
-        sg[c] = -two3 * k.lambda * H[c] - k.lambda * QH[c] + T(2.0) * k.lambda * trQH * Q[c];
-        qn[c] = Q[c] + k.dt * (advc[c] + cor[c] + k.lambda * (two3 * E[c] + aln2[c] + aln3) + k.gamma * H[c]);
+        emit(c, Q[c] + k.dt * (r.advc[c] + cor + k.lambda * (two3 * r.E[c] + aln2 + aln3) + k.gamma * r.H[c]),
+             -two3 * k.lambda * r.H[c] - k.lambda * QH + T(2.0) * k.lambda * trQH * Q[c]);
     }
+}
+template <typename T>
+__device__ __forceinline__ void q_pointwise(const Phys<T>& k, const T Q[5], const T u[3], const Deriv<T> dq[5],
+                                            const T g[3][3], T qn[5], T sg[5], T ta[3], T fe[3]) {
+    QRates<T> r;
+    q_rates(k, Q, g, r);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) q_component(k, c, Q[c], u, dq[c], r);
+    q_finish(k, Q, r, ta, fe, [&](int c, T q, T s) {
+        qn[c] = q;
+        sg[c] = s;
+    });
 }
 
 // Active force + passive stress divergence - friction, added to the Ericksen

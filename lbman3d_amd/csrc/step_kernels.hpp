@@ -40,8 +40,9 @@ __device__ __forceinline__ void sto(T* base, unsigned boff, T v) {
     *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + boff) = v;
 }
 
-// A cell by position and index. Off is 32 bits while an array stays below
-// 4 GiB (an index is then one register next to the array's scalar base).
+// A cell by position and index. Off is 32 bits while every array, the 15
+// populations together included, stays below 4 GiB: an address is then one
+// register next to a scalar base.
 template <typename Off>
 struct Node {
     int x, y, z;
@@ -130,7 +131,7 @@ __device__ __forceinline__ void gather(const Fields<T>& f, const BCDesc<T>& bc, 
         e[j] = (uint16_t)(words[j >> 1] >> (16 * (j & 1)));
         const Off nb = p.c + d[0][cx(j) + 1] + d[1][cy(j) + 1] + d[2][cz(j) + 1];
         const bool stream = slot_kind(e[j]) == SLOT_STREAM;
-        out[j] = g[(size_t)(stream ? j : slot_src(e[j])) * (size_t)vs + (stream ? nb : p.c)];
+        out[j] = ldn(g, (Off)(stream ? (Off)j * (Off)vs + nb : (Off)slot_src(e[j]) * (Off)vs + p.c));
     }
     if (f.wdot) {
         const T rho_prev = bc.rho_base + ldn(f.rho, p.c);
@@ -189,6 +190,10 @@ __device__ __forceinline__ bool on_wall(const int pos[3], const int n[3], const 
 // large ones. With force_lbm_cell, a step of the two kernels went from 23.7
 // to 14.4 us at 32^3 FP64, 48.6 to 36.4 us (FP64) and 30.7 to 19.0 us (FP32)
 // on a 20x100x100 channel, and 2.82 to 2.56 ms at 256^3 FP64.
+template <typename T>
+__device__ __forceinline__ void settle(T& x) {
+    if constexpr (sizeof(T) == 8) asm volatile("" : "+v"(x));
+}
 template <bool WALLS, typename T, typename Off>
 __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                            const Node<Off>& p, bool own) {
@@ -197,55 +202,67 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
     Off qs[7], us[7];
     stencil<WALLS>(p, bc.n, bc.qkind, qs);
     stencil<WALLS>(p, bc.n, bc.ukind, us);
-    T v[8][7];
+    T Q[5], u[3], g[3][3], w[3][7], v[5][7];
+#pragma unroll
+    for (int A = 0; A < 3; ++A)
+#pragma unroll
+        for (int i = 0; i < 7; ++i) w[A][i] = ldn(f.u[A], us[i]);
 #pragma unroll
     for (int m = 0; m < 5; ++m)
 #pragma unroll
         for (int i = 0; i < 7; ++i) v[m][i] = ldn(f.q[m], qs[i]);
 #pragma unroll
-    for (int A = 0; A < 3; ++A)
+    for (int m = 0; m < 5; ++m) Q[m] = v[m][0];
+    const bool wall_wave = WALLS && __builtin_amdgcn_ballot_w64(on_wall(pos, bc.n, bc.qkind, bc.ukind)) != 0;
+    if (wall_wave) {
 #pragma unroll
-        for (int i = 0; i < 7; ++i) v[5 + A][i] = ldn(f.u[A], us[i]);
-    if (WALLS && __builtin_amdgcn_ballot_w64(on_wall(pos, bc.n, bc.qkind, bc.ukind)) != 0) {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) q_ghosts(bc, pos, m, v[m]);
-#pragma unroll
-        for (int A = 0; A < 3; ++A) u_ghosts(bc, pos, A, v[5 + A]);
+        for (int A = 0; A < 3; ++A) u_ghosts(bc, pos, A, w[A]);
     }
-    T Q[5];
-    Deriv<T> dq[5];
-#pragma unroll
-    for (int m = 0; m < 5; ++m) {
-        Q[m] = v[m][0];
-        dq[m] = q_deriv<T, true>(bc, m, pos, Q[m], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
-    }
-    T u[3], g[3][3];
 #pragma unroll
     for (int A = 0; A < 3; ++A) {
-        u[A] = v[5 + A][0];
+        u[A] = w[A][0];
 #pragma unroll
-        for (int B = 0; B < 3; ++B)
-            g[A][B] = u_grad<T, true>(bc, B, A, pos[B], v[5 + A][1 + 2 * B], u[A], v[5 + A][2 + 2 * B]);
+        for (int B = 0; B < 3; ++B) g[A][B] = (w[A][2 + 2 * B] - w[A][1 + 2 * B]) / T(2.0);
     }
-    T qn[5], sg[5], ta[3], fe[3];
-    q_pointwise(k, Q, u, dq, g, qn, sg, ta, fe);
+    QRates<T> r;
+    q_rates(k, Q, g, r);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) settle(r.E[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) settle(r.W[i]);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+        if (wall_wave && bc.q_ghosts) q_ghosts(bc, pos, m, v[m]);   // otherwise the clamped value is the ghost
+        q_component(k, m, Q[m], u, q_deriv<T, true>(bc, m, pos, Q[m], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]), r);
+        settle(r.H[m]);
+        settle(r.advc[m]);
+    }
+    T ta[3], fe[3];
     if constexpr (sizeof(T) == 4) {
-        T pxy[6], pz[3];
+        T qn[5], sg[5], pxy[6], pz[3];
+        q_finish(k, Q, r, ta, fe, [&](int c, T qc, T sc) {
+            qn[c] = qc;
+            sg[c] = sc;
+        });
         p_sets(k.alpha, qn, sg, ta, pxy, pz);
 #pragma unroll
         for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, pxy[m]);
         stn(f.tau[0], p.c, pxy[5]);
         stn(f.tau[1], p.c, pz[0]);
         stn(f.tau[2], p.c, pz[1]);
-    } else {
+        if (own) {
 #pragma unroll
-        for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, sg[m]);
+            for (int m = 0; m < 5; ++m) stn(f.qn[m], p.c, qn[m]);
+        }
+    } else {
+        q_finish(k, Q, r, ta, fe, [&](int c, T qc, T sc) {
+            stn(f.sig[c], p.c, sc);
+            if (own) stn(f.qn[c], p.c, qc);
+        });
 #pragma unroll
         for (int m = 0; m < 3; ++m) stn(f.tau[m], p.c, ta[m]);
     }
     if (own) {
-#pragma unroll
-        for (int m = 0; m < 5; ++m) stn(f.qn[m], p.c, qn[m]);
 #pragma unroll
         for (int m = 0; m < 3; ++m) stn(f.F[m], p.c, fe[m]);
     }
@@ -298,8 +315,9 @@ __device__ __forceinline__ Node<Off> node_at(const CellGrid& g, unsigned c) {
     return {(int)(r - y * g.nx), (int)y, (int)z, (Off)c};
 }
 
-template <typename T, bool WALLS, typename Off>
+template <typename T, bool WALLS, int ADV, typename Off>
 __global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg) {
+    k.advection = ADV;
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
     qstep_cell<WALLS>(f, bc, k, node_at<Off>(cg, c), true);
@@ -307,10 +325,17 @@ __global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc
 
 // ---- body force and collide-stream ----------------------------------------
 // Both forms add the active and passive force to the Ericksen force in F.
-// FP64: differences of Q^{n+1}, Sigma and Tau in the reference's order.
-template <bool WALLS, typename T, typename Off>
+// FP64: differences of Q^{n+1}, Sigma and Tau in the reference's order. The
+// stencil's clamped value is the ghost of Q too, unless GHOSTS (see
+// BCDesc::q_ghosts). The velocity is read where friction uses it.
+template <bool WALLS, bool GHOSTS, typename T, typename Off>
 __device__ __forceinline__ void force_differences(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                                   const Node<Off>& p, T F[3]) {
+    T u[3] = {T(0), T(0), T(0)};
+    if (k.mu != T(0)) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m) u[m] = ldn(f.u[m], p.c);
+    }
     const int pos[3] = {p.x, p.y, p.z};
     Off nb[7];
     stencil<WALLS>(p, bc.n, bc.qkind, nb);
@@ -321,12 +346,11 @@ __device__ __forceinline__ void force_differences(const Fields<T>& f, const BCDe
 #pragma unroll
         for (int i = 0; i < 7; ++i) v[m][i] = ldn(a, nb[i]);
     }
-    const T u[3] = {ldn(f.u[0], p.c), ldn(f.u[1], p.c), ldn(f.u[2], p.c)};
     T dQ[5][3], dS[8][3];
 #pragma unroll
     for (int m = 0; m < 5; ++m) {
         const Deriv<T> d =
-            q_deriv<T, !WALLS>(bc, m, pos, v[m][0], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
+            q_deriv<T, !GHOSTS>(bc, m, pos, v[m][0], v[m][1], v[m][2], v[m][3], v[m][4], v[m][5], v[m][6]);
 #pragma unroll
         for (int a = 0; a < 3; ++a) dQ[m][a] = d.d[a];
     }
@@ -339,7 +363,7 @@ __device__ __forceinline__ void force_differences(const Fields<T>& f, const BCDe
 }
 
 // FP32: the divergence form, from the components qstep_cell stored.
-template <bool WALLS, typename T, typename Off>
+template <bool WALLS, bool GHOSTS, typename T, typename Off>
 __device__ __forceinline__ void force_divergence(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                                  const Node<Off>& p, T F[3]) {
     Off nb[7];
@@ -364,7 +388,7 @@ __device__ __forceinline__ void force_divergence(const Fields<T>& f, const BCDes
     d[2][0] = v[2][0][1] - v[2][0][0];
     d[2][1] = v[2][1][1] - v[2][1][0];
     d[2][2] = (v[2][2][0] - v[2][2][1]) + (v[2][3][0] - v[2][3][1]);
-    if (WALLS && bc.q_ghosts) {
+    if constexpr (GHOSTS) {
         // Where the ghost of Q is not the value beyond the face that the
         // stresses use (anchoring; a periodic high face opposite a wall), the
         // set there holds -alpha times the wrong Q. The sets' Q components:
@@ -404,7 +428,7 @@ __device__ __forceinline__ void force_divergence(const Fields<T>& f, const BCDes
 // One cell. UN: the velocity goes to un (fused-step buffers, where u still
 // holds u^{n-1} for other cells) instead of replacing u in place. Loads first,
 // as in qstep_cell.
-template <typename T, bool SHIFTED, bool UN, bool WALLS, typename Off>
+template <typename T, bool SHIFTED, bool UN, bool WALLS, bool GHOSTS, typename Off>
 __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                                const Node<Off>& p, int flags, int pull) {
     T pop[kQ], F[3];
@@ -413,8 +437,8 @@ __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<
     for (int m = 0; m < 3; ++m) F[m] = ldn(f.F[m], p.c);   // the Ericksen force, or the whole force
     if (flags & FL_FORCE) {
         if (k.force_full) {
-            if constexpr (sizeof(T) == 4) force_divergence<WALLS>(f, bc, k, p, F);
-            else force_differences<WALLS>(f, bc, k, p, F);
+            if constexpr (sizeof(T) == 4) force_divergence<WALLS, GHOSTS>(f, bc, k, p, F);
+            else force_differences<WALLS, GHOSTS>(f, bc, k, p, F);
         }
         if (flags & FL_STORE_F) {
 #pragma unroll
@@ -436,12 +460,12 @@ __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<
 
 // FLAGS is a template argument so that the step's own combination is one
 // straight run from the loads to the stores.
-template <typename T, bool SHIFTED, bool WALLS, int FLAGS, typename Off>
+template <typename T, bool SHIFTED, bool WALLS, bool GHOSTS, int FLAGS, typename Off>
 __global__ void __launch_bounds__(kBlock)
 force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg, int store, int pull) {
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
-    force_lbm_cell<T, SHIFTED, false, WALLS>(f, bc, k, node_at<Off>(cg, c),
+    force_lbm_cell<T, SHIFTED, false, WALLS, GHOSTS>(f, bc, k, node_at<Off>(cg, c),
                                                FLAGS | (store & (FL_STORE_F | FL_STORE_RHO)), pull);
 }
 
@@ -582,14 +606,15 @@ order_director_kernel(Fields<T> f, long c0, long n, double* order, double* direc
 inline unsigned grid_for(long V) { return (unsigned)((V + kBlock - 1) / kBlock); }
 
 // fn(walls, offset) with the kernels' template arguments: whether any face has
-// a wall, and 32-bit indices while an array stays below 4 GiB.
+// a wall, and the index type (Node).
 template <typename T, typename F>
-void with_step_form(const BCDesc<T>& bc, const CellGrid& cg, F&& fn) {
+void with_step_form(const BCDesc<T>& bc, long vs, F&& fn) {
+    const bool narrow = (size_t)kQ * vs * sizeof(T) < (1ull << 32);
     bool walls = false;
     for (int face = 0; face < 6; ++face)
         walls = walls || bc.qkind[face] != QB_PERIODIC || bc.ukind[face] != UB_PERIODIC;
     auto with_offset = [&](auto w) {
-        if ((size_t)cg.cells * sizeof(T) < (1ull << 32)) fn(w, 0u);
+        if (narrow) fn(w, 0u);
         else fn(w, (size_t)0);
     };
     if (walls) with_offset(std::true_type{});
@@ -599,9 +624,13 @@ void with_step_form(const BCDesc<T>& bc, const CellGrid& cg, F&& fn) {
 template <typename T>
 void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, hipStream_t s) {
     const CellGrid cg = cell_grid<T>(bc.n);
-    with_step_form(bc, cg, [&](auto w, auto off) {
-        hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, decltype(off)>), dim3(cg.blocks),
-                           dim3(cg.threads), 0, s, f, bc, k, cg);
+    with_step_form(bc, f.vs, [&](auto w, auto off) {
+        if (k.advection)
+            hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, 1, decltype(off)>), dim3(cg.blocks),
+                               dim3(cg.threads), 0, s, f, bc, k, cg);
+        else
+            hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, 0, decltype(off)>), dim3(cg.blocks),
+                               dim3(cg.threads), 0, s, f, bc, k, cg);
     });
 }
 
@@ -610,10 +639,17 @@ void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                       hipStream_t s) {
     const CellGrid cg = cell_grid<T>(bc.n);
     const int store = flags & (FL_STORE_F | FL_STORE_RHO);
-    with_step_form(bc, cg, [&](auto w, auto off) {
+    with_step_form(bc, f.vs, [&](auto w, auto off) {
+        constexpr bool walls = decltype(w)::value;
+        auto launch = [&](auto parts, auto ghosts) {
+            hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED, walls, decltype(ghosts)::value, decltype(parts)::value,
+                                                 decltype(off)>), dim3(cg.blocks), dim3(cg.threads), 0, s, f, bc, k, cg, store, pull);
+        };
         auto go = [&](auto parts) {
-            hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED, decltype(w)::value, decltype(parts)::value, decltype(off)>),
-                               dim3(cg.blocks), dim3(cg.threads), 0, s, f, bc, k, cg, store, pull);
+            if constexpr (walls && (decltype(parts)::value & FL_FORCE) != 0) {
+                if (bc.q_ghosts) return launch(parts, std::true_type{});
+            }
+            launch(parts, std::false_type{});
         };
         switch (flags & (FL_FORCE | FL_LBM)) {
             case FL_FORCE: go(std::integral_constant<int, FL_FORCE>{}); break;
@@ -626,7 +662,7 @@ void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
 template <typename T>
 void launch_stream_only(const Fields<T>& f, const BCDesc<T>& bc, int pull, T* out, hipStream_t s) {
     const CellGrid cg = cell_grid<T>(bc.n);
-    with_step_form(bc, cg, [&](auto w, auto off) {
+    with_step_form(bc, f.vs, [&](auto w, auto off) {
         hipLaunchKernelGGL((stream_only_kernel<T, decltype(w)::value, decltype(off)>), dim3(cg.blocks),
                            dim3(cg.threads), 0, s, f, bc, cg, pull, out);
     });
