@@ -164,7 +164,7 @@ batch_shell_q_kernel(const SimDesc* __restrict__ descs, int nsims, int total, in
     const SimDesc& d = descs[find_sim(nsims, w, [&](int i) { return descs[i].sq_begin; })];
     int q[3];
     region_cell(d.r3, d.bc.n, w - d.sq_begin, q);
-    qstep_cell<true>(d.f[parity], d.bc, d.k, shell_node(q, d.bc.n), !cell_mask(d.bc, 1, q[0], q[1]).writes(q[2]));
+    qstep_cell<true, false>(d.f[parity], d.bc, d.k, shell_node(q, d.bc.n), !cell_mask(d.bc, 1, q[0], q[1]).writes(q[2]));
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -177,7 +177,7 @@ batch_shell_force_kernel(const SimDesc* __restrict__ descs, int nsims, int total
     Fields<float> fq = d.f[parity];
     for (int m = 0; m < 5; ++m) fq.q[m] = fq.qn[m];   // the force reads Q^{n+1}
     const int flags = FL_FORCE | FL_LBM | ((aux | d.aux_always) ? (FL_STORE_F | FL_STORE_RHO) : 0);
-    force_lbm_cell<float, true, true, true, true>(fq, d.bc, d.k, shell_node(q, d.bc.n), flags, d.pull);
+    force_lbm_cell<float, true, true, true, true, false>(fq, d.bc, d.k, shell_node(q, d.bc.n), flags, d.pull);
 }
 
 template <int KIND, int TX, int TY, int ZC>

@@ -730,7 +730,7 @@ shell_qstep_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRegion
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    qstep_cell<true>(f, bc, k, shell_node(q, bc.n), !cell_mask(bc, 1, q[0], q[1]).writes(q[2]));
+    qstep_cell<true, false>(f, bc, k, shell_node(q, bc.n), !cell_mask(bc, 1, q[0], q[1]).writes(q[2]));
 }
 
 // Body force and collide-stream of the shell cells (w = 2); f.q points at
@@ -741,7 +741,7 @@ shell_force_lbm_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRe
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    force_lbm_cell<float, true, true, true, true>(f, bc, k, shell_node(q, bc.n), flags, pull);
+    force_lbm_cell<float, true, true, true, true, false>(f, bc, k, shell_node(q, bc.n), flags, pull);
 }
 #endif  // LBM_FUSED_BODY_ONLY
 

@@ -53,10 +53,12 @@ __device__ __forceinline__ T ldn(const T* base, Off o) {
     if constexpr (sizeof(Off) == 4) return ldo(base, o * (unsigned)sizeof(T));
     else return base[o];
 }
-template <typename Off, typename T>
+// NT: non-temporal, for outputs that leave the caches before they are read.
+template <bool NT = false, typename Off, typename T>
 __device__ __forceinline__ void stn(T* base, Off o, T v) {
-    if constexpr (sizeof(Off) == 4) sto(base, o * (unsigned)sizeof(T), v);
-    else base[o] = v;
+    T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(base) + o * (Off)sizeof(T));
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
 }
 
 // The node and its six stencil neighbours (xm, xp, ym, yp, zm, zp) under one
@@ -194,7 +196,7 @@ template <typename T>
 __device__ __forceinline__ void settle(T& x) {
     if constexpr (sizeof(T) == 8) asm volatile("" : "+v"(x));
 }
-template <bool WALLS, typename T, typename Off>
+template <bool WALLS, bool NT, typename T, typename Off>
 __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                            const Node<Off>& p, bool own) {
     const int pos[3] = {p.x, p.y, p.z};
@@ -246,25 +248,25 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
         });
         p_sets(k.alpha, qn, sg, ta, pxy, pz);
 #pragma unroll
-        for (int m = 0; m < 5; ++m) stn(f.sig[m], p.c, pxy[m]);
-        stn(f.tau[0], p.c, pxy[5]);
-        stn(f.tau[1], p.c, pz[0]);
-        stn(f.tau[2], p.c, pz[1]);
+        for (int m = 0; m < 5; ++m) stn<NT>(f.sig[m], p.c, pxy[m]);
+        stn<NT>(f.tau[0], p.c, pxy[5]);
+        stn<NT>(f.tau[1], p.c, pz[0]);
+        stn<NT>(f.tau[2], p.c, pz[1]);
         if (own) {
 #pragma unroll
-            for (int m = 0; m < 5; ++m) stn(f.qn[m], p.c, qn[m]);
+            for (int m = 0; m < 5; ++m) stn<NT>(f.qn[m], p.c, qn[m]);
         }
     } else {
         q_finish(k, Q, r, ta, fe, [&](int c, T qc, T sc) {
-            stn(f.sig[c], p.c, sc);
-            if (own) stn(f.qn[c], p.c, qc);
+            stn<NT>(f.sig[c], p.c, sc);
+            if (own) stn<NT>(f.qn[c], p.c, qc);
         });
 #pragma unroll
-        for (int m = 0; m < 3; ++m) stn(f.tau[m], p.c, ta[m]);
+        for (int m = 0; m < 3; ++m) stn<NT>(f.tau[m], p.c, ta[m]);
     }
     if (own) {
 #pragma unroll
-        for (int m = 0; m < 3; ++m) stn(f.F[m], p.c, fe[m]);
+        for (int m = 0; m < 3; ++m) stn<NT>(f.F[m], p.c, fe[m]);
     }
 }
 
@@ -315,12 +317,12 @@ __device__ __forceinline__ Node<Off> node_at(const CellGrid& g, unsigned c) {
     return {(int)(r - y * g.nx), (int)y, (int)z, (Off)c};
 }
 
-template <typename T, bool WALLS, int ADV, typename Off>
+template <typename T, bool WALLS, bool NT, int ADV, typename Off>
 __global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg) {
     k.advection = ADV;
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
-    qstep_cell<WALLS>(f, bc, k, node_at<Off>(cg, c), true);
+    qstep_cell<WALLS, NT>(f, bc, k, node_at<Off>(cg, c), true);
 }
 
 // ---- body force and collide-stream ----------------------------------------
@@ -428,7 +430,7 @@ __device__ __forceinline__ void force_divergence(const Fields<T>& f, const BCDes
 // One cell. UN: the velocity goes to un (fused-step buffers, where u still
 // holds u^{n-1} for other cells) instead of replacing u in place. Loads first,
 // as in qstep_cell.
-template <typename T, bool SHIFTED, bool UN, bool WALLS, bool GHOSTS, typename Off>
+template <typename T, bool SHIFTED, bool UN, bool WALLS, bool GHOSTS, bool NT, typename Off>
 __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                                const Node<Off>& p, int flags, int pull) {
     T pop[kQ], F[3];
@@ -453,19 +455,19 @@ __device__ __forceinline__ void force_lbm_cell(const Fields<T>& f, const BCDesc<
     if (flags & FL_STORE_RHO) stn(f.rho, p.c, rho_st);
     T* const* uo = UN ? f.un : f.u;
 #pragma unroll
-    for (int m = 0; m < 3; ++m) stn(uo[m], p.c, u[m]);
+    for (int m = 0; m < 3; ++m) stn<NT>(uo[m], p.c, u[m]);
 #pragma unroll
-    for (int j = 0; j < kQ; ++j) stn(f.gn + j * f.vs, p.c, pop[j]);
+    for (int j = 0; j < kQ; ++j) stn<NT>(f.gn + j * f.vs, p.c, pop[j]);
 }
 
 // FLAGS is a template argument so that the step's own combination is one
 // straight run from the loads to the stores.
-template <typename T, bool SHIFTED, bool WALLS, bool GHOSTS, int FLAGS, typename Off>
+template <typename T, bool SHIFTED, bool WALLS, bool GHOSTS, bool NT, int FLAGS, typename Off>
 __global__ void __launch_bounds__(kBlock)
 force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg, int store, int pull) {
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
-    force_lbm_cell<T, SHIFTED, false, WALLS, GHOSTS>(f, bc, k, node_at<Off>(cg, c),
+    force_lbm_cell<T, SHIFTED, false, WALLS, GHOSTS, NT>(f, bc, k, node_at<Off>(cg, c),
                                                FLAGS | (store & (FL_STORE_F | FL_STORE_RHO)), pull);
 }
 
@@ -625,12 +627,16 @@ template <typename T>
 void launch_qstep(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, hipStream_t s) {
     const CellGrid cg = cell_grid<T>(bc.n);
     with_step_form(bc, f.vs, [&](auto w, auto off) {
-        if (k.advection)
-            hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, 1, decltype(off)>), dim3(cg.blocks),
-                               dim3(cg.threads), 0, s, f, bc, k, cg);
-        else
-            hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, 0, decltype(off)>), dim3(cg.blocks),
-                               dim3(cg.threads), 0, s, f, bc, k, cg);
+        auto go = [&](auto nt, auto adv) {
+            hipLaunchKernelGGL((qstep_kernel<T, decltype(w)::value, decltype(nt)::value, decltype(adv)::value, decltype(off)>),
+                               dim3(cg.blocks), dim3(cg.threads), 0, s, f, bc, k, cg);
+        };
+        auto with_adv = [&](auto nt) {
+            if (k.advection) go(nt, std::integral_constant<int, 1>{});
+            else go(nt, std::integral_constant<int, 0>{});
+        };
+        if (cg.run) with_adv(std::false_type{});
+        else with_adv(std::true_type{});
     });
 }
 
@@ -641,20 +647,25 @@ void launch_force_lbm(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
     const int store = flags & (FL_STORE_F | FL_STORE_RHO);
     with_step_form(bc, f.vs, [&](auto w, auto off) {
         constexpr bool walls = decltype(w)::value;
-        auto launch = [&](auto parts, auto ghosts) {
-            hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED, walls, decltype(ghosts)::value, decltype(parts)::value,
-                                                 decltype(off)>), dim3(cg.blocks), dim3(cg.threads), 0, s, f, bc, k, cg, store, pull);
+        auto launch = [&](auto parts, auto ghosts, auto nt) {
+            hipLaunchKernelGGL((force_lbm_kernel<T, SHIFTED, walls, decltype(ghosts)::value, decltype(nt)::value,
+                                                 decltype(parts)::value, decltype(off)>),
+                               dim3(cg.blocks), dim3(cg.threads), 0, s, f, bc, k, cg, store, pull);
         };
-        auto go = [&](auto parts) {
+        auto go = [&](auto parts, auto nt) {
             if constexpr (walls && (decltype(parts)::value & FL_FORCE) != 0) {
-                if (bc.q_ghosts) return launch(parts, std::true_type{});
+                if (bc.q_ghosts) return launch(parts, std::true_type{}, nt);
             }
-            launch(parts, std::false_type{});
+            launch(parts, std::false_type{}, nt);
         };
+        constexpr std::integral_constant<int, FL_FORCE | FL_LBM> both{};
         switch (flags & (FL_FORCE | FL_LBM)) {
-            case FL_FORCE: go(std::integral_constant<int, FL_FORCE>{}); break;
-            case FL_LBM: go(std::integral_constant<int, FL_LBM>{}); break;
-            default: go(std::integral_constant<int, FL_FORCE | FL_LBM>{}); break;
+            case FL_FORCE: go(std::integral_constant<int, FL_FORCE>{}, std::false_type{}); break;
+            case FL_LBM: go(std::integral_constant<int, FL_LBM>{}, std::false_type{}); break;
+            default:
+                if (cg.run) go(both, std::false_type{});
+                else go(both, std::true_type{});
+                break;
         }
     });
 }
