@@ -203,9 +203,9 @@ int lbm_profile_kernels(lbm_handle h, int32_t n, double* ms_out, int32_t max,
                         char* names, size_t names_len, int32_t* count);
 /* Kernel schedule. 0 = automatic (autotuned on first use), 1 = two-kernel
  * split, 2.. = a fixed fused tile shape. FP32 tiles: lbm_tile_count /
- * lbm_tile_name. FP64: fully periodic domains also have fused single-kernel
- * tiles, whose results equal the two-kernel split bit for bit; other domains
- * run the two-kernel split. */
+ * lbm_tile_name. FP64: fully periodic domains, and domains with walls from 2^20
+ * cells on, also have fused tiles, whose results equal the two-kernel split bit
+ * for bit; other domains run the two-kernel split. */
 int lbm_set_schedule(lbm_handle h, int32_t schedule);
 int lbm_get_schedule(lbm_handle h, int32_t* schedule);
 int lbm_tile_count(void);

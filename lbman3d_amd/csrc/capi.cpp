@@ -258,6 +258,9 @@ namespace {
 // 64 MiB apart and the 46 streams of the fused step ran 4-5% slower.)
 constexpr long kStagger = 64;
 
+// Cells from which a walled FP64 grid has the fused schedules.
+constexpr long kFused64Walls = 1L << 20;
+
 template <typename T>
 int alloc_fields(lbm_solver* s, Fields<T>& f) {
     const long V = s->V, vs = s->vs;
@@ -540,7 +543,9 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
         bool periodic = true;
         for (int face = 0; face < 6; ++face)
             periodic = periodic && cfg->walls[face].qbc == LBM_Q_PERIODIC && cfg->walls[face].ubc == LBM_U_PERIODIC;
-        s->fused64_ok = s->fp64 && periodic && fused64_tile_count() > 0 &&
+        // With walls the fused FP64 step is an interior launch and two shell
+        // passes, which pays from about a million cells on.
+        s->fused64_ok = s->fp64 && (periodic || s->V >= kFused64Walls) && fused64_tile_count() > 0 &&
                         (double)kQ * s->vs * sizeof(double) < 4294967296.0;
     }
     auto cleanup = [&](int r) {

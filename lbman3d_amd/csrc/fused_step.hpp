@@ -32,6 +32,9 @@
 
 namespace lbm {
 
+__device__ __forceinline__ void sto_nt(double* base, unsigned boff, double v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<double*>(reinterpret_cast<char*>(base) + boff));
+}
 // Store with an optional non-temporal hint (streaming output read back only
 // next step, so it need not displace the halo rows held in L2).
 template <bool NT>
@@ -169,20 +172,12 @@ __device__ __forceinline__ void load_column(const Fields<T>& f, int qcol, int uc
 // (xy neighbours) and the column's own z neighbours.
 template <int TX, int TY, bool NOGHOST, typename T>
 __device__ __forceinline__ void stage_a(const BCDesc<T>& bc, const Phys<T>& k,
-                                        const T (*sIn)[TileGeom<TX, TY>::NI], int ii, int jj,
+                                        const T (*sIn)[TileGeom<TX, TY>::NI], int cc,
                                         const T zm[kNumIn], const T c[kNumIn], const T zp[kNumIn],
                                         const int qpos[3], const int upos[3], StageAT<T>& out, T fe[3]) {
     using G = TileGeom<TX, TY>;
-    const int cc = jj * G::IX + ii;
     const int xm = cc - 1, xp = cc + 1, ym = cc - G::IX, yp = cc + G::IX;
-    T Q[5];
-    Deriv<T> dq[5];
-#pragma unroll
-    for (int m = 0; m < 5; ++m) {
-        Q[m] = c[m];
-        dq[m] = q_deriv<T, NOGHOST>(bc, m, qpos, c[m], sIn[m][xm], sIn[m][xp], sIn[m][ym], sIn[m][yp], zm[m], zp[m]);
-    }
-    T u[3], g[3][3];
+    T Q[5], u[3], g[3][3];
 #pragma unroll
     for (int A = 0; A < 3; ++A) {
         const T v0 = c[5 + A];
@@ -191,7 +186,26 @@ __device__ __forceinline__ void stage_a(const BCDesc<T>& bc, const Phys<T>& k,
         g[A][1] = u_grad<T, NOGHOST>(bc, 1, A, upos[1], sIn[5 + A][ym], v0, sIn[5 + A][yp]);
         g[A][2] = u_grad<T, NOGHOST>(bc, 2, A, upos[2], zm[5 + A], v0, zp[5 + A]);
     }
-    q_pointwise(k, Q, u, dq, g, out.qn, out.sg, out.ta, fe);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) Q[m] = c[m];
+    QRates<T> r;
+    q_rates(k, Q, g, r);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) settle(r.E[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) settle(r.W[i]);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+        q_component(k, m, Q[m], u, q_deriv<T, NOGHOST>(bc, m, qpos, c[m], sIn[m][xm], sIn[m][xp], sIn[m][ym],
+                                                       sIn[m][yp], zm[m], zp[m]), r);
+        settle(r.H[m]);
+        settle(r.advc[m]);
+        if constexpr (sizeof(T) == 8) asm volatile("" ::: "memory");   // the next component's LDS reads stay below
+    }
+    q_finish(k, Q, r, out.ta, fe, [&](int m, T qn, T sg) {
+        out.qn[m] = qn;
+        out.sg[m] = sg;
+    });
 }
 
 // Register-lean form of the Q update for the FP32 fused kernels: the same
@@ -394,16 +408,7 @@ __device__ __forceinline__ CellMask cell_mask(const BCDesc<T>& bc, int mode, int
 // column tile (tx, ty), writing the cells that `mode` selects. LDS buffers
 // come from the calling kernel so that a kernel instantiating several
 // variants does not allocate LDS per variant.
-//
-// UNCOND (fully periodic grids whose x and y sides are whole tiles, every
-// cell written): the ring and outer-ring loads, the pull gather and the
-// stores are issued by every thread and the first two planes of the chunk
-// are peeled, so that no memory instruction sits under a branch. The memory
-// counter waits the compiler places after such a branch assume its loads or
-// stores were skipped and then wait for everything issued before, the
-// previous plane's stores included, and at one wave per SIMD (FP64) nothing
-// covers that wait.
-template <int TX, int TY, int ZC, bool PERIODIC, typename T, bool UNCOND = false>
+template <int TX, int TY, int ZC, bool PERIODIC, typename T>
 __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
                                            int pull, int aux, int tx, int ty, int tz,
                                            T (*sIn)[TileGeom<TX, TY>::NI],
@@ -463,14 +468,11 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
 
     // Input history of the interior column in iteration pa: planes pa-1, pa,
     // pa+1 (registers); the next plane, pa + 2, is loaded one iteration ahead
-    // of its use. It joins the history at the end of the iteration in the
-    // unconditional form (the wait for it then falls after the stores are
-    // issued) and at the start of the next iteration otherwise.
-    static_assert(!UNCOND || PERIODIC, "unconditional form: fully periodic grids");
+    // of its use and joins the history at the start of the next iteration.
     T hin[3][kNumIn], hnext[kNumIn];
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[UNCOND ? 0 : 1]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[UNCOND ? 1 : 2]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0), uplane(z0), UNCOND ? hin[2] : hnext);
+    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[1]);
+    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[2]);
+    load_column<TX, TY>(f, qc0, uc0, qplane(z0), uplane(z0), hnext);
     if (has_ring) {
         T v[kNumIn];
         load_column<TX, TY>(f, qcr, ucr, qplane(z0 - 2), uplane(z0 - 2), v);
@@ -483,19 +485,15 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     // Ring and outer-ring inputs are loaded one plane ahead of their LDS
     // store: ring plane pa + 1 and outer plane pa arrive in iteration pa.
     T rnext[kNumIn], onext[kNumIn];
-    // Columns of the ring and outer-ring loads; in the unconditional form a
-    // thread without such a column loads its own (the values go unused).
-    const int rq = (UNCOND && !has_ring) ? qc0 : qcr, ru = (UNCOND && !has_ring) ? uc0 : ucr;
-    const int oq = (UNCOND && !has_outer) ? qc0 : oqc, ou = (UNCOND && !has_outer) ? uc0 : ouc;
-    if (UNCOND || has_ring) load_column<TX, TY>(f, rq, ru, qplane(z0), uplane(z0), rnext);
+    if (has_ring) load_column<TX, TY>(f, qcr, ucr, qplane(z0), uplane(z0), rnext);
     auto load_outer = [&](int z, T* v) {
-        const unsigned qo = (qplane(z) + (unsigned)oq) * E, uo = (uplane(z) + (unsigned)ou) * E;
+        const unsigned qo = (qplane(z) + (unsigned)oqc) * E, uo = (uplane(z) + (unsigned)ouc) * E;
 #pragma unroll
         for (int m = 0; m < 5; ++m) v[m] = ldo(f.q[m], qo);
 #pragma unroll
         for (int m = 0; m < 3; ++m) v[5 + m] = ldo(f.u[m], uo);
     };
-    if (UNCOND || has_outer) load_outer(z0 - 1, onext);
+    if (has_outer) load_outer(z0 - 1, onext);
 
     // z-difference values of the interior column's stage A at plane pa - 2
     // (the lower z neighbour of the plane finished in step 3), and the
@@ -505,18 +503,14 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     for (int m = 0; m < kNumDZ; ++m) dz_back[m] = T(0);
     T fe_prev[3] = {0, 0, 0}, fe_cur[3] = {0, 0, 0};
 
-    // One iteration: WB (compile time) false skips the gather and the force
-    // stage, for the two peeled planes of the unconditional form.
-    auto iteration = [&](const int pa, auto WB) {
+    for (int pa = z0 - 1; pa <= z1; ++pa) {
         const int pb = pa - 1;
-        const bool do_b = decltype(WB)::value && (UNCOND || (pb >= z0 && active));
-        if constexpr (!UNCOND) {
+        const bool do_b = pb >= z0 && active;
 #pragma unroll
-            for (int m = 0; m < kNumIn; ++m) {
-                hin[0][m] = hin[1][m];
-                hin[1][m] = hin[2][m];
-                hin[2][m] = hnext[m];
-            }
+        for (int m = 0; m < kNumIn; ++m) {
+            hin[0][m] = hin[1][m];
+            hin[1][m] = hin[2][m];
+            hin[2][m] = hnext[m];
         }
         // ---- step 1: input plane pa into LDS; next-plane loads ----
         // At pa == z1 the loaded plane is never used; clamping it to z1 + 1
@@ -543,16 +537,14 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
                 sRing[r_p][m][t] = rnext[m];
                 sIn[m][cc] = sRing[r_c][m][t];
             }
-            if (!UNCOND && pa < z1) load_column<TX, TY>(f, rq, ru, qplane(pa + 2), uplane(pa + 2), rnext);
+            if (pa < z1) load_column<TX, TY>(f, qcr, ucr, qplane(pa + 2), uplane(pa + 2), rnext);
         }
-        if (UNCOND) load_column<TX, TY>(f, rq, ru, qplane(pn), uplane(pn), rnext);
         if (has_outer) {
             const int cc = oj * G::IX + oi;
 #pragma unroll
             for (int m = 0; m < kNumIn; ++m) sIn[m][cc] = onext[m];
-            if (!UNCOND && pa < z1) load_outer(pa + 1, onext);
+            if (pa < z1) load_outer(pa + 1, onext);
         }
-        if (UNCOND) load_outer(min(pa + 1, z1), onext);
         __syncthreads();
 
         // ---- step 2: Q update (stage A) at plane pa ----
@@ -592,7 +584,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
             upos[2] = zu;
             StageAT<T> a;
             T fe[3];
-            stage_a<TX, TY, PERIODIC>(bc, k, sIn, ci + 1, cj + 1, zm, c, zp, qpos, upos, a, fe);
+            stage_a<TX, TY, PERIODIC>(bc, k, sIn, (cj + 1) * G::IX + ci + 1, zm, c, zp, qpos, upos, a, fe);
 #pragma unroll
             for (int m = 0; m < kNumA; ++m) sA[par][m][acol] = stage_value(a, m);
             if (slot == 0) {
@@ -659,7 +651,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
             if constexpr (sizeof(T) == 4) collide_shifted(k, pop, F, drho, u);
             else collide_plain(k, pop, F, drho, u);
             const unsigned vs4 = (unsigned)f.vs * E, c4 = cpb * E;
-            if (UNCOND || wmask.writes(pb)) {
+            if (wmask.writes(pb)) {
 #pragma unroll
                 for (int j = 0; j < kQ; ++j) sto(f.gn, j * vs4 + c4, pop[j]);
 #pragma unroll
@@ -678,26 +670,10 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
 #pragma unroll
         for (int m = 0; m < kNumA; ++m)
             if (dz_slot(m) >= 0) dz_back[dz_slot(m)] = A(m, acell);
-        if constexpr (UNCOND) {
-            // History advance: planes pa, pa + 1, pa + 2 for the next iteration.
-#pragma unroll
-            for (int m = 0; m < kNumIn; ++m) {
-                hin[0][m] = hin[1][m];
-                hin[1][m] = hin[2][m];
-                hin[2][m] = hnext[m];
-            }
-        }
-    };
-    if constexpr (UNCOND) {
-        iteration(z0 - 1, std::false_type{});
-        iteration(z0, std::false_type{});
-        for (int pa = z0 + 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
-    } else {
-        for (int pa = z0 - 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
     }
 }
 
-template <int TX, int TY, int ZC, bool PERIODIC, typename T = float, bool UNCOND = false>
+template <int TX, int TY, int ZC, bool PERIODIC, typename T = float>
 __global__ void __launch_bounds__(TX * TY)
 fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int ntx, int nty,
                   int nzc, int mode) {
@@ -713,19 +689,246 @@ fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int n
     const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (L >= nblk) return;
     const int tx = L % ntx, ty = (L / ntx) % nty, tz = L / (ntx * nty);
-    fused_body<TX, TY, ZC, PERIODIC, T, UNCOND>(f, bc, k, pull, aux, tx, ty, tz, sIn, sA, sRing, mode);
+    fused_body<TX, TY, ZC, PERIODIC, T>(f, bc, k, pull, aux, tx, ty, tz, sIn, sA, sRing, mode);
+}
+
+// The FP64 step. The arithmetic is the unfused kernels' (stage_a, body_force,
+// collide_plain, no contraction), so the results are theirs bit for bit; the
+// data flow is the first pipeline's with half its LDS and registers, so that
+// two wavefronts share a SIMD: FP64 arithmetic is four cycles an instruction
+// and a wavefront alone leaves the SIMD idle two thirds of the time, in LDS
+// and memory waits and at barriers.
+//   * one plane of Q-update results in LDS: the force of plane pa - 1 reads it
+//     while the own column's results of plane pa wait in registers; after a
+//     barrier they take its place, and the ring columns are updated then;
+//   * a thread prefetches one more column: its ring or its outer-ring column
+//     (NR + NO <= threads), the ring's a plane further ahead;
+//   * the pull gather is issued after the Q update, under the force.
+// Per plane: stage inputs | Q update, force and collide-stream of the plane
+// below | publish, ring update |, a barrier at each bar.
+//
+// MASKED: a domain with walls. The periodic form is exact for class-0 cells
+// (CellMask); the shell passes that follow overwrite the others, and rho and F
+// are stored for class-0 cells alone.
+//
+// 256^3 on 32x8 tiles: 2.14 ms for the first pipeline's best tile, 1.56 ms
+// here; 128^3 0.244 -> 0.213 ms. What it must not do is spill: with every halo
+// load issued unconditionally (14 registers more) the prefetched values went
+// to scratch as they arrived and the step took 2.05 ms. Non-temporal stores
+// (the outputs leave the L2 before they are read): 2.12 -> 2.05 ms then.
+template <int TX, int TY, bool MASKED, int ADV>
+__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(2, 2)))
+fused64_kernel(Fields<double> f, BCDesc<double> bc, Phys<double> k, int pull, int aux, int ntx, int nty, int nzc,
+               int zc) {
+    using G = TileGeom<TX, TY>;
+    using T = double;
+    constexpr unsigned E = sizeof(T);
+    static_assert(G::NR + G::NO <= G::NT, "a thread owns one halo column");
+    __shared__ T sIn[kNumIn][G::NI];        // input plane pa, extended region
+    // Q-update results, one plane, at the input region's row length: a column
+    // has one index in both arrays, less the offset of their corners.
+    constexpr int kCorner = G::IX + 1;
+    __shared__ T sA[kNumA][G::IX * G::AY];
+    __shared__ T sRing[3][kNumIn][G::NR];   // inputs of the ring columns, planes mod 3
+    k.advection = ADV;
+    const int nblk = ntx * nty * nzc;
+    const int per_xcd = (nblk + 7) / 8;
+    const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (L >= nblk) return;
+    const int tx = L % ntx, ty = (L / ntx) % nty, tz = L / (ntx * nty);
+    const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
+    const int x0 = tx * TX, y0 = ty * TY;
+    const int z0 = tz * zc, z1 = min(z0 + zc, nz);
+    const unsigned plane = (unsigned)nx * ny;
+
+    const int t = threadIdx.x;
+    const int ia = t % TX + 1, ib = t / TX + 1;
+    const int gx = x0 + ia - 1, gy = y0 + ib - 1;
+    const bool active = gx < nx && gy < ny;
+    const bool has_ring = t < G::NR, has_outer = t >= G::NT - G::NO;
+    int ra = 0, rb = 0, oi = 0, oj = 0;
+    if (has_ring) ring_col(t, G::AX, G::AY, ra, rb);
+    if (has_outer) ring_col(t - (G::NT - G::NO), G::IX, G::IY, oi, oj);
+    const int qx = map_col(gx, nx, true, true), qy = map_col(gy, ny, true, true);
+    const unsigned c0 = (unsigned)qy * nx + qx;
+    unsigned cx_halo = c0;   // the halo column of this thread (its own without one)
+    if (has_ring) cx_halo = (unsigned)map_col(y0 - 1 + rb, ny, true, true) * nx + map_col(x0 - 1 + ra, nx, true, true);
+    if (has_outer) cx_halo = (unsigned)map_col(y0 - 2 + oj, ny, true, true) * nx + map_col(x0 - 2 + oi, nx, true, true);
+    const bool has_halo = has_ring || has_outer;
+    const int cc_int = (ib + 1) * G::IX + ia + 1, acell = cc_int - kCorner;
+    const int cc_halo = has_ring ? (rb + 1) * G::IX + ra + 1 : oj * G::IX + oi;
+    auto zplane = [&](int z) { return (unsigned)map_coord(z, nz, true, true) * plane; };
+    auto load = [&](unsigned col, int z, T v[kNumIn]) {
+        const unsigned o = (zplane(z) + col) * E;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) v[m] = ldo(f.q[m], o);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) v[5 + m] = ldo(f.u[m], o);
+    };
+    // In-plane steps to the wrapped pull sources, index c + 1: the one at -c.
+    const unsigned dx[3] = {qx == nx - 1 ? 1u - nx : 1u, 0u, qx == 0 ? nx - 1u : ~0u};
+    const unsigned dy[3] = {qy == ny - 1 ? nx - plane : (unsigned)nx, 0u, qy == 0 ? plane - nx : 0u - nx};
+
+    // Own column: planes pa - 1 and pa + 1 (plane pa is in sIn). Halo column: the ring's plane pa + 1
+    // or the outer ring's plane pa, loaded one iteration ahead.
+    T below[kNumIn], above[kNumIn], halo[kNumIn];
+    load(c0, z0 - 2, below);
+    load(c0, z0 - 1, above);
+#pragma unroll
+    for (int m = 0; m < kNumIn; ++m) sIn[m][cc_int] = above[m];
+    load(c0, z0, above);
+    if (has_ring) {
+        T v[kNumIn];
+#pragma unroll 1
+        for (int z = z0 - 2; z < z0; ++z) {
+            load(cx_halo, z, v);
+#pragma unroll
+            for (int m = 0; m < kNumIn; ++m) sRing[(z + 6) % 3][m][t] = v[m];
+        }
+    }
+    if (has_halo) load(cx_halo, has_ring ? z0 : z0 - 1, halo);
+    // z-difference values of the own column two planes below the Q update, and
+    // its Ericksen force one plane below.
+    T dz_back[kNumDZ], fe_prev[3] = {0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < kNumDZ; ++m) dz_back[m] = T(0);
+    const int none[3] = {0, 0, 0};
+
+    // WB false: the first two iterations, whose planes pb lie below the chunk.
+    auto iteration = [&](const int pa, auto WB) {
+        const int pb = pa - 1;
+        const bool do_b = decltype(WB)::value && active;
+        const int r_m = (pa + 5) % 3, r_c = (pa + 6) % 3, r_p = (pa + 7) % 3;
+        // ---- input plane pa into LDS (the own column is there); next-plane loads ----
+        if (has_halo) {
+#pragma unroll
+            for (int m = 0; m < kNumIn; ++m) {
+                T v = halo[m];
+                if (has_ring) {
+                    sRing[r_p][m][t] = v;
+                    v = sRing[r_c][m][t];
+                }
+                sIn[m][cc_halo] = v;
+            }
+        }
+        // Past the chunk's end the loaded planes are not used; the clamp keeps
+        // every request within one plane of it.
+        T hnext[kNumIn];
+        load(c0, min(pa + 2, z1 + 1), hnext);
+        if (has_halo) load(cx_halo, has_ring ? min(pa + 2, z1 + 1) : min(pa + 1, z1), halo);
+        __syncthreads();
+
+        // ---- Q update of the own column at plane pa ----
+        StageAT<T> a;
+        T fe_new[3];
+        {
+            T c[kNumIn];
+#pragma unroll
+            for (int m = 0; m < kNumIn; ++m) c[m] = sIn[m][cc_int];
+            stage_a<TX, TY, true>(bc, k, sIn, cc_int, below, c, above, none, none, a, fe_new);
+        }
+
+        // ---- force + collide-stream at plane pb (sA holds plane pb) ----
+        if (do_b) {
+            T pop[kQ];
+            const unsigned vsb = (unsigned)f.vs * E, cb = (zplane(pb) + c0) * E;
+            if (pull) {
+                const unsigned zo[3] = {zplane(pb + 1) + c0, zplane(pb) + c0, zplane(pb - 1) + c0};
+#pragma unroll
+                for (int j = 0; j < kQ; ++j)
+                    pop[j] = ldo(f.g, j * vsb + (zo[cz(j) + 1] + dx[cx(j) + 1] + dy[cy(j) + 1]) * E);
+            } else {
+#pragma unroll
+                for (int j = 0; j < kQ; ++j) pop[j] = ldo(f.g, j * vsb + cb);
+            }
+            auto zmv = [&](int m) -> T { return dz_slot(m) < 0 ? sA[m][acell] : dz_back[dz_slot(m)]; };
+            auto zpv = [&](int m) -> T { return dz_slot(m) < 0 ? sA[m][acell] : stage_value(a, m); };
+            // body_force with each difference taken where its sum needs it;
+            // rows of sA: Q 0-4, Sigma 5-9, Tau 10-12.
+            auto ddx = [&](int m) { return (sA[m][acell + 1] - sA[m][acell - 1]) / T(2.0); };
+            auto ddy = [&](int m) { return (sA[m][acell + G::IX] - sA[m][acell - G::IX]) / T(2.0); };
+            auto ddz = [&](int m) { return (zpv(m) - zmv(m)) / T(2.0); };
+            auto done = [](T& x) { asm volatile("" : "+v"(x)::"memory"); };
+            T F[3] = {fe_prev[0], fe_prev[1], fe_prev[2]};
+            if (k.force_full) {
+                T aq = ddx(0) + ddy(1) + ddz(2);
+                done(aq);
+                T pd = ddx(5) + (ddy(6) + ddy(10)) + (ddz(7) + ddz(11));
+                done(pd);
+                F[0] = F[0] + (-k.alpha * aq + pd - k.mu * below[5]);   // below: u^{n-1} at (gx, gy, pb)
+                aq = ddx(1) + ddy(3) + ddz(4);
+                done(aq);
+                pd = (ddx(6) - ddx(10)) + ddy(8) + (ddz(9) + ddz(12));
+                done(pd);
+                F[1] = F[1] + (-k.alpha * aq + pd - k.mu * below[6]);
+                aq = ddx(2) + ddy(4) - ddz(0) - ddz(3);
+                done(aq);
+                pd = (ddx(7) - ddx(11)) + (ddy(9) - ddy(12)) + -(ddz(5) + ddz(8));
+                done(pd);
+                F[2] = F[2] + (-k.alpha * aq + pd - k.mu * below[7]);
+            }
+            T rho, u[3];
+            collide_plain(k, pop, F, rho, u);
+#pragma unroll
+            for (int j = 0; j < kQ; ++j) sto_nt(f.gn, j * vsb + cb, pop[j]);
+#pragma unroll
+            for (int m = 0; m < 3; ++m) sto_nt(f.un[m], cb, u[m]);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) sto_nt(f.qn[m], cb, sA[m][acell]);
+            if (aux && (!MASKED || cell_mask(bc, 1, gx, gy).writes(pb))) {
+                sto(f.rho, cb, rho);
+#pragma unroll
+                for (int m = 0; m < 3; ++m) sto(f.F[m], cb, F[m]);
+            }
+        }
+        // Plane pb becomes the lower z neighbour of the next plane.
+#pragma unroll
+        for (int m = 0; m < kNumA; ++m)
+            if (dz_slot(m) >= 0) dz_back[dz_slot(m)] = sA[m][acell];
+        __syncthreads();
+
+        // ---- publish plane pa: the own column, then the ring columns ----
+#pragma unroll
+        for (int m = 0; m < kNumA; ++m) sA[m][acell] = stage_value(a, m);
+        if (has_ring) {
+            T zm[kNumIn], c[kNumIn], zp[kNumIn], fer[3];
+#pragma unroll
+            for (int m = 0; m < kNumIn; ++m) {
+                zm[m] = sRing[r_m][m][t];
+                c[m] = sRing[r_c][m][t];
+                zp[m] = sRing[r_p][m][t];
+            }
+            StageAT<T> ar;
+            stage_a<TX, TY, true>(bc, k, sIn, cc_halo, zm, c, zp, none, none, ar, fer);
+#pragma unroll
+            for (int m = 0; m < kNumA; ++m) sA[m][cc_halo - kCorner] = stage_value(ar, m);
+        }
+#pragma unroll
+        for (int m = 0; m < 3; ++m) fe_prev[m] = fe_new[m];
+#pragma unroll
+        for (int m = 0; m < kNumIn; ++m) below[m] = sIn[m][cc_int];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < kNumIn; ++m) {
+            sIn[m][cc_int] = above[m];
+            above[m] = hnext[m];
+        }
+    };
+    iteration(z0 - 1, std::false_type{});
+    iteration(z0, std::false_type{});
+    for (int pa = z0 + 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
 }
 
 // ---- wall shells of a single simulation, one thread per cell ------------------
 __device__ __forceinline__ Node<unsigned> shell_node(const int q[3], const int n[3]) {
     return {q[0], q[1], q[2], ((unsigned)q[2] * n[1] + q[1]) * n[0] + q[0]};
 }
-#ifndef LBM_FUSED_BODY_ONLY
 // Q update over the shell and its one-cell halo (w = 3). Every cell stores
-// Sigma and Tau for the force pass; only shell cells store Q^{n+1} and the
+// the stresses for the force pass; only shell cells store Q^{n+1} and the
 // Ericksen force (the interior launch owns the rest).
-static __global__ void __launch_bounds__(kBlock)
-shell_qstep_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRegion r) {
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+shell_qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, ShellRegion r) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= region_cells(r)) return;
     int q[3];
@@ -735,15 +938,34 @@ shell_qstep_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRegion
 
 // Body force and collide-stream of the shell cells (w = 2); f.q points at
 // Q^{n+1}, and the velocity goes to un.
-static __global__ void __launch_bounds__(kBlock)
-shell_force_lbm_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, ShellRegion r, int flags, int pull) {
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+shell_force_lbm_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, ShellRegion r, int flags, int pull) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= region_cells(r)) return;
     int q[3];
     region_cell(r, bc.n, i, q);
-    force_lbm_cell<float, true, true, true, true, false>(f, bc, k, shell_node(q, bc.n), flags, pull);
+    force_lbm_cell<T, sizeof(T) == 4, true, true, true, false>(f, bc, k, shell_node(q, bc.n), flags, pull);
 }
-#endif  // LBM_FUSED_BODY_ONLY
+
+// Shell launches of a domain with walls: after the interior launch, the
+// unfused step kernels' per-cell code recomputes the cells within two cells
+// of an open face, with full wall handling, in two passes over the shell
+// (one thread per cell, so the few shell cells of a large or small grid are
+// spread over the whole GPU). Both passes read the previous state, the new
+// Q^{n+1} of the interior launch next to the shell, and the stresses that the
+// first pass writes.
+template <typename T>
+void launch_shells(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k, int pull, int aux, hipStream_t s) {
+    const ShellRegion r3 = make_shell_region(bc, 3), r2 = make_shell_region(bc, 2);
+    if (region_cells(r2) == 0) return;
+    hipLaunchKernelGGL(shell_qstep_kernel<T>, dim3(grid_for(region_cells(r3))), dim3(kBlock), 0, s, f, bc, k, r3);
+    Fields<T> fq = f;
+    for (int m = 0; m < 5; ++m) fq.q[m] = f.qn[m];
+    const int flags = FL_FORCE | FL_LBM | (aux ? (FL_STORE_F | FL_STORE_RHO) : 0);
+    hipLaunchKernelGGL(shell_force_lbm_kernel<T>, dim3(grid_for(region_cells(r2))), dim3(kBlock), 0, s, fq, bc, k, r2,
+                       flags, pull);
+}
 
 // Second pipeline: the same computation with one stage-A plane in LDS (the
 // force stage reads plane pb while the fresh plane pa waits in registers and
@@ -1389,25 +1611,6 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 int fused_tile_count() { return kNumTiles; }
 const char* fused_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles) ? kTiles[tile].name : "?"; }
-
-// Shell launches of a domain with walls: after the interior launch, the
-// unfused step kernels' per-cell code recomputes the cells within two cells
-// of an open face, with full wall handling, in two passes over the shell
-// (one thread per cell, so the few shell cells of a large or small grid are
-// spread over the whole GPU). Both passes read the previous state, the new
-// Q^{n+1} of the interior launch next to the shell, and Sigma/Tau that the
-// first pass writes.
-static void launch_shells(const Fields<float>& f, const BCDesc<float>& bc, const Phys<float>& k, int pull, int aux,
-                          hipStream_t s) {
-    const ShellRegion r3 = make_shell_region(bc, 3), r2 = make_shell_region(bc, 2);
-    if (region_cells(r2) == 0) return;
-    hipLaunchKernelGGL(shell_qstep_kernel, dim3(grid_for(region_cells(r3))), dim3(kBlock), 0, s, f, bc, k, r3);
-    Fields<float> fq = f;
-    for (int m = 0; m < 5; ++m) fq.q[m] = f.qn[m];
-    const int flags = FL_FORCE | FL_LBM | (aux ? (FL_STORE_F | FL_STORE_RHO) : 0);
-    hipLaunchKernelGGL(shell_force_lbm_kernel, dim3(grid_for(region_cells(r2))), dim3(kBlock), 0, s, fq, bc, k, r2,
-                       flags, pull);
-}
 
 template <int KIND, int TX, int TY, int ZC>
 static void launch_tile(const Fields<float>& f, const BCDesc<float>& bc, const Phys<float>& k, int pull, int aux,

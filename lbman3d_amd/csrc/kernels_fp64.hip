@@ -13,47 +13,67 @@ template void launch_diagnostics<double>(const Fields<double>&, const BCDesc<dou
                                          double*, double*, int, double*, hipStream_t);
 template void launch_order_director<double>(const Fields<double>&, long, long, double*, double*, hipStream_t);
 
-// FP64 tile catalogue of the fused step (first pipeline, periodic
-// specialisation). Rows of 16 doubles are one 128-byte line.
-struct Tile64 {
-    int tx, ty, zc;
-    const char* name;
-};
-constexpr Tile64 kTiles64[] = {
-    {32, 4, 64, "fp64:32x4x64"}, {32, 4, 128, "fp64:32x4x128"}, {16, 8, 64, "fp64:16x8x64"},
-    {16, 8, 32, "fp64:16x8x32"}, {32, 8, 64, "fp64:32x8x64"},   {64, 4, 64, "fp64:64x4x64"},
-    {32, 4, 32, "fp64:32x4x32"},
-};
+// FP64 tile catalogue of the fused step (fused64_kernel).
+constexpr const char* kTiles64[] = {"fp64:32x8", "fp64:16x16"};
 constexpr int kNumTiles64 = sizeof(kTiles64) / sizeof(kTiles64[0]);
 
 int fused64_tile_count() { return kNumTiles64; }
-const char* fused64_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles64) ? kTiles64[tile].name : "?"; }
+const char* fused64_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles64) ? kTiles64[tile] : "?"; }
 
-template <int TX, int TY, int ZC>
+// Length of the z chunks of a grid of `columns` column tiles: a chunk costs its
+// planes and two more, and the chunks run in rounds of two blocks per CU, so
+// that one block too many costs a whole round (150x130x100 on 32x8 tiles: 595
+// chunks of 16 planes in two rounds, 329 us; 510 of 17 in one, 270 us). Chunks
+// longer than 64 planes drift apart and share less in the L2 (256^3: 1.56 ms
+// with 64 planes, 1.64 ms with 128).
+static int chunk_planes(int columns, int nz) {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    const long slots = 2L * std::max(1, cus);
+    long best = 1L << 62;
+    int planes = std::min(nz, 64);
+    for (int n = (nz + 63) / 64; n <= nz; ++n) {
+        const int zc = (nz + n - 1) / n;
+        const long chunks = (long)columns * ((nz + zc - 1) / zc);
+        const long cost = (chunks + slots - 1) / slots * (zc + 2);
+        if (cost < best) {
+            best = cost;
+            planes = zc;
+        }
+        if (chunks > 8 * slots) break;
+    }
+    return planes;
+}
+
+template <int TX, int TY>
 static void launch_tile64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int pull,
                           int aux, hipStream_t s) {
-    const int ntx = (bc.n[0] + TX - 1) / TX, nty = (bc.n[1] + TY - 1) / TY, nzc = (bc.n[2] + ZC - 1) / ZC;
+    const int ntx = (bc.n[0] + TX - 1) / TX, nty = (bc.n[1] + TY - 1) / TY;
+    const int zc = chunk_planes(ntx * nty, bc.n[2]), nzc = (bc.n[2] + zc - 1) / zc;
     const int grid = (ntx * nty * nzc + 7) / 8 * 8;
-    // Grids of whole column tiles take the form with every memory
-    // instruction issued unconditionally.
-    if (bc.n[0] % TX == 0 && bc.n[1] % TY == 0)
-        hipLaunchKernelGGL((fused_step_kernel<TX, TY, ZC, true, double, true>), dim3(grid), dim3(TX * TY), 0, s, f,
-                           bc, k, pull, aux, ntx, nty, nzc, 0);
-    else
-        hipLaunchKernelGGL((fused_step_kernel<TX, TY, ZC, true, double>), dim3(grid), dim3(TX * TY), 0, s, f, bc, k,
-                           pull, aux, ntx, nty, nzc, 0);
+    bool walls = false;
+    for (int face = 0; face < 6; ++face)
+        walls = walls || bc.qkind[face] != QB_PERIODIC || bc.ukind[face] != UB_PERIODIC;
+    auto go = [&](auto masked, auto adv) {
+        hipLaunchKernelGGL((fused64_kernel<TX, TY, decltype(masked)::value, decltype(adv)::value>), dim3(grid),
+                           dim3(TX * TY), 0, s, f, bc, k, pull, aux, ntx, nty, nzc, zc);
+    };
+    auto with_adv = [&](auto masked) {
+        if (k.advection) go(masked, std::integral_constant<int, 1>{});
+        else go(masked, std::integral_constant<int, 0>{});
+    };
+    if (walls) {
+        with_adv(std::true_type{});
+        launch_shells(f, bc, k, pull, aux, s);
+    } else {
+        with_adv(std::false_type{});
+    }
 }
 
 void launch_fused_step_f64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int tile,
                            int pull, int aux, hipStream_t s) {
-    switch (tile) {
-        case 0: launch_tile64<32, 4, 64>(f, bc, k, pull, aux, s); break;
-        case 1: launch_tile64<32, 4, 128>(f, bc, k, pull, aux, s); break;
-        case 2: launch_tile64<16, 8, 64>(f, bc, k, pull, aux, s); break;
-        case 3: launch_tile64<16, 8, 32>(f, bc, k, pull, aux, s); break;
-        case 4: launch_tile64<32, 8, 64>(f, bc, k, pull, aux, s); break;
-        case 5: launch_tile64<64, 4, 64>(f, bc, k, pull, aux, s); break;
-        default: launch_tile64<32, 4, 32>(f, bc, k, pull, aux, s); break;
-    }
+    if (tile == 0) launch_tile64<32, 8>(f, bc, k, pull, aux, s);
+    else launch_tile64<16, 16>(f, bc, k, pull, aux, s);
 }
 }  // namespace lbm

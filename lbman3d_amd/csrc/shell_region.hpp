@@ -18,7 +18,8 @@ struct ShellRegion {
     long part[3];   // cells of the x, y and z parts
 };
 
-inline ShellRegion make_shell_region(const BCDesc<float>& bc, int w) {
+template <typename T>
+ShellRegion make_shell_region(const BCDesc<T>& bc, int w) {
     ShellRegion r{};
     int band[3];
     for (int a = 0; a < 3; ++a) {
