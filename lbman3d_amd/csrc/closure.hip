@@ -68,7 +68,10 @@ __device__ __forceinline__ int wrap(int t, int n) { return t < 0 ? t + n : (t >=
 // EPI: 0 = store BF16 with bias + ReLU,
 // 2 = store FP32 channels-first [co][cell] with bias (final layer),
 // 3 = add alpha * (value + bias) / out_scale to the simulation's Q (final
-// layer applied in place), 4 = store BF16 linear, zero where the stored
+// layer applied in place), 5 = the loss of a training sample in place of the
+// prediction: dL/dpred = 2 (pred - target) / (5 V) as BF16 [cell][8] (channels
+// 5..7 zero) for the backward convolutions, and the block's sum of squared
+// errors, 4 = store BF16 linear, zero where the stored
 // activation `act` of the same cell and channel is not positive (the input
 // gradient through a ReLU).
 constexpr int kTX = 16, kTY = 4;
@@ -77,11 +80,14 @@ struct ConvIO {
     const __bf16* in;          // SRC 0
     const float* fin[8];       // SRC 1: Qxx, Qxy, Qxz, Qyy, Qyz, ux, uy, uz
     const float* in_scale;     // SRC 1
-    void* out;                 // EPI 0-2, 4
+    void* out;                 // EPI 0-2, 4, 5
     const __bf16* act;         // EPI 4: [cell][cout]
     float* q[5];               // EPI 3
     const float* out_scale;    // EPI 3
     float alpha;               // EPI 3
+    const float* target;       // EPI 5: [5][cell]
+    float* loss;               // EPI 5: one sum per block
+    float scale;               // EPI 5: 2 / (5 V)
 };
 
 template <int CIN, int NT, int EPI, int WZ, int SRC>
@@ -151,7 +157,7 @@ conv_fwd_kernel(ConvIO io, const bf16x8* __restrict__ wpk, const float* __restri
     }
     // D fragment: lane holds rows 4*kb + r (x within the row tile), column n*16 + m (channel).
     const long V = (long)nx * ny * nz;
-    if constexpr (EPI == 2 || EPI == 3) {
+    if constexpr (EPI == 2 || EPI == 3 || EPI == 5) {
         // FP32 channels-first output: in fragment order each store would
         // touch 4 cells 16 B apart per channel. The values go through LDS
         // (the input tile is no longer read) so that a thread finishes one
@@ -170,13 +176,39 @@ conv_fwd_kernel(ConvIO io, const bf16x8* __restrict__ wpk, const float* __restri
                 for (int r = 0; r < 4; ++r) so[m * NC + (w * kTY + t) * kTX + 4 * kb + r] = acc[t][0][r] + bco;
         }
         __syncthreads();
+        float sq = 0.f;
         for (int i = threadIdx.x; i < NC; i += 64 * WZ) {
             const int lx = i % kTX, ly = (i / kTX) % kTY, lz = i / (kTX * kTY);
             const long cell = ((long)(bz * WZ + lz) * ny + by * kTY + ly) * nx + bx * kTX + lx;
+            if constexpr (EPI == 5) {
+                bf16x8 grad;
+#pragma unroll
+                for (int co = 0; co < 8; ++co) {
+                    float d = 0.f;
+                    if (co < kOutC) {
+                        d = so[co * NC + i] - io.target[(long)co * V + cell];
+                        sq += d * d;
+                    }
+                    grad[co] = to_bf16(io.scale * d);
+                }
+                reinterpret_cast<bf16x8*>(io.out)[cell] = grad;
+                continue;
+            }
             for (int co = 0; co < cout; ++co) {
                 const float v = so[co * NC + i];
                 if (EPI == 3) io.q[co][cell] += io.alpha * v / io.out_scale[co];
                 else reinterpret_cast<float*>(io.out)[(long)co * V + cell] = v;
+            }
+        }
+        if constexpr (EPI == 5) {
+            for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off, 64);
+            __syncthreads();   // so is read
+            if (lane == 0) so[w] = sq;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                float sum = so[0];
+                for (int i = 1; i < WZ; ++i) sum += so[i];
+                io.loss[blockIdx.x] = sum;
             }
         }
         return;
@@ -360,68 +392,6 @@ conv_wgrad_kernel(const __bf16* __restrict__ in, const __bf16* __restrict__ dout
     }
 }
 
-// Sum of the per-block partials [block][27 cin + 1][cout]: the weight rows go
-// to gw ([off][ci][co]), the last row to gb. A block of 256 threads owns 64
-// consecutive outputs; its four wavefronts add every fourth partial (eight
-// loads in flight per lane), and LDS adds the four sums.
-__global__ void __launch_bounds__(256)
-wgrad_reduce_kernel(const float* __restrict__ part, int nblocks, int krows, int cout, float* __restrict__ gw,
-                    float* __restrict__ gb) {
-    __shared__ float red[4][64];
-    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const long n = (long)krows * cout;
-    const long i = (long)blockIdx.x * 64 + lane;
-    float s = 0.f;
-    if (i < n) {
-        int b = g;
-        for (; b + 28 < nblocks; b += 32) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = part[(long)(b + 4 * u) * n + i];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) s += v[u];
-        }
-        for (; b < nblocks; b += 4) s += part[(long)b * n + i];
-    }
-    red[g][lane] = s;
-    __syncthreads();
-    if (g == 0 && i < n) {
-        const float t = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-        if (i < (long)(krows - 1) * cout) gw[i] = t;
-        else gb[i - (long)(krows - 1) * cout] = t;
-    }
-}
-
-// Mean-squared loss over V cells x 5 channels: dL/dpred = 2 (pred - y) / (5 V),
-// written as BF16 [cell][8] (channels 5..7 zero) for the backward convolutions;
-// per-block partial sums of the squared error.
-__global__ void __launch_bounds__(256)
-loss_grad_kernel(const float* __restrict__ pred, const float* __restrict__ target, long V, __bf16* __restrict__ dout,
-                 float* __restrict__ partial) {
-    __shared__ float red[256];
-    float s = 0.f;
-    const float scale = 2.0f / (kOutC * (float)V);
-    for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < V; c += (long)gridDim.x * blockDim.x) {
-#pragma unroll
-        for (int co = 0; co < 8; ++co) {
-            float g = 0.f;
-            if (co < kOutC) {
-                const float d = pred[co * V + c] - target[co * V + c];
-                s += d * d;
-                g = scale * d;
-            }
-            dout[c * 8 + co] = to_bf16(g);
-        }
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
 // Pack FP32 master weights W[off][ci][co] into B fragments for a
 // convolution kernel whose input has kcin channels per cell (K index
 // off * kcin + c). transpose: pack the input-gradient weights
@@ -463,17 +433,71 @@ __global__ void pack_kernel(PackJobs jobs) {
     jobs.out[jb][idx] = v;
 }
 
-__global__ void adam_kernel(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, long n, float lr, float b1, float b2, float eps, float c1,
-                            float c2) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// Gradient of every layer from the partials of its weight-gradient blocks
+// ([block][27 cin + 1][cout], the last row the bias), and (adam) the Adam step
+// with the new weights written into the B fragments that hold them, all in
+// one launch: as a reduction per layer, an Adam pass and a pack pass these were
+// five launches and 25 us of a 64^3 training step. A block of 256 threads owns 64
+// consecutive outputs of one layer; its four wavefronts add every fourth
+// partial (eight loads in flight per lane), LDS adds the four sums.
+struct UpdateLayer {
+    const float* part;
+    int nblocks, cin, cout;
+    long off_w, off_b;   // in the flat parameter arrays
+    __bf16 *pk, *pkt;    // forward and (or null) input-gradient fragments
+    int nt, ntt, kcin_t;
+    int first;           // first block of this layer
+};
+struct UpdateJobs {
+    UpdateLayer layer[3];
+};
+struct AdamArgs {
+    float *w, *g, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+    int adam;
+};
+// Place of B element (k, n) in fragments of nt column tiles.
+__device__ __forceinline__ long fragment_index(int k, int n, int nt) {
+    return ((((long)(k >> 5) * nt + (n >> 4)) * 64 + ((k >> 3) & 3) * 16 + (n & 15)) << 3) + (k & 7);
+}
+
+__global__ void __launch_bounds__(256) update_kernel(UpdateJobs jobs, AdamArgs a) {
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int l = (int)blockIdx.x >= jobs.layer[2].first ? 2 : ((int)blockIdx.x >= jobs.layer[1].first ? 1 : 0);
+    const UpdateLayer& L = jobs.layer[l];
+    const int weights = 27 * L.cin * L.cout;
+    const long n = weights + L.cout;
+    const long i = (long)(blockIdx.x - L.first) * 64 + lane;
+    float s = 0.f;
+    if (i < n) {
+        int b = grp;
+        for (; b + 28 < L.nblocks; b += 32) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = L.part[(long)(b + 4 * u) * n + i];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; b < L.nblocks; b += 4) s += L.part[(long)b * n + i];
+    }
+    red[grp][lane] = s;
+    __syncthreads();
+    if (grp != 0 || i >= n) return;
+    const float gi = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    const long p = i < weights ? L.off_w + i : L.off_b + (i - weights);
+    a.g[p] = gi;
+    if (!a.adam) return;
+    const float mi = a.b1 * a.m[p] + (1.f - a.b1) * gi;
+    const float vi = a.b2 * a.v[p] + (1.f - a.b2) * gi * gi;
+    a.m[p] = mi;
+    a.v[p] = vi;
+    const float wi = a.w[p] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+    a.w[p] = wi;
+    if (i >= weights) return;
+    const int co = (int)i % L.cout, oc = (int)i / L.cout, ci = oc % L.cin, off = oc / L.cin;
+    L.pk[fragment_index(off * L.cin + ci, co, L.nt)] = to_bf16(wi);
+    if (L.pkt) L.pkt[fragment_index((26 - off) * L.kcin_t + co, ci, L.ntt)] = to_bf16(wi);
 }
 
 // MFMA lane-layout check: D = A (16x32) * B (32x16) through the same
@@ -515,9 +539,9 @@ struct lbm_closure {
     __bf16 *x = nullptr, *a1 = nullptr, *a2 = nullptr;   // activations [cell][C]
     __bf16 *d3 = nullptr, *d2 = nullptr, *d1 = nullptr;   // gradients [cell][C]
     float* pred = nullptr;                                // [5][cell]
-    float* part = nullptr;                                // weight-gradient partials
-    long part_elems = 0;
-    float* loss_part = nullptr;
+    float* part[3] = {nullptr, nullptr, nullptr};         // weight-gradient partials per layer
+    int part_blocks[3] = {0, 0, 0};                       // blocks that wrote them
+    float* loss_part = nullptr;                           // [kLossSteps][loss_blocks] sums of squared errors
     int loss_blocks = 0;
     float* in_scale = nullptr;
     float* out_scale = nullptr;
@@ -559,6 +583,9 @@ int cl_alloc(lbm_closure* c, T** p, size_t elems) {
     return LBM_OK;
 }
 
+// Stored channels of layer l's output gradient.
+int gradient_channels(const lbm_closure* c, int l) { return c->cout[l] <= 8 ? 8 : c->cout[l]; }
+
 int repack(lbm_closure* c) {
     PackJobs jobs{};
     long n = 0;
@@ -578,22 +605,26 @@ int repack(lbm_closure* c) {
     for (int l = 0; l < 3; ++l) add(l, 0, c->cin[l], c->kch[l], c->nt[l], c->pk[l]);
     // input of the transposed convolution: the layer's output gradient,
     // stored with 8 channels (padded) for the last layer, else cout
-    for (int l = 1; l < 3; ++l)
-        add(l, 1, c->cout[l] <= 8 ? 8 : c->cout[l], c->kcht[l - 1], c->ntt[l - 1], c->pkt[l - 1]);
+    for (int l = 1; l < 3; ++l) add(l, 1, gradient_channels(c, l), c->kcht[l - 1], c->ntt[l - 1], c->pkt[l - 1]);
     hipLaunchKernelGGL(pack_kernel, dim3(blocks_for(n)), dim3(256), 0, c->stream, jobs);
     CHK(hipGetLastError());
     return LBM_OK;
 }
 
+// Losses stay on the device for this many training steps between two reads.
+constexpr int kLossSteps = 64;
+
 // One convolution launch: blocks of 8 wavefronts (16 x 4 x 8 output cells)
 // when nz is a multiple of 8, else of 4 (nz is a multiple of 4).
+long conv_blocks(const lbm_closure* c) { return c->V / (kTX * kTY * (c->nz % 8 == 0 ? 8 : 4)); }
+
 template <int CIN, int NT, int EPI, int SRC = 0>
 void conv(const lbm_closure* c, const ConvIO& io, const bf16x8* wpk, const float* bias, int cout, hipStream_t s) {
     if (c->nz % 8 == 0)
-        hipLaunchKernelGGL((conv_fwd_kernel<CIN, NT, EPI, 8, SRC>), dim3(c->V / (kTX * kTY * 8)), dim3(512), 0, s,
+        hipLaunchKernelGGL((conv_fwd_kernel<CIN, NT, EPI, 8, SRC>), dim3((unsigned)conv_blocks(c)), dim3(512), 0, s,
                            io, wpk, bias, cout, c->nx, c->ny, c->nz);
     else
-        hipLaunchKernelGGL((conv_fwd_kernel<CIN, NT, EPI, 4, SRC>), dim3(c->V / (kTX * kTY * 4)), dim3(256), 0, s,
+        hipLaunchKernelGGL((conv_fwd_kernel<CIN, NT, EPI, 4, SRC>), dim3((unsigned)conv_blocks(c)), dim3(256), 0, s,
                            io, wpk, bias, cout, c->nx, c->ny, c->nz);
 }
 
@@ -635,62 +666,104 @@ int forward_apply(lbm_closure* c, const Fields<float>& f, double alpha, hipStrea
     return LBM_OK;
 }
 
-// Weight and bias gradient of one layer (input `in` with cin channels per
-// cell, output gradient `dout` with cs stored channels of which cout are
-// real) into gw [off][ci][co] and gb [co].
-int wgrad(lbm_closure* c, const __bf16* in, int cin, const __bf16* dout, int cs, int cout, float* gw, float* gb) {
+// Weight- and bias-gradient partials of one layer (input `in` with cin channels
+// per cell, output gradient `dout` with cs stored channels of which cout are
+// real).
+int wgrad(lbm_closure* c, int layer, const __bf16* in, const __bf16* dout, int cs) {
+    const int cin = c->cin[layer], cout = c->cout[layer];
     const int ntiles = (int)(c->V / (kWgTX * kWgTY * kWgTZ));
     const int nblk = std::min(ntiles, c->wg_blocks);
     const int per = (ntiles + nblk - 1) / nblk;
     const int blocks = (ntiles + per - 1) / per;
-    const int krows = 27 * cin + 1;
-    if ((long)blocks * krows * cout > c->part_elems) return fail(LBM_ERR_STATE, "wgrad scratch too small");
+    c->part_blocks[layer] = blocks;
+    float* part = c->part[layer];
     const dim3 grid(blocks), block(64 * kWgWaves);
     if (cin == 8 && cs == 32)
-        hipLaunchKernelGGL((conv_wgrad_kernel<8, 32>), grid, block, 0, c->stream, in, dout, cout, c->part, ntiles, per,
+        hipLaunchKernelGGL((conv_wgrad_kernel<8, 32>), grid, block, 0, c->stream, in, dout, cout, part, ntiles, per,
                            c->nx, c->ny, c->nz);
     else if (cin == 32 && cs == 32)
-        hipLaunchKernelGGL((conv_wgrad_kernel<32, 32>), grid, block, 0, c->stream, in, dout, cout, c->part, ntiles,
+        hipLaunchKernelGGL((conv_wgrad_kernel<32, 32>), grid, block, 0, c->stream, in, dout, cout, part, ntiles,
                            per, c->nx, c->ny, c->nz);
     else if (cin == 32 && cs == 8)
-        hipLaunchKernelGGL((conv_wgrad_kernel<32, 8>), grid, block, 0, c->stream, in, dout, cout, c->part, ntiles, per,
+        hipLaunchKernelGGL((conv_wgrad_kernel<32, 8>), grid, block, 0, c->stream, in, dout, cout, part, ntiles, per,
                            c->nx, c->ny, c->nz);
     else
         return fail(LBM_ERR_UNSUPPORTED, "closure layer shape");
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(blocks_for((long)krows * cout, 64)), dim3(256), 0, c->stream,
-                       c->part, blocks, krows, cout, gw, gb);
-    CHK(hipGetLastError());
     return LBM_OK;
 }
 
-// Forward + backward for one sample; gradient into c->g, loss (sum of
-// squared errors / (5V)) returned through loss_out (synchronises).
-int loss_and_grad(lbm_closure* c, const __bf16* x, const float* y, double* loss_out) {
-    if (int r = forward(c, x, c->stream)) return r;
+// Forward and backward of one sample up to the gradient partials; the block
+// sums of the squared error go to row `slot` of c->loss_part.
+int backward(lbm_closure* c, const __bf16* x, const float* y, int slot) {
     const int H = c->hidden;
-    const long V = c->V;
-    hipLaunchKernelGGL(loss_grad_kernel, dim3(c->loss_blocks), dim3(256), 0, c->stream, c->pred, y, V, c->d3,
-                       c->loss_part);
+    conv<8, 2, 0>(c, io_bf16(x, c->a1), c->pk[0], c->w + c->off_b[0], H, c->stream);
+    conv<32, 2, 0>(c, io_bf16(c->a1, c->a2), c->pk[1], c->w + c->off_b[1], H, c->stream);
+    ConvIO last = io_bf16(c->a2, c->d3);
+    last.target = y;
+    last.loss = c->loss_part + (long)slot * c->loss_blocks;
+    last.scale = 2.0f / (kOutC * (float)c->V);
+    conv<32, 1, 5>(c, last, c->pk[2], c->w + c->off_b[2], kOutC, c->stream);
     // layer 3: weights, bias, input gradient (8-channel padded gradient in, H out)
-    if (int r = wgrad(c, c->a2, H, c->d3, 8, kOutC, c->g + c->off_w[2], c->g + c->off_b[2])) return r;
+    if (int r = wgrad(c, 2, c->a2, c->d3, 8)) return r;
     ConvIO g2 = io_bf16(c->d3, c->d2);
     g2.act = c->a2;
     conv<8, 2, 4>(c, g2, c->pkt[1], nullptr, H, c->stream);
     // layer 2
-    if (int r = wgrad(c, c->a1, H, c->d2, H, H, c->g + c->off_w[1], c->g + c->off_b[1])) return r;
+    if (int r = wgrad(c, 1, c->a1, c->d2, H)) return r;
     ConvIO g1 = io_bf16(c->d2, c->d1);
     g1.act = c->a1;
     conv<32, 2, 4>(c, g1, c->pkt[0], nullptr, H, c->stream);
     // layer 1
-    if (int r = wgrad(c, x, kInC, c->d1, H, H, c->g + c->off_w[0], c->g + c->off_b[0])) return r;
+    if (int r = wgrad(c, 0, x, c->d1, H)) return r;
     CHK(hipGetLastError());
-    if (loss_out) {
-        std::vector<float> lp(c->loss_blocks);
-        CHK(hipMemcpyAsync(lp.data(), c->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-        CHK(hipStreamSynchronize(c->stream));
+    return LBM_OK;
+}
+
+// Gradient into c->g, and the Adam step `step` (from 1) where lr is given.
+int update(lbm_closure* c, const double* lr, long step) {
+    const float b1 = 0.9f, b2 = 0.999f;
+    UpdateJobs jobs{};
+    int first = 0;
+    for (int l = 0; l < 3; ++l) {
+        UpdateLayer& u = jobs.layer[l];
+        u.part = c->part[l];
+        u.nblocks = c->part_blocks[l];
+        u.cin = c->cin[l];
+        u.cout = c->cout[l];
+        u.off_w = c->off_w[l];
+        u.off_b = c->off_b[l];
+        u.pk = reinterpret_cast<__bf16*>(c->pk[l]);
+        u.nt = c->nt[l];
+        if (l > 0) {
+            u.pkt = reinterpret_cast<__bf16*>(c->pkt[l - 1]);
+            u.ntt = c->ntt[l - 1];
+            u.kcin_t = gradient_channels(c, l);
+        }
+        u.first = first;
+        first += (int)blocks_for(27L * u.cin * u.cout + u.cout, 64);
+    }
+    AdamArgs a{c->w, c->g, c->m, c->v, 0.f, b1, b2, 1e-8f, 1.f, 1.f, 0};
+    if (lr) {
+        a.lr = (float)*lr;
+        a.c1 = 1.f - std::pow(b1, (float)step);
+        a.c2 = 1.f - std::pow(b2, (float)step);
+        a.adam = 1;
+    }
+    hipLaunchKernelGGL(update_kernel, dim3(first), dim3(256), 0, c->stream, jobs, a);
+    CHK(hipGetLastError());
+    return LBM_OK;
+}
+
+// Adds the mean squared errors of the first `rows` rows of c->loss_part to sum
+// (synchronises).
+int read_losses(lbm_closure* c, int rows, double* sum) {
+    std::vector<float> lp((size_t)rows * c->loss_blocks);
+    CHK(hipMemcpyAsync(lp.data(), c->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+    CHK(hipStreamSynchronize(c->stream));
+    for (int r = 0; r < rows; ++r) {
         double s = 0.0;
-        for (float f : lp) s += f;
-        *loss_out = s / (kOutC * (double)V);
+        for (int b = 0; b < c->loss_blocks; ++b) s += lp[(size_t)r * c->loss_blocks + b];
+        *sum += s / (kOutC * (double)c->V);
     }
     return LBM_OK;
 }
@@ -776,10 +849,10 @@ int lbm_closure_create(int32_t nx, int32_t ny, int32_t nz, int32_t hidden, uint6
         (r = cl_alloc(c, &c->d3, V * 8)) || (r = cl_alloc(c, &c->d2, V * H)) || (r = cl_alloc(c, &c->d1, V * H)) ||
         (r = cl_alloc(c, &c->pred, V * kOutC)))
         return bail(r);
-    c->part_elems = (long)c->wg_blocks * (27L * 32 + 1) * 32;
-    if ((r = cl_alloc(c, &c->part, c->part_elems))) return bail(r);
-    c->loss_blocks = 512;
-    if ((r = cl_alloc(c, &c->loss_part, c->loss_blocks))) return bail(r);
+    for (int l = 0; l < 3; ++l)
+        if ((r = cl_alloc(c, &c->part[l], (size_t)c->wg_blocks * (27L * c->cin[l] + 1) * c->cout[l]))) return bail(r);
+    c->loss_blocks = (int)conv_blocks(c);
+    if ((r = cl_alloc(c, &c->loss_part, (size_t)kLossSteps * c->loss_blocks))) return bail(r);
     if ((r = cl_alloc(c, &c->in_scale, 8)) || (r = cl_alloc(c, &c->out_scale, 8))) return bail(r);
     // He-normal initial weights from the counter-based stream, zero biases.
     std::vector<float> w(c->nparams, 0.f);
@@ -885,18 +958,16 @@ int lbm_closure_train(lbm_closure_handle c, int32_t iters, double lr, uint64_t s
     if (c->sx.empty()) return fail(LBM_ERR_STATE, "no training samples");
     double acc = 0.0;
     const int ns = (int)c->sx.size();
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    int row = 0;   // losses wait on the device, so that a step waits for nothing
     for (int it = 0; it < iters; ++it) {
         const int s = (int)(uniform01(seed, (uint64_t)(c->step), 11) * ns) % ns;
-        double loss = 0.0;
-        const bool want = mean_loss != nullptr;
-        if (int r = loss_and_grad(c, c->sx[s], c->sy[s], want ? &loss : nullptr)) return r;
-        acc += loss;
-        ++c->step;
-        const float c1 = 1.f - std::pow(b1, (float)c->step), c2 = 1.f - std::pow(b2, (float)c->step);
-        hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(c->nparams)), dim3(256), 0, c->stream, c->w, c->g, c->m, c->v,
-                           c->nparams, (float)lr, b1, b2, eps, c1, c2);
-        if (int r = repack(c)) return r;
+        if (int r = backward(c, c->sx[s], c->sy[s], row)) return r;
+        if (int r = update(c, &lr, ++c->step)) return r;
+        if (++row == kLossSteps || it == iters - 1) {
+            if (mean_loss)
+                if (int r = read_losses(c, row, &acc)) return r;
+            row = 0;
+        }
     }
     CHK(hipStreamSynchronize(c->stream));
     if (mean_loss) *mean_loss = acc / iters;
@@ -909,7 +980,10 @@ int lbm_closure_loss_and_grad(lbm_closure_handle c, const double* x, const doubl
     CHK(hipMalloc(&dy, c->V * kOutC * sizeof(float)));
     int r = upload_x(c, x, c->x);
     if (!r) r = upload_y(c, y, dy);
-    if (!r) r = loss_and_grad(c, c->x, dy, loss);
+    if (!r) r = backward(c, c->x, dy, 0);
+    if (!r) r = update(c, nullptr, 0);
+    *loss = 0.0;
+    if (!r) r = read_losses(c, 1, loss);
     if (!r && grad) {
         std::vector<float> h(c->nparams);
         if (hipMemcpyAsync(h.data(), c->g, h.size() * sizeof(float), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
