@@ -288,37 +288,68 @@ conv_wgrad_kernel(const __bf16* __restrict__ in, const __bf16* __restrict__ dout
 #pragma unroll
     for (int j = 0; j < 8; ++j) ones[j] = to_bf16(1.f);
 
-    for (int tile = t0; tile < t1; ++tile) {
+    // The vectors of the next tile are loaded into registers before the products
+    // of the current one (two cells of a pair each: 10 pairs x 24 rows x CVI of
+    // the input halo, 8 pairs x 8 rows x CVO of dOut): at 64^3 a block takes eight
+    // tiles, and loading each between its barriers left the matrix cores
+    // waiting for memory eight times.
+    constexpr int kThreads = 64 * kWgWaves;
+    constexpr int kItA = 10 * kWgHY * kWgHZ * CVI, kItB = 8 * kWgTY * kWgTZ * CVO;
+    constexpr int kA = (kItA + kThreads - 1) / kThreads, kB = (kItB + kThreads - 1) / kThreads;
+    u16x8 ra[kA][2], rb[kB][2];
+    auto load_tile = [&](int tile) {
         // tiles z-fastest, so a block's consecutive tiles share halo planes in L2
         const int tz = tile % (nz / kWgTZ), txy = tile / (nz / kWgTZ);
         const int x0 = (txy % ntx) * kWgTX, y0 = (txy / ntx) * kWgTY, z0 = tz * kWgTZ;
-        __syncthreads();   // the previous tile's LDS reads are done
-        // input halo: 10 cell pairs per row x 24 rows x CVI vectors
-        for (int it = tid; it < 10 * kWgHY * kWgHZ * CVI; it += 64 * kWgWaves) {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+            const int it = tid + i * kThreads;
+            if (it >= kItA) continue;
             const int cv = it % CVI, pr = it / CVI;
             const int p = pr % 10, row = pr / 10;
-            const int hy = row % kWgHY, hz = row / kWgHY;
-            const long rbase = ((long)wrap(z0 - 1 + hz, nz) * ny + wrap(y0 - 1 + hy, ny)) * nx;
-            const int xa = wrap(x0 - 2 + 2 * p, nx), xb = wrap(x0 - 1 + 2 * p, nx);
-            const u16x8 va = *reinterpret_cast<const u16x8*>(in + (rbase + xa) * CIN + cv * 8);
-            const u16x8 vb = *reinterpret_cast<const u16x8*>(in + (rbase + xb) * CIN + cv * 8);
-            const int e = 8 + row * kWgRL + 2 * p - 2;   // element index of x0 - 2 + 2p in channel 0
-#pragma unroll
-            for (int j = 0; j < 8; ++j) sA32[((cv * 8 + j) * kWgAStr + e) >> 1] = (uint32_t)va[j] | ((uint32_t)vb[j] << 16);
+            const long rbase = ((long)wrap(z0 - 1 + row / kWgHY, nz) * ny + wrap(y0 - 1 + row % kWgHY, ny)) * nx;
+            ra[i][0] = *reinterpret_cast<const u16x8*>(in + (rbase + wrap(x0 - 2 + 2 * p, nx)) * CIN + cv * 8);
+            ra[i][1] = *reinterpret_cast<const u16x8*>(in + (rbase + wrap(x0 - 1 + 2 * p, nx)) * CIN + cv * 8);
         }
-        // dOut tile: 8 cell pairs per row x 8 rows x CVO vectors
-        for (int it = tid; it < 8 * kWgTY * kWgTZ * CVO; it += 64 * kWgWaves) {
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            const int it = tid + i * kThreads;
+            if (it >= kItB) continue;
             const int cv = it % CVO, pr = it / CVO;
             const int p = pr % 8, row = pr / 8;
-            const int yy = row % kWgTY, zz = row / kWgTY;
-            const long c = ((long)(z0 + zz) * ny + y0 + yy) * nx + x0 + 2 * p;
-            const u16x8 va = *reinterpret_cast<const u16x8*>(dout + c * CS + cv * 8);
-            const u16x8 vb = *reinterpret_cast<const u16x8*>(dout + (c + 1) * CS + cv * 8);
-            const int e = row * kWgTX + 2 * p;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) sB32[((cv * 8 + j) * kWgBStr + e) >> 1] = (uint32_t)va[j] | ((uint32_t)vb[j] << 16);
+            const long c = ((long)(z0 + row / kWgTY) * ny + y0 + row % kWgTY) * nx + x0 + 2 * p;
+            rb[i][0] = *reinterpret_cast<const u16x8*>(dout + c * CS + cv * 8);
+            rb[i][1] = *reinterpret_cast<const u16x8*>(dout + (c + 1) * CS + cv * 8);
         }
+    };
+    auto store_tile = [&]() {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+            const int it = tid + i * kThreads;
+            if (it >= kItA) continue;
+            const int cv = it % CVI, pr = it / CVI;
+            const int e = 8 + (pr / 10) * kWgRL + 2 * (pr % 10) - 2;   // element index of the pair in channel 0
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                sA32[((cv * 8 + j) * kWgAStr + e) >> 1] = (uint32_t)ra[i][0][j] | ((uint32_t)ra[i][1][j] << 16);
+        }
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            const int it = tid + i * kThreads;
+            if (it >= kItB) continue;
+            const int cv = it % CVO, pr = it / CVO;
+            const int e = (pr / 8) * kWgTX + 2 * (pr % 8);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                sB32[((cv * 8 + j) * kWgBStr + e) >> 1] = (uint32_t)rb[i][0][j] | ((uint32_t)rb[i][1][j] << 16);
+        }
+    };
+    if (t0 < t1) load_tile(t0);
+    for (int tile = t0; tile < t1; ++tile) {
+        __syncthreads();   // the previous tile's LDS reads are done
+        store_tile();
         __syncthreads();
+        if (tile + 1 < t1) load_tile(tile + 1);
 #pragma unroll
         for (int s = 0; s < kWgTY * kWgTZ / 2; ++s) {
             const int rr = 2 * s + (kb >> 1), xo = 8 * (kb & 1);
