@@ -97,7 +97,11 @@ conv_fwd_kernel(ConvIO io, const bf16x8* __restrict__ wpk, const float* __restri
     static_assert(SRC == 0 || CIN == 8, "field input has 8 channels");
     constexpr int CV = CIN / 8;                  // 16-byte vectors per cell
     constexpr int HX = kTX + 2, HY = kTY + 2, HZ = WZ + 2, NH = HX * HY * HZ;
-    __shared__ bf16x8 tile[NH * CV];
+    // The input gradient leaves through LDS: 16-byte vectors of a cell's channels,
+    // records padded to kRec so that a fragment's four rows of cells fall into
+    // different banks.
+    constexpr int kRec = 16 * NT + 8, kOutVecs = EPI == 4 ? WZ * kTY * kTX * kRec / 8 : 0;
+    __shared__ bf16x8 tile[NH * CV > kOutVecs ? NH * CV : kOutVecs];
     const int ntx = nx / kTX, nty = ny / kTY;
     const int bx = blockIdx.x % ntx, by = (blockIdx.x / ntx) % nty, bz = blockIdx.x / (ntx * nty);
     const int x0 = bx * kTX - 1, y0 = by * kTY - 1, z0 = bz * WZ - 1;
@@ -213,23 +217,46 @@ conv_fwd_kernel(ConvIO io, const bf16x8* __restrict__ wpk, const float* __restri
         }
         return;
     }
+    if constexpr (EPI == 4) {
+        // In fragment order every lane read one saved activation and stored one
+        // gradient of 2 bytes, 64 B apart: 26 against 19 us for the same 32 -> 32
+        // convolution forward at 64^3.
+        __bf16* so = reinterpret_cast<__bf16*>(tile);
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int t = 0; t < kTY; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    so[((w * kTY + t) * kTX + 4 * kb + r) * kRec + n * 16 + m] = to_bf16(acc[t][n][r]);
+        __syncthreads();
+        constexpr int kVecs = 2 * NT;   // vectors per cell: cout is 16 NT
+        for (int v = threadIdx.x; v < WZ * kTY * kTX * kVecs; v += 64 * WZ) {
+            const int i = v / kVecs, q = v % kVecs;
+            const int lx = i % kTX, ly = (i / kTX) % kTY, lz = i / (kTX * kTY);
+            const long cell = ((long)(bz * WZ + lz) * ny + by * kTY + ly) * nx + bx * kTX + lx;
+            const bf16x8 act = *reinterpret_cast<const bf16x8*>(io.act + cell * (16 * NT) + q * 8);
+            bf16x8 g = *reinterpret_cast<const bf16x8*>(so + i * kRec + q * 8);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (!(from_bf16(act[j]) > 0.f)) g[j] = to_bf16(0.f);
+            *reinterpret_cast<bf16x8*>(reinterpret_cast<__bf16*>(io.out) + cell * (16 * NT) + q * 8) = g;
+        }
+        return;
+    }
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int co = n * 16 + m;
         if (co >= cout) continue;
-        const float bco = EPI == 4 ? 0.f : bias[co];
+        const float bco = bias[co];
 #pragma unroll
         for (int t = 0; t < kTY; ++t) {
             const long row = ((long)(bz * WZ + w) * ny + by * kTY + t) * nx + bx * kTX;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const long cell = row + 4 * kb + r;
-                float v = acc[t][n][r] + bco;
-                if (EPI == 0) v = v > 0.f ? v : 0.f;
-                if (EPI == 4 && !(from_bf16(io.act[cell * cout + co]) > 0.f)) v = 0.f;
-                if (EPI == 3) io.q[co][cell] += io.alpha * v / io.out_scale[co];
-                else if (EPI == 2) reinterpret_cast<float*>(io.out)[(long)co * V + cell] = v;
-                else reinterpret_cast<__bf16*>(io.out)[cell * cout + co] = to_bf16(v);
+                const float v = acc[t][n][r] + bco;
+                reinterpret_cast<__bf16*>(io.out)[(row + 4 * kb + r) * cout + co] = to_bf16(v > 0.f ? v : 0.f);
             }
         }
     }
