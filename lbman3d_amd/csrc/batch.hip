@@ -38,6 +38,7 @@ struct SimDesc {
     Phys<float> k;
     int periodic;
     int ntx, nty, nzc;
+    int tile_x, tile_y;   // columns of a tile (third pipeline)
     int tile_begin;       // first work item of this simulation
     int pull;             // 0 until the first step after an upload
     int aux_always;       // moving walls read rho every step
@@ -74,7 +75,7 @@ constexpr BatchTile kBatchTiles[] = {
     {0, 32, 8, 32, "32x8x32"},       {0, 16, 16, 32, "16x16x32"},     {0, 32, 8, 16, "32x8x16"},
     {0, 16, 16, 16, "16x16x16"},     {0, 16, 16, 8, "16x16x8"},       {0, 32, 8, 8, "32x8x8"},
     {1, 32, 8, 64, "p2:32x8x64"},    {1, 32, 8, 32, "p2:32x8x32"},    {1, 32, 8, 16, "p2:32x8x16"},
-    {1, 64, 4, 32, "p2:64x4x32"},
+    {1, 64, 4, 32, "p2:64x4x32"},    {1, 0, 0, 64, "p2:rows:64"},
 };
 constexpr int kNumBatchTiles = sizeof(kBatchTiles) / sizeof(kBatchTiles[0]);
 
@@ -104,53 +105,40 @@ struct BatchItem {
     int sim, txy, z0, z1;
 };
 
-// The work list on the third pipeline, as an explicit item list that the
-// host orders longest first (see build_items). A simulation's advection
-// scheme picks the instantiation per work item (uniform over the block).
-template <int TX, int TY, int ZC>
-__global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(2, 2)))
-batch_step_kernel_p2(const SimDesc* __restrict__ descs, const BatchItem* __restrict__ items, int total,
-                     int parity, int aux, unsigned* __restrict__ queue) {
-    using G = TileGeom<TX, TY>;
-    __shared__ float sIn[2][kNumIn][G::NI];
-    __shared__ float sP[2][6][G::NA];
-    __shared__ float sRing[4][kNumIn][G::NR];
-    __shared__ int s_item;
-    // Work queue: blocks take the next item as they finish one, which
-    // balances tiles of uneven length. queue[0] (next item) only grows, so
-    // every block leaves once it passes total; the last block to leave
-    // (queue[1] counts them) resets both for the next launch on the stream.
-    for (;;) {
-        if (threadIdx.x == 0) s_item = (int)atomicAdd(&queue[0], 1u);
-        __syncthreads();
-        const int w = s_item;
-        if (w >= total) break;
+// The work list on the third pipeline: block b runs the items
+// [ranges[b].x, ranges[b].y), which the host has cut so that every block has
+// the same work (see build_items). A simulation's advection scheme and walls
+// pick the instantiation per work item (uniform over the block); its tile
+// shape is a run-time value, which costs 2-3 % of a sweep of equal boxes,
+// but one set of bodies for both shapes is what a mixed sweep's blocks share
+// in the instruction cache (64 mixed boxes 313 us, compile-time shapes 316).
+__global__ void __launch_bounds__(RowGeom::NT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+batch_step_kernel_p2(const SimDesc* __restrict__ descs, const BatchItem* __restrict__ items,
+                     const int2* __restrict__ ranges, int parity, int aux) {
+    using G = RowGeom;
+    __shared__ float sIn[2][kNumIn][G::LI];
+    __shared__ float sP[2][6][G::LA];
+    __shared__ float sRing[4][kNumIn][G::LR];
+    const int2 range = ranges[blockIdx.x];
+    for (int w = range.x; w < range.y; ++w) {
         const BatchItem it = items[w];
         const SimDesc& d = descs[it.sim];
         const int tx = it.txy % d.ntx, ty = it.txy / d.ntx;
         const int a = aux | d.aux_always;
+        const G geo(d.tile_x, d.tile_y);
         if (d.walls) {
             if (d.k.advection != 0)
-                p2_range<TX, TY, false, true, true, false, true>(d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0,
-                                                                 it.z1, sIn, sP, sRing);
+                p2_range<false, true, true, false, true>(geo, d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1,
+                                                         sIn, sP, sRing);
             else
-                p2_range<TX, TY, false, false, true, false, true>(d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0,
-                                                                  it.z1, sIn, sP, sRing);
+                p2_range<false, false, true, false, true>(geo, d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1,
+                                                          sIn, sP, sRing);
         } else if (d.k.advection != 0) {
-            p2_range<TX, TY, true, true, true>(d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1, sIn, sP,
-                                               sRing);
+            p2_range<true, true, true>(geo, d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1, sIn, sP, sRing);
         } else {
-            p2_range<TX, TY, true, false, true>(d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1, sIn, sP,
-                                                sRing);
+            p2_range<true, false, true>(geo, d.f[parity], d.bc, d.k, d.pull, a, tx, ty, it.z0, it.z1, sIn, sP, sRing);
         }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        __threadfence();
-        if (atomicAdd(&queue[1], 1u) == gridDim.x - 1) {
-            atomicExch(&queue[0], 0u);
-            atomicExch(&queue[1], 0u);
-        }
     }
 }
 
@@ -187,23 +175,22 @@ int occupancy_blocks() {
     if constexpr (KIND == 0)
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_step_kernel<TX, TY, ZC>, TX * TY, 0);
     else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_step_kernel_p2<TX, TY, ZC>, TX * TY, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_step_kernel_p2, RowGeom::NT, 0);
     return e == hipSuccess ? std::max(1, nb) : 1;
 }
 
 template <int KIND, int TX, int TY, int ZC>
-void launch_batch(const SimDesc* d, int nsims, int total, const BatchItem* items, int parity, int aux, int grid,
-                  unsigned* queue, hipStream_t s) {
+void launch_batch(const SimDesc* d, int nsims, int total, const BatchItem* items, const int2* ranges, int parity,
+                  int aux, int grid, hipStream_t s) {
     if constexpr (KIND == 0)
         hipLaunchKernelGGL((batch_step_kernel<TX, TY, ZC>), dim3(grid), dim3(TX * TY), 0, s, d, nsims, total,
                            parity, aux);
     else
-        hipLaunchKernelGGL((batch_step_kernel_p2<TX, TY, ZC>), dim3(grid), dim3(TX * TY), 0, s, d, items, total,
-                           parity, aux, queue);
+        hipLaunchKernelGGL(batch_step_kernel_p2, dim3(grid), dim3(RowGeom::NT), 0, s, d, items, ranges, parity, aux);
 }
 
 // Every batch tile shape, in catalogue order: fn(TileTag<KIND, TX, TY, ZC>{}).
-static_assert(kNumBatchTiles == 10, "the dispatch below lists every catalogue entry");
+static_assert(kNumBatchTiles == 11, "the dispatch below lists every catalogue entry");
 template <int K, int X, int Y, int Z>
 struct TileTag {
     static constexpr int kind = K, tx = X, ty = Y, zc = Z;
@@ -217,10 +204,7 @@ auto with_batch_tile(int tile, F&& fn) {
         case 3: return fn(TileTag<0, 16, 16, 16>{});
         case 4: return fn(TileTag<0, 16, 16, 8>{});
         case 5: return fn(TileTag<0, 32, 8, 8>{});
-        case 6: return fn(TileTag<1, 32, 8, 64>{});
-        case 7: return fn(TileTag<1, 32, 8, 32>{});
-        case 8: return fn(TileTag<1, 32, 8, 16>{});
-        default: return fn(TileTag<1, 64, 4, 32>{});
+        default: return fn(TileTag<1, 0, 0, 0>{});
     }
 }
 
@@ -230,10 +214,12 @@ struct lbm_batch {
     std::vector<lbm_handle> sims;
     std::vector<SimDesc> desc;
     SimDesc* d_desc = nullptr;
-    unsigned* d_queue = nullptr;   // work-queue counters of the third-pipeline kernel (reset by the kernel)
-    BatchItem* d_items = nullptr;  // its item list (third-pipeline tiles only)
-    int items_cap = 0;
-    std::vector<BatchItem> items;  // host copy (the upload reads it asynchronously)
+    // Third-pipeline tiles only: the items, and behind them each block's range of them.
+    char* d_items = nullptr;
+    size_t items_cap = 0;          // bytes
+    std::vector<BatchItem> items;  // host copies (the upload reads them asynchronously)
+    std::vector<int2> ranges;
+    std::vector<int> order;        // simulations in the order in which their columns are cut
     hipStream_t stream = nullptr;
     int total = 0;
     int sq_total = 0;      // cells of the shell Q pass (simulations with walls)
@@ -256,13 +242,38 @@ void drop_graphs(lbm_batch* b) {
         }
 }
 
-int tiles_of(const lbm_batch* b, int i, int& ntx, int& nty, int& nzc) {
+int tiles_up(int n, int tile) { return (n + tile - 1) / tile; }
+
+// Columns of a tile of simulation c: the catalogue's, or the shape of 64 x 4
+// and 32 x 8 that covers the nx x ny columns with fewer tiles; 64 x 4 for as
+// many (whole rows: 24 boxes of 48 x 64 x 64 take 258 us with it, 327 us with
+// 32 x 8, whose tiles then begin inside cache lines; 18 boxes of 64^3 take
+// 226 and 241 us). Tiles that fit the columns exactly but begin inside a line
+// (24 x 10, 48 x 5) fetch up to three times the bytes: 698 and 406 us.
+void tile_shape(const BatchTile& t, const lbm_config& c, int& tx, int& ty) {
+    tx = t.tx;
+    ty = t.ty;
+    if (tx) return;
+    long best = 0;
+    for (int w = 64; w >= 32; w /= 2) {
+        const int h = 256 / w;
+        const long cost = (long)tiles_up(c.nx, w) * tiles_up(c.ny, h);
+        if (tx == 0 || cost < best) {
+            best = cost;
+            tx = w;
+            ty = h;
+        }
+    }
+}
+
+int tiles_of(const lbm_batch* b, int i, SimDesc& d) {
     const BatchTile& t = kBatchTiles[b->tile];
     const lbm_config& c = b->sims[i]->cfg;
-    ntx = (c.nx + t.tx - 1) / t.tx;
-    nty = (c.ny + t.ty - 1) / t.ty;
-    nzc = (c.nz + t.zc - 1) / t.zc;
-    return ntx * nty * nzc;
+    tile_shape(t, c, d.tile_x, d.tile_y);
+    d.ntx = tiles_up(c.nx, d.tile_x);
+    d.nty = tiles_up(c.ny, d.tile_y);
+    d.nzc = tiles_up(c.nz, t.zc);
+    return d.ntx * d.nty * d.nzc;
 }
 
 int grid_for_tile(int tile, int total, int limit) {
@@ -279,50 +290,101 @@ int grid_for_tile(int tile, int total, int limit) {
     return limit > 0 ? std::min(grid, limit) : grid;
 }
 
-// Item list of the third-pipeline kernel: every z chunk of every column
-// tile, longest first, so that the blocks of the persistent grid end
-// together; the items of the last round (grid of them) are split into two
-// halves so that the final round is short. Sets total and grid.
-int build_items(lbm_batch* b) {
-    const BatchTile& t = kBatchTiles[b->tile];
-    std::vector<BatchItem>& items = b->items;
-    items.clear();
-    for (size_t i = 0; i < b->sims.size(); ++i) {
+// Items and block ranges of the third-pipeline kernel. The columns of all
+// simulations, one after another, are cut into one range per resident block
+// so that the costliest range is the cheapest possible (by bisection over
+// its cost). Costs, in eighths of a periodic plane: a piece of n planes also
+// fills the pipeline, about two planes' time, and the wall-aware form takes
+// about an eighth more per plane. Before, blocks drew chunks of 16, 32 or 64
+// planes from a queue, longest first, so a sweep with fewer chunks than a few
+// rounds of blocks waited for the last ones: 6 boxes of 24 to 64 per side 95
+// -> 40 us, 20 boxes 127 -> 97 us, 64 boxes 335 -> 308 us, 80 boxes 377 ->
+// 357 us (with the tile shapes above and one loop body).
+// Simulations of one form are neighbours in the order, so that a compute
+// unit's blocks run the same body (18 boxes of 64^3, half of them slits: 256
+// -> 240 us), and neighbouring ranges run on the same XCD (block b runs on
+// XCD b mod 8), whose L2 then holds their shared halo columns.
+constexpr int kPlane = 8, kWallPlane = 9;
+constexpr int kPieceStart = 2 * kPlane;
+constexpr int kPieceMin = 4;   // planes; 6 boxes: 2 the same, 8: 45 -> 57 us
+
+struct BatchSplit {
+    std::vector<BatchItem> items;
+    std::vector<int> first;   // first item of each range
+};
+
+// Greedy cut with every range's cost at most `bound` (or one piece).
+void cut_columns(const lbm_batch* b, int zc, int bound, BatchSplit& out) {
+    out.items.clear();
+    out.first.assign(1, 0);
+    int load = 0;
+    for (int i : b->order) {
         const SimDesc& d = b->desc[i];
         const int nz = d.bc.n[2];
+        const int wp = d.walls ? kWallPlane : kPlane;
         for (int txy = 0; txy < d.ntx * d.nty; ++txy)
-            for (int z0 = 0; z0 < nz; z0 += t.zc) items.push_back({(int)i, txy, z0, std::min(z0 + t.zc, nz)});
-    }
-    auto longer = [](const BatchItem& a, const BatchItem& c) { return a.z1 - a.z0 > c.z1 - c.z0; };
-    std::stable_sort(items.begin(), items.end(), longer);
-    const int grid = grid_for_tile(b->tile, (int)items.size(), b->grid_limit);
-    if ((int)items.size() > 2 * grid) {
-        std::vector<BatchItem> tail(items.end() - grid, items.end());
-        items.resize(items.size() - grid);
-        for (const BatchItem& it : tail) {
-            const int mid = it.z0 + (it.z1 - it.z0) / 2;
-            if (mid > it.z0) {
-                items.push_back({it.sim, it.txy, it.z0, mid});
-                items.push_back({it.sim, it.txy, mid, it.z1});
-            } else {
-                items.push_back(it);
+            for (int z = 0; z < nz;) {
+                const int left = nz - z;
+                const int room = (bound - load - kPieceStart) / wp;
+                if (room < std::min(kPieceMin, left) && load > 0) {
+                    out.first.push_back((int)out.items.size());
+                    load = 0;
+                    continue;
+                }
+                int n = std::min({left, zc, std::max(room, kPieceMin)});
+                if (left - n == 1 && left <= zc) n = left;   // one plane more, not a piece of one
+                out.items.push_back({(int)i, txy, z, z + n});
+                load += kPieceStart + n * wp;
+                z += n;
             }
-        }
-        std::stable_sort(items.begin(), items.end(), longer);
     }
-    if ((int)items.size() > b->items_cap) {
+    out.first.push_back((int)out.items.size());
+}
+
+int build_items(lbm_batch* b) {
+    const int zc = kBatchTiles[b->tile].zc;
+    int planes = 0;
+    for (const SimDesc& d : b->desc) planes += d.ntx * d.nty * d.bc.n[2];
+    const int slots = grid_for_tile(b->tile, planes, b->grid_limit);
+    b->order.resize(b->sims.size());
+    for (size_t i = 0; i < b->order.size(); ++i) b->order[i] = (int)i;
+    auto form = [&](int i) { return 4 * (b->desc[i].tile_x > 32) + 2 * b->desc[i].walls + (b->desc[i].k.advection != 0); };
+    std::stable_sort(b->order.begin(), b->order.end(), [&](int x, int y) { return form(x) < form(y); });
+    BatchSplit split;
+    int lo = kPieceStart + kPlane * kPieceMin, hi = lo;
+    auto fits = [&](int bound) {
+        cut_columns(b, zc, bound, split);
+        return (int)split.first.size() - 1 <= slots;
+    };
+    while (!fits(hi)) hi *= 2;
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (fits(mid)) hi = mid;
+        else lo = mid + 1;
+    }
+    cut_columns(b, zc, hi, split);
+    const int n = (int)split.first.size() - 1;
+    b->items = std::move(split.items);
+    b->ranges.resize(n);
+    for (int r = 0, q = n / 8, m = n % 8; r < n; ++r) {
+        const int xcd = r % 8, at = xcd * q + std::min(xcd, m) + r / 8;
+        b->ranges[r] = int2{split.first[at], split.first[at + 1]};
+    }
+    const size_t item_bytes = b->items.size() * sizeof(BatchItem), range_bytes = n * sizeof(int2);
+    if (item_bytes + range_bytes > b->items_cap) {
         if (b->d_items) (void)hipFree(b->d_items);
         b->d_items = nullptr;
         b->items_cap = 0;
-        if (hipMalloc(&b->d_items, items.size() * sizeof(BatchItem)) != hipSuccess)
+        if (hipMalloc(&b->d_items, item_bytes + range_bytes) != hipSuccess)
             return fail(LBM_ERR_HIP, "hipMalloc(batch items) failed");
-        b->items_cap = (int)items.size();
+        b->items_cap = item_bytes + range_bytes;
     }
-    if (hipMemcpyAsync(b->d_items, items.data(), items.size() * sizeof(BatchItem), hipMemcpyHostToDevice,
-                       b->stream) != hipSuccess)
+    if (hipMemcpyAsync(b->d_items, b->items.data(), item_bytes, hipMemcpyHostToDevice, b->stream) != hipSuccess ||
+        hipMemcpyAsync(b->d_items + item_bytes, b->ranges.data(), range_bytes, hipMemcpyHostToDevice, b->stream) !=
+            hipSuccess)
         return fail(LBM_ERR_HIP, "batch item upload failed");
-    b->total = (int)items.size();
-    b->grid = grid_for_tile(b->tile, b->total, b->grid_limit);
+    b->total = (int)b->items.size();
+    b->grid = n;
     return LBM_OK;
 }
 
@@ -344,7 +406,7 @@ int rebuild(lbm_batch* b) {
         for (int f = 0; f < 6; ++f)
             if (s->cfg.walls[f].qbc != LBM_Q_PERIODIC || s->cfg.walls[f].ubc != LBM_U_PERIODIC) d.periodic = 0;
         d.tile_begin = begin;
-        begin += tiles_of(b, (int)i, d.ntx, d.nty, d.nzc);
+        begin += tiles_of(b, (int)i, d);
         d.pull = s->pulled;
         d.aux_always = s->moving ? 1 : 0;
         d.walls = (!d.periodic && kBatchTiles[b->tile].kind == 1 && p2_walls_ok(d.bc)) ? 1 : 0;
@@ -390,8 +452,9 @@ void launch_step(lbm_batch* b, int aux) {
     const int n = (int)b->sims.size();
     with_batch_tile(b->tile, [&](auto t) {
         using T = decltype(t);
-        launch_batch<T::kind, T::tx, T::ty, T::zc>(b->d_desc, n, b->total, b->d_items, b->parity, aux, b->grid,
-                                                   b->d_queue, b->stream);
+        launch_batch<T::kind, T::tx, T::ty, T::zc>(b->d_desc, n, b->total, (const BatchItem*)b->d_items,
+                                                   (const int2*)(b->d_items + b->items.size() * sizeof(BatchItem)),
+                                                   b->parity, aux, b->grid, b->stream);
     });
     if (b->sf_total > 0) {
         hipLaunchKernelGGL(batch_shell_q_kernel, dim3(grid_for(b->sq_total)), dim3(kBlock), 0, b->stream, b->d_desc,
@@ -492,9 +555,6 @@ int lbm_batch_create(const lbm_config* cfgs, int32_t count, lbm_batch_handle* ou
         return bail(fail(LBM_ERR_HIP, "hipStreamCreate failed"));
     if (hipMalloc(&b->d_desc, count * sizeof(SimDesc)) != hipSuccess)
         return bail(fail(LBM_ERR_HIP, "hipMalloc(descriptors) failed"));
-    if (hipMalloc(&b->d_queue, 2 * sizeof(unsigned)) != hipSuccess ||
-        hipMemsetAsync(b->d_queue, 0, 2 * sizeof(unsigned), b->stream) != hipSuccess)
-        return bail(fail(LBM_ERR_HIP, "hipMalloc(work queue) failed"));
     if (int r = rebuild(b)) return bail(r);
     *out = b;
     return LBM_OK;
@@ -507,7 +567,6 @@ int lbm_batch_destroy(lbm_batch_handle b) {
     for (lbm_handle h : b->sims) lbm_destroy(h);
     if (b->d_desc) (void)hipFree(b->d_desc);
     if (b->d_items) (void)hipFree(b->d_items);
-    if (b->d_queue) (void)hipFree(b->d_queue);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return LBM_OK;

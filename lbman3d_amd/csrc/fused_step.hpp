@@ -124,15 +124,37 @@ __device__ __forceinline__ void gather32_row(const Fields<float>& f, const BCDes
     }
 }
 
-template <int TX, int TY>
+template <int W, int H>
 struct TileGeom {
+    static constexpr int TX = W, TY = H;
     static constexpr int NT = TX * TY;               // threads = interior columns
     static constexpr int AX = TX + 2, AY = TY + 2;   // Q-update region
     static constexpr int IX = TX + 4, IY = TY + 4;   // input region
     static constexpr int NA = AX * AY, NI = IX * IY;
     static constexpr int NR = 2 * AX + 2 * (AY - 2); // Q-update ring columns
     static constexpr int NO = 2 * IX + 2 * (IY - 2); // input outer ring columns
+    static constexpr int LI = NI, LA = NA, LR = NR;  // LDS row lengths
+    static constexpr bool kOneLoop = false;
     static_assert(NR <= NT && NO <= NT, "tile too small for its halo");
+};
+
+// The same for a tile of w x h columns known at run time, w x h = 256 with w
+// 32 or 64. The LDS rows hold the 64 x 4 tile, which has the most columns of
+// each kind.
+// Every plane of a range runs the same copy of the iteration: a third of the
+// code, which a sweep's blocks share in the instruction cache (64 mixed boxes
+// 314 -> 308 us; a single 256^3 channel is faster with its first two
+// iterations apart, 778 against 791 us), and a cell's result does not depend
+// on where its column is cut.
+struct RowGeom {
+    static constexpr bool kOneLoop = true;
+    static constexpr int NT = 256;
+    static constexpr int LI = TileGeom<64, 4>::NI, LA = TileGeom<64, 4>::NA, LR = TileGeom<64, 4>::NR;
+    static_assert(TileGeom<32, 8>::NI <= LI && TileGeom<32, 8>::NA <= LA && TileGeom<32, 8>::NR <= LR);
+    int TX, TY, AX, AY, IX, IY, NR, NO;
+    __device__ RowGeom(int w, int h)
+        : TX(w), TY(h), AX(w + 2), AY(h + 2), IX(w + 4), IY(h + 4), NR(2 * (w + 2) + 2 * h),
+          NO(2 * (w + 4) + 2 * (h + 2)) {}
 };
 
 // Border column r of a W x H rectangle (top row, bottom row, left, right).
@@ -157,7 +179,7 @@ using StageA = StageAT<float>;
 constexpr int kNumIn = 8;    // Q (5) + u (3)
 constexpr int kNumA = 13;    // Q^{n+1} (5) + Sigma (5) + Tau (3)
 
-template <int TX, int TY, typename T>
+template <typename T>
 __device__ __forceinline__ void load_column(const Fields<T>& f, int qcol, int ucol_xy, unsigned qplane,
                                             unsigned uplane, T v[kNumIn]) {
     constexpr unsigned E = sizeof(T);
@@ -216,15 +238,14 @@ __device__ __forceinline__ void stage_a(const BCDesc<T>& bc, const Phys<T>& k,
 // rounding of q_pointwise).
 // GH: 1 every face periodic (no ghosts), 0 the general ghost rules, 2 walls
 // on x and y faces only (Neumann Q; no-slip or specular velocity; z periodic).
-template <int TX, int TY, int GH, bool UPWIND>
-__device__ __forceinline__ void stage_a_lean(const BCDesc<float>& bc, const Phys<float>& k,
-                                             const float (*sIn)[TileGeom<TX, TY>::NI], int ii, int jj,
+template <int GH, bool UPWIND, typename G>
+__device__ __forceinline__ void stage_a_lean(const G& geo, const BCDesc<float>& bc, const Phys<float>& k,
+                                             const float (*sIn)[G::LI], int ii, int jj,
                                              const float zm[kNumIn], const float c[kNumIn],
                                              const float zp[kNumIn], const int qpos[3], const int upos[3],
                                              StageA& out, float fe[3]) {
-    using G = TileGeom<TX, TY>;
-    const int cc = jj * G::IX + ii;
-    const int xm = cc - 1, xp = cc + 1, ym = cc - G::IX, yp = cc + G::IX;
+    const int cc = jj * geo.IX + ii;
+    const int xm = cc - 1, xp = cc + 1, ym = cc - geo.IX, yp = cc + geo.IX;
     // Velocity gradient -> strain rate E and vorticity W.
     float g[3][3];
 #pragma unroll
@@ -470,22 +491,22 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     // pa+1 (registers); the next plane, pa + 2, is loaded one iteration ahead
     // of its use and joins the history at the start of the next iteration.
     T hin[3][kNumIn], hnext[kNumIn];
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[1]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[2]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0), uplane(z0), hnext);
+    load_column(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[1]);
+    load_column(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[2]);
+    load_column(f, qc0, uc0, qplane(z0), uplane(z0), hnext);
     if (has_ring) {
         T v[kNumIn];
-        load_column<TX, TY>(f, qcr, ucr, qplane(z0 - 2), uplane(z0 - 2), v);
+        load_column(f, qcr, ucr, qplane(z0 - 2), uplane(z0 - 2), v);
 #pragma unroll
         for (int m = 0; m < kNumIn; ++m) sRing[(z0 - 2 + 6) % 3][m][t] = v[m];
-        load_column<TX, TY>(f, qcr, ucr, qplane(z0 - 1), uplane(z0 - 1), v);
+        load_column(f, qcr, ucr, qplane(z0 - 1), uplane(z0 - 1), v);
 #pragma unroll
         for (int m = 0; m < kNumIn; ++m) sRing[(z0 - 1 + 6) % 3][m][t] = v[m];
     }
     // Ring and outer-ring inputs are loaded one plane ahead of their LDS
     // store: ring plane pa + 1 and outer plane pa arrive in iteration pa.
     T rnext[kNumIn], onext[kNumIn];
-    if (has_ring) load_column<TX, TY>(f, qcr, ucr, qplane(z0), uplane(z0), rnext);
+    if (has_ring) load_column(f, qcr, ucr, qplane(z0), uplane(z0), rnext);
     auto load_outer = [&](int z, T* v) {
         const unsigned qo = (qplane(z) + (unsigned)oqc) * E, uo = (uplane(z) + (unsigned)ouc) * E;
 #pragma unroll
@@ -516,7 +537,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
         // At pa == z1 the loaded plane is never used; clamping it to z1 + 1
         // keeps every request within one plane past the chunk.
         const int pn = min(pa + 2, z1 + 1);
-        load_column<TX, TY>(f, qc0, uc0, qplane(pn), uplane(pn), hnext);
+        load_column(f, qc0, uc0, qplane(pn), uplane(pn), hnext);
         // The pull gather of plane pb = pa - 1 reads the previous state only,
         // so it is issued here and completes under the barrier and the Q
         // update. (The moving-wall term reads rho of the own cell, which only
@@ -537,7 +558,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
                 sRing[r_p][m][t] = rnext[m];
                 sIn[m][cc] = sRing[r_c][m][t];
             }
-            if (pa < z1) load_column<TX, TY>(f, qcr, ucr, qplane(pa + 2), uplane(pa + 2), rnext);
+            if (pa < z1) load_column(f, qcr, ucr, qplane(pa + 2), uplane(pa + 2), rnext);
         }
         if (has_outer) {
             const int cc = oj * G::IX + oi;
@@ -1040,20 +1061,20 @@ fused_step_kernel_pf(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull,
 
     // Prologue: interior planes z0-2 .. z0, ring planes z0-2 .. z0, outer plane z0-1.
     float hin[3][kNumIn];
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[0]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[1]);
-    load_column<TX, TY>(f, qc0, uc0, qplane(z0), uplane(z0), hin[2]);
+    load_column(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[0]);
+    load_column(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[1]);
+    load_column(f, qc0, uc0, qplane(z0), uplane(z0), hin[2]);
     if (has_ring) {
 #pragma unroll 1
         for (int z = z0 - 2; z <= z0; ++z) {
             float v[kNumIn];
-            load_column<TX, TY>(f, qcr, ucr, qplane(z), uplane(z), v);
+            load_column(f, qcr, ucr, qplane(z), uplane(z), v);
 #pragma unroll
             for (int m = 0; m < kNumIn; ++m) sRing[z & 3][m][t] = v[m];
         }
     }
     float ov[kNumIn];
-    if (has_outer) load_column<TX, TY>(f, oqc, ouc, qplane(z0 - 1), uplane(z0 - 1), ov);
+    if (has_outer) load_column(f, oqc, ouc, qplane(z0 - 1), uplane(z0 - 1), ov);
 
     float dz_back[kNumDZ];
 #pragma unroll
@@ -1068,9 +1089,9 @@ fused_step_kernel_pf(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull,
         // At pa == z1 the loaded plane is never used; clamping it to z1 + 1
         // keeps every request within one plane past the chunk.
         const int pn = min(pa + 2, z1 + 1);
-        load_column<TX, TY>(f, qc0, uc0, qplane(pn), uplane(pn), hnext);
-        if (has_ring) load_column<TX, TY>(f, qcr, ucr, qplane(pn), uplane(pn), rnext);
-        if (has_outer) load_column<TX, TY>(f, oqc, ouc, qplane(pa + 1), uplane(pa + 1), onext);
+        load_column(f, qc0, uc0, qplane(pn), uplane(pn), hnext);
+        if (has_ring) load_column(f, qcr, ucr, qplane(pn), uplane(pn), rnext);
+        if (has_outer) load_column(f, oqc, ouc, qplane(pa + 1), uplane(pa + 1), onext);
         const unsigned cb = (unsigned)pb * plane + (unsigned)gy * nx + gx;
         if (do_b) gather32<PERIODIC>(f, bc, gx, gy, pb, cb, pull, pop);
 #pragma unroll
@@ -1094,7 +1115,7 @@ fused_step_kernel_pf(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull,
         {
             const int qpos[3] = {qx0, qy0, zq};
             const int upos[3] = {ux0, uy0, zu};
-            stage_a_lean<TX, TY, PERIODIC, UPWIND>(bc, k, sIn, ia + 1, ib + 1, hin[0], hin[1], hin[2], qpos, upos, ai, fe_cur);
+            stage_a_lean<PERIODIC, UPWIND>(G{}, bc, k, sIn, ia + 1, ib + 1, hin[0], hin[1], hin[2], qpos, upos, ai, fe_cur);
         }
         if (has_ring) {
             const int qpos[3] = {qxr, qyr, zq};
@@ -1106,7 +1127,7 @@ fused_step_kernel_pf(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull,
                 c[m] = sRing[pa & 3][m][t];
                 zp[m] = sRing[(pa + 1) & 3][m][t];
             }
-            stage_a_lean<TX, TY, PERIODIC, UPWIND>(bc, k, sIn, ra + 1, rb + 1, zm, c, zp, qpos, upos, ar, fer);
+            stage_a_lean<PERIODIC, UPWIND>(G{}, bc, k, sIn, ra + 1, rb + 1, zm, c, zp, qpos, upos, ar, fer);
         }
 
         // ---- step 3: force + collide-stream at plane pb (sA holds plane pb) ----
@@ -1227,8 +1248,8 @@ inline bool p2_walls_ok(const BCDesc<float>& bc) {
 //   after it: Q update at plane pa, then force + collide-stream at plane pa - 1.
 // A wave can run at most one iteration ahead of the slowest (the next
 // barrier), which the two LDS buffers and the four ring-input slots cover.
-// One call computes z planes [z0, z1) (0 <= z0 < z1 <= nz) of the TX x TY
-// column tile (tx, ty), with LDS buffers from the calling kernel; a kernel
+// One call computes z planes [z0, z1) (0 <= z0 < z1 <= nz) of the column
+// tile (tx, ty) of shape geo, with LDS buffers from the calling kernel; a kernel
 // that runs several tiles per block puts a barrier between them.
 //
 // WALLS: the x and y faces may be walls (Q tag periodic or Neumann, velocity
@@ -1240,29 +1261,28 @@ inline bool p2_walls_ok(const BCDesc<float>& bc) {
 // reference clamps. For a Neumann face the clamped neighbour is the ghost of
 // Q^{n+1} as well as of Sigma and Tau, so the divergence-form sets clamp as
 // a whole.
-template <int TX, int TY, bool MASKED, bool UPWIND, bool NT, bool UNCOND = false, bool WALLS = false>
-__device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<float>& bc, const Phys<float>& k,
-                                        int pull, int aux, int tx, int ty, int z0, int z1,
-                                        float (*sIn)[kNumIn][TileGeom<TX, TY>::NI],
-                                        float (*sP)[6][TileGeom<TX, TY>::NA],
-                                        float (*sRing)[kNumIn][TileGeom<TX, TY>::NR]) {
-    using G = TileGeom<TX, TY>;
+template <bool MASKED, bool UPWIND, bool NT, bool UNCOND = false, bool WALLS = false, typename G>
+__device__ __forceinline__ void p2_range(const G& geo, const Fields<float>& f, const BCDesc<float>& bc,
+                                        const Phys<float>& k, int pull, int aux, int tx, int ty, int z0, int z1,
+                                        float (*sIn)[kNumIn][G::LI],
+                                        float (*sP)[6][G::LA],
+                                        float (*sRing)[kNumIn][G::LR]) {
     const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
-    const int x0 = tx * TX, y0 = ty * TY;
+    const int x0 = tx * geo.TX, y0 = ty * geo.TY;
     const unsigned plane = (unsigned)nx * ny;
 
     const int t = threadIdx.x;
-    const int ia = t % TX + 1, ib = t / TX + 1;
-    const int acell = ib * G::AX + ia;
+    const int ia = t % geo.TX + 1, ib = t / geo.TX + 1;
+    const int acell = ib * geo.AX + ia;
     const int gx = x0 + ia - 1, gy = y0 + ib - 1;
     const bool active = gx < nx && gy < ny;
-    const bool has_ring = t < G::NR;
+    const bool has_ring = t < geo.NR;
     int ra = 0, rb = 0;
-    if (has_ring) ring_col(t, G::AX, G::AY, ra, rb);
-    const int orank = t - (G::NT - G::NO);
+    if (has_ring) ring_col(t, geo.AX, geo.AY, ra, rb);
+    const int orank = t - (G::NT - geo.NO);
     const bool has_outer = orank >= 0;
     int oi = 0, oj = 0;
-    if (has_outer) ring_col(orank, G::IX, G::IY, oi, oj);
+    if (has_outer) ring_col(orank, geo.IX, geo.IY, oi, oj);
 
     // Periodic flags of the x and y faces (all periodic unless WALLS; Q and
     // velocity agree, see p2_walls_ok).
@@ -1280,10 +1300,10 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
     if (has_outer) oc = map_col(y0 - 2 + oj, ny, plo[1], phi[1]) * nx + map_col(x0 - 2 + oi, nx, plo[0], phi[0]);
     const int c0 = qy0 * nx + qx0, cr = qyr * nx + qxr;
     auto zplane = [&](int z) { return (unsigned)map_coord(z, nz, true, true) * plane; };
-    const int cc_int = (ib + 1) * G::IX + ia + 1;
-    const int cc_ring = (rb + 1) * G::IX + ra + 1;
-    const int cc_out = oj * G::IX + oi;
-    const int rcell = rb * G::AX + ra;
+    const int cc_int = (ib + 1) * geo.IX + ia + 1;
+    const int cc_ring = (rb + 1) * geo.IX + ra + 1;
+    const int cc_out = oj * geo.IX + oi;
+    const int rcell = rb * geo.AX + ra;
     const int qpos_i[3] = {qx0, qy0, 0}, qpos_r[3] = {qxr, qyr, 0};
     // In-plane parts of the periodic pull sources (x - cx, y - cy) of this
     // column, [cy + 1][cx + 1]: each plane's gather adds the plane offset of
@@ -1299,7 +1319,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
     }
     // Force-stage x and y neighbours in the set arrays: the cell itself where
     // a face clamps (Neumann).
-    int lxm = acell - 1, lxp = acell + 1, lym = acell - G::AX, lyp = acell + G::AX;
+    int lxm = acell - 1, lxp = acell + 1, lym = acell - geo.AX, lyp = acell + geo.AX;
     // Slot-table rows of the 16 x, y classes (no z bits; see
     // BCDesc::slots_xy), two entries per word, in LDS; the class of this
     // column; and
@@ -1331,20 +1351,20 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
     // z0-1 (LDS) and z0 (registers, stored in the first iteration), outer
     // plane z0-1.
     float hin[3][kNumIn], rcur[kNumIn], ov[kNumIn];
-    load_column<TX, TY>(f, c0, c0, zplane(z0 - 2), zplane(z0 - 2), hin[0]);
-    load_column<TX, TY>(f, c0, c0, zplane(z0 - 1), zplane(z0 - 1), hin[1]);
-    load_column<TX, TY>(f, c0, c0, zplane(z0), zplane(z0), hin[2]);
+    load_column(f, c0, c0, zplane(z0 - 2), zplane(z0 - 2), hin[0]);
+    load_column(f, c0, c0, zplane(z0 - 1), zplane(z0 - 1), hin[1]);
+    load_column(f, c0, c0, zplane(z0), zplane(z0), hin[2]);
     if (has_ring) {
 #pragma unroll 1
         for (int z = z0 - 2; z <= z0 - 1; ++z) {
             float v[kNumIn];
-            load_column<TX, TY>(f, cr, cr, zplane(z), zplane(z), v);
+            load_column(f, cr, cr, zplane(z), zplane(z), v);
 #pragma unroll
             for (int m = 0; m < kNumIn; ++m) sRing[z & 3][m][t] = v[m];
         }
-        load_column<TX, TY>(f, cr, cr, zplane(z0), zplane(z0), rcur);
+        load_column(f, cr, cr, zplane(z0), zplane(z0), rcur);
     }
-    if (has_outer) load_column<TX, TY>(f, oc, oc, zplane(z0 - 1), zplane(z0 - 1), ov);
+    if (has_outer) load_column(f, oc, oc, zplane(z0 - 1), zplane(z0 - 1), ov);
 
     // Carried across iterations (interior column): sets of plane pa - 1 to
     // publish, z sets of planes pa - 2 and pa - 1, Q^{n+1} and Ericksen force
@@ -1376,14 +1396,14 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
         float hnext[kNumIn], rnext[kNumIn], onext[kNumIn], pop[kQ];
         const int pn = min(pa + 2, z1 + 1);   // unused at pa == z1, as in fused_step_kernel_pf
         const unsigned cb = (unsigned)pb * plane + (unsigned)gy * nx + gx;
-        load_column<TX, TY>(f, c0, c0, zplane(pn), zplane(pn), hnext);
+        load_column(f, c0, c0, zplane(pn), zplane(pn), hnext);
         if (UNCOND) {
             const int rc = has_ring ? cr : c0, ocol = has_outer ? oc : c0;
-            load_column<TX, TY>(f, rc, rc, zplane(pn), zplane(pn), rnext);
-            load_column<TX, TY>(f, ocol, ocol, zplane(pa + 1), zplane(pa + 1), onext);
+            load_column(f, rc, rc, zplane(pn), zplane(pn), rnext);
+            load_column(f, ocol, ocol, zplane(pa + 1), zplane(pa + 1), onext);
         } else {
-            if (has_ring) load_column<TX, TY>(f, cr, cr, zplane(pn), zplane(pn), rnext);
-            if (has_outer) load_column<TX, TY>(f, oc, oc, zplane(pa + 1), zplane(pa + 1), onext);
+            if (has_ring) load_column(f, cr, cr, zplane(pn), zplane(pn), rnext);
+            if (has_outer) load_column(f, oc, oc, zplane(pa + 1), zplane(pa + 1), onext);
         }
         if (do_b) {
             if constexpr (WALLS) {
@@ -1428,7 +1448,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
         float fe_new[3], z_new[3], pxy_new[6];
         {
             const int qpos[3] = {qpos_i[0], qpos_i[1], zq};
-            stage_a_lean<TX, TY, WALLS ? 2 : 1, UPWIND>(bc, k, sIn[bi], ia + 1, ib + 1, hin[0], hin[1], hin[2], qpos,
+            stage_a_lean<WALLS ? 2 : 1, UPWIND>(geo, bc, k, sIn[bi], ia + 1, ib + 1, hin[0], hin[1], hin[2], qpos,
                                                         qpos, ai, fe_new);
             p_sets(k.alpha, ai.qn, ai.sg, ai.ta, pxy_new, z_new);
         }
@@ -1443,7 +1463,7 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
                 zp[m] = sRing[(pa + 1) & 3][m][t];
             }
             StageA ar;
-            stage_a_lean<TX, TY, WALLS ? 2 : 1, UPWIND>(bc, k, sIn[bi], ra + 1, rb + 1, zm, c, zp, qpos, qpos, ar, fer);
+            stage_a_lean<WALLS ? 2 : 1, UPWIND>(geo, bc, k, sIn[bi], ra + 1, rb + 1, zm, c, zp, qpos, qpos, ar, fer);
             p_sets(k.alpha, ar.qn, ar.sg, ar.ta, pr_new, zr);
         }
 
@@ -1454,8 +1474,8 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
             if (k.force_full) {
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    const float dx = P[a * G::NA + lxp] - P[a * G::NA + lxm];
-                    const float dy = P[(3 + a) * G::NA + lyp] - P[(3 + a) * G::NA + lym];
+                    const float dx = P[a * G::LA + lxp] - P[a * G::LA + lxm];
+                    const float dy = P[(3 + a) * G::LA + lyp] - P[(3 + a) * G::LA + lym];
                     const float dz = z_new[a] - zm2[a];
                     F[a] = fe_prev[a] + (0.5f * ((dx + dy) + dz) - k.mu * hin[0][5 + a]);
                 }
@@ -1509,9 +1529,13 @@ __device__ __forceinline__ void p2_range(const Fields<float>& f, const BCDesc<fl
             for (int m = 0; m < kNumIn; ++m) ov[m] = onext[m];
         }
     };
-    iteration(z0 - 1, std::false_type{});
-    iteration(z0, std::false_type{});
-    for (int pa = z0 + 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
+    if constexpr (G::kOneLoop) {
+        for (int pa = z0 - 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
+    } else {
+        iteration(z0 - 1, std::false_type{});
+        iteration(z0, std::false_type{});
+        for (int pa = z0 + 1; pa <= z1; ++pa) iteration(pa, std::true_type{});
+    }
 }
 
 // Chunk tz of ZC planes of the column tile (tx, ty).
@@ -1522,8 +1546,8 @@ __device__ __forceinline__ void p2_tile(const Fields<float>& f, const BCDesc<flo
                                        float (*sP)[6][TileGeom<TX, TY>::NA],
                                        float (*sRing)[kNumIn][TileGeom<TX, TY>::NR]) {
     const int z0 = tz * ZC;
-    p2_range<TX, TY, MASKED, UPWIND, NT, UNCOND, WALLS>(f, bc, k, pull, aux, tx, ty, z0, min(z0 + ZC, bc.n[2]), sIn,
-                                                       sP, sRing);
+    p2_range<MASKED, UPWIND, NT, UNCOND, WALLS>(TileGeom<TX, TY>{}, f, bc, k, pull, aux, tx, ty, z0,
+                                                min(z0 + ZC, bc.n[2]), sIn, sP, sRing);
 }
 
 template <int TX, int TY, int ZC, bool MASKED, int WPE, bool UPWIND, bool NT, bool ZSLOW, bool UNCOND = false,
