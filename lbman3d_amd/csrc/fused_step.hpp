@@ -32,14 +32,11 @@
 
 namespace lbm {
 
-__device__ __forceinline__ void sto_nt(double* base, unsigned boff, double v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<double*>(reinterpret_cast<char*>(base) + boff));
-}
 // Store with an optional non-temporal hint (streaming output read back only
 // next step, so it need not displace the halo rows held in L2).
-template <bool NT>
-__device__ __forceinline__ void sto_hint(float* base, unsigned boff, float v) {
-    float* p = reinterpret_cast<float*>(reinterpret_cast<char*>(base) + boff);
+template <bool NT, typename T>
+__device__ __forceinline__ void sto_hint(T* base, unsigned boff, T v) {
+    T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(base) + boff);
     if (NT) __builtin_nontemporal_store(v, p);
     else *p = v;
 }
@@ -735,9 +732,9 @@ fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int n
 // 256^3 on 32x8 tiles: 2.14 ms for the first pipeline's best tile, 1.56 ms
 // here; 128^3 0.244 -> 0.213 ms. What it must not do is spill: with every halo
 // load issued unconditionally (14 registers more) the prefetched values went
-// to scratch as they arrived and the step took 2.05 ms. Non-temporal stores
-// (the outputs leave the L2 before they are read): 2.12 -> 2.05 ms then.
-template <int TX, int TY, bool MASKED, int ADV>
+// to scratch as they arrived and the step took 2.05 ms. NT: non-temporal
+// stores (see launch_tile64).
+template <int TX, int TY, bool MASKED, int ADV, bool NT>
 __global__ void __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fused64_kernel(Fields<double> f, BCDesc<double> bc, Phys<double> k, int pull, int aux, int ntx, int nty, int nzc,
                int zc) {
@@ -891,11 +888,11 @@ fused64_kernel(Fields<double> f, BCDesc<double> bc, Phys<double> k, int pull, in
             T rho, u[3];
             collide_plain(k, pop, F, rho, u);
 #pragma unroll
-            for (int j = 0; j < kQ; ++j) sto_nt(f.gn, j * vsb + cb, pop[j]);
+            for (int j = 0; j < kQ; ++j) sto_hint<NT>(f.gn, j * vsb + cb, pop[j]);
 #pragma unroll
-            for (int m = 0; m < 3; ++m) sto_nt(f.un[m], cb, u[m]);
+            for (int m = 0; m < 3; ++m) sto_hint<NT>(f.un[m], cb, u[m]);
 #pragma unroll
-            for (int m = 0; m < 5; ++m) sto_nt(f.qn[m], cb, sA[m][acell]);
+            for (int m = 0; m < 5; ++m) sto_hint<NT>(f.qn[m], cb, sA[m][acell]);
             if (aux && (!MASKED || cell_mask(bc, 1, gx, gy).writes(pb))) {
                 sto(f.rho, cb, rho);
 #pragma unroll

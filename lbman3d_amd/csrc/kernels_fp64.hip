@@ -55,13 +55,24 @@ static void launch_tile64(const Fields<double>& f, const BCDesc<double>& bc, con
     bool walls = false;
     for (int face = 0; face < 6; ++face)
         walls = walls || bc.qkind[face] != QB_PERIODIC || bc.ukind[face] != UB_PERIODIC;
-    auto go = [&](auto masked, auto adv) {
-        hipLaunchKernelGGL((fused64_kernel<TX, TY, decltype(masked)::value, decltype(adv)::value>), dim3(grid),
-                           dim3(TX * TY), 0, s, f, bc, k, pull, aux, ntx, nty, nzc, zc);
+    auto go = [&](auto masked, auto adv, auto nt) {
+        hipLaunchKernelGGL((fused64_kernel<TX, TY, decltype(masked)::value, decltype(adv)::value, decltype(nt)::value>),
+                           dim3(grid), dim3(TX * TY), 0, s, f, bc, k, pull, aux, ntx, nty, nzc, zc);
+    };
+    // Rows of whole 64-byte pieces are stored past the L2 (they leave it before
+    // they are read again): 32x8 tiles at 128, 136, 152 and 168 x 128 x 128
+    // take 200, 257, 266 and 303 us so and 207, 262, 274 and 312 us with plain
+    // stores. In other rows a tile begins inside a piece, which then reaches
+    // memory in two parts; plain stores let the L2 put it together: 130, 131,
+    // 140 and 150 x 128 x 128 306, 321, 291 and 326 -> 270, 273, 271 and 283 us.
+    const bool nt = bc.n[0] % 8 == 0;
+    auto with_nt = [&](auto masked, auto adv) {
+        if (nt) go(masked, adv, std::true_type{});
+        else go(masked, adv, std::false_type{});
     };
     auto with_adv = [&](auto masked) {
-        if (k.advection) go(masked, std::integral_constant<int, 1>{});
-        else go(masked, std::integral_constant<int, 0>{});
+        if (k.advection) with_nt(masked, std::integral_constant<int, 1>{});
+        else with_nt(masked, std::integral_constant<int, 0>{});
     };
     if (walls) {
         with_adv(std::true_type{});
