@@ -278,7 +278,7 @@ conv_fwd_kernel(ConvIO io, const bf16x8* __restrict__ wpk, const float* __restri
 // (dy = dz = 0) also multiplies an all-ones A fragment into its dOut
 // fragments: the bias gradient. A block accumulates over its tiles in
 // registers and writes one partial [27 CIN + 1][cout] (weights, then the bias
-// row); wgrad_reduce_kernel adds the partials of all blocks.
+// row); update_kernel adds the partials of all blocks.
 constexpr int kWgTX = 16, kWgTY = 4, kWgTZ = 2;
 constexpr int kWgRL = 24;                                     // bf16 per LDS row (x0 - 2 .. x0 + 17, padded)
 constexpr int kWgHY = kWgTY + 2, kWgHZ = kWgTZ + 2;
