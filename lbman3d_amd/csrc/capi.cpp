@@ -34,8 +34,12 @@ using namespace lbm;
 namespace lbm {
 thread_local std::string g_last_error;
 
+// A HIP error is reported here and so taken from the thread's last error, or
+// the launch check of the thread's next call would report it again (a grid
+// that does not fit, then a smaller one).
 int fail(int code, const std::string& msg) {
     g_last_error = msg;
+    if (code == LBM_ERR_HIP) (void)hipGetLastError();
     return code;
 }
 }  // namespace lbm

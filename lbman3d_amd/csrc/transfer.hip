@@ -128,8 +128,10 @@ int for_pieces(hipStream_t stream, long cells, int arrays, long most, F&& work) 
             if (e != hipSuccess) error = (int)e;
             return e == hipSuccess;
         };
-        for (long i; !error && (i = next++) < pieces;)
+        for (long i; !error && (i = next++) < pieces;) {
+            (void)hipGetLastError();   // what an earlier call left is not this piece's error
             work(i * piece, std::min(piece, cells - i * piece), buffer, finish);
+        }
         if (error) (void)hipStreamSynchronize(stream);   // nothing may still use the buffer
         if (done) (void)hipEventDestroy(done);
         stage_release(buffer);
@@ -282,6 +284,7 @@ int put_state_typed(hipStream_t stream, const Fields<T>& f, double rho0, const d
 template <typename T>
 int rest_typed(hipStream_t stream, const Fields<T>& f, double rho0, long cells) {
     constexpr long kPiece = 1 << 28;   // cells per launch
+    (void)hipGetLastError();           // what an earlier call left is not this one's error
     for (long c0 = 0; c0 < cells; c0 += kPiece) {
         const long n = std::min(kPiece, cells - c0);
         hipLaunchKernelGGL(state_kernel<T>, piece_grid(n, 1), dim3(256), 0, stream, f, rho0,
