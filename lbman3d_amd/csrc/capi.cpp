@@ -533,8 +533,11 @@ int lbm_create(const lbm_config* cfg, lbm_handle* out) {
     int ndev = 0;
     HIPCHK(hipGetDeviceCount(&ndev));
     if (ndev < 1) return fail(LBM_ERR_HIP, "no HIP device");
+    int device = 0;
+    HIPCHK(hipGetDevice(&device));
 
     lbm_solver* s = new lbm_solver();
+    s->device = device;
     staging_open();
     s->cfg = *cfg;
     s->V = (long)cfg->nx * cfg->ny * cfg->nz;
@@ -695,6 +698,7 @@ int lbm_download_force(lbm_handle s, double* fx, double* fy, double* fz) {
 
 int lbm_download_populations(lbm_handle s, double* f) {
     if (!s || !f) return fail(LBM_ERR_INVALID, "null argument");
+    const OnDevice on(s);
     void* tmp = nullptr;
     HIPCHK(hipMalloc(&tmp, kQ * s->vs * s->esize()));
     auto release = scope_exit([&] { (void)hipFree(tmp); });
@@ -832,6 +836,7 @@ int lbm_order_director_noalloc(lbm_handle s, double* order, double* director) {
 
 int lbm_time_steps(lbm_handle s, int32_t n, double* ms) {
     if (!s || !ms || n < 1) return fail(LBM_ERR_INVALID, "bad argument");
+    const OnDevice on(s);
     ensure_tuned(s);
     hipEvent_t a = nullptr, b = nullptr;
     auto release = scope_exit([&] {
@@ -1017,6 +1022,7 @@ extern "C" {
 int lbm_autotune(lbm_handle s, int32_t n, double* ms_out, int32_t max, int32_t* count) {
     if (!s || n < 1) return fail(LBM_ERR_INVALID, "bad argument");
     if (count) *count = 0;
+    const OnDevice on(s);
     std::vector<int> cands = {1};
     if (s->fp64) {
         if (s->fused64_ok)

@@ -18,6 +18,7 @@ struct lbm_solver {
     lbm_config cfg{};
     long V = 0, vs = 0;
     bool fp64 = true;
+    int device = 0;        // the device that was current at creation
     hipStream_t stream = nullptr;
     std::vector<void*> allocs;
     Fields<double> d64{};
@@ -42,6 +43,24 @@ struct lbm_solver {
 };
 
 namespace lbm {
+// The handle's device is the thread's current one while this lives: events and
+// allocations of a call belong to it, whatever the caller has current.
+class OnDevice {
+public:
+    explicit OnDevice(const lbm_solver* s) {
+        if (hipGetDevice(&before_) != hipSuccess || before_ == s->device || hipSetDevice(s->device) != hipSuccess)
+            before_ = -1;
+    }
+    ~OnDevice() {
+        if (before_ >= 0) (void)hipSetDevice(before_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+private:
+    int before_ = -1;   // to be restored, or -1
+};
+
 // One full step of a handle (capi.cpp); `last` materialises rho and F.
 int run_step(lbm_solver* s, bool last, KernelRecorder* rec);
 // Tunes the automatic FP32 schedule on first use (capi.cpp).

@@ -101,9 +101,13 @@ int host_threads(size_t bytes) {
 
 // work(first cell, cells, buffer, finish) for pieces of at most `most` cells;
 // finish() waits for what the piece has put on the stream. `arrays` host values
-// belong to a cell.
+// belong to a cell. The caller's thread and the helpers work on the handle's
+// device: an event can be recorded on a stream of its own device only.
 template <typename F>
-int for_pieces(hipStream_t stream, long cells, int arrays, long most, F&& work) {
+int for_pieces(const lbm_solver* s, int arrays, long most, F&& work) {
+    const OnDevice on(s);
+    const hipStream_t stream = s->stream;
+    const long cells = s->V;
     const long pieces = (cells + most - 1) / most;
     const long piece = std::min(most, ((cells + pieces - 1) / pieces + 63) / 64 * 64);
     const int threads = (int)std::min<long>(host_threads((size_t)cells * arrays * sizeof(double)), pieces);
@@ -113,10 +117,8 @@ int for_pieces(hipStream_t stream, long cells, int arrays, long most, F&& work) 
     // in each of them would hold that many CPUs.
     if (threads > 1 && hipStreamSynchronize(stream) != hipSuccess)
         return fail(LBM_ERR_HIP, "field transfer: synchronize failed");
-    int dev = 0;
-    (void)hipGetDevice(&dev);
     auto run = [&](bool own) {
-        if (own && hipSetDevice(dev) != hipSuccess) error = (int)hipErrorInvalidDevice;
+        if (own && hipSetDevice(s->device) != hipSuccess) error = (int)hipErrorInvalidDevice;
         void* buffer = stage_acquire();
         hipEvent_t done = nullptr;
         if (!buffer || hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess)
@@ -216,11 +218,11 @@ state_kernel(Fields<T> f, double rho0, double base, unsigned has, bool rest, lon
 dim3 piece_grid(long n, int arrays) { return dim3((unsigned)((n + 255) / 256), (unsigned)arrays); }
 
 template <typename T>
-int fetch_typed(hipStream_t stream, const FetchItem* items, int count, long cells) {
+int fetch_typed(const lbm_solver* s, const FetchItem* items, int count) {
     Arrays<const T> src{};
     for (int k = 0; k < count; ++k) src.p[k] = (const T*)items[k].dev;
-    return for_pieces(stream, cells, count, piece_cells(count, sizeof(T)), [&](long c0, long n, void* buffer, auto finish) {
-        hipLaunchKernelGGL(pack_kernel<T>, piece_grid(n, count), dim3(256), 0, stream, src, c0, (int)n, (T*)buffer);
+    return for_pieces(s, count, piece_cells(count, sizeof(T)), [&](long c0, long n, void* buffer, auto finish) {
+        hipLaunchKernelGGL(pack_kernel<T>, piece_grid(n, count), dim3(256), 0, s->stream, src, c0, (int)n, (T*)buffer);
         if (!finish()) return;
         const T* in = (const T*)buffer;
         for (int k = 0; k < count; ++k, in += n) {
@@ -236,25 +238,26 @@ int fetch_typed(hipStream_t stream, const FetchItem* items, int count, long cell
 }
 
 template <typename T>
-int put_typed(hipStream_t stream, const PutItem* items, int count, long cells) {
+int put_typed(const lbm_solver* s, const PutItem* items, int count) {
     Arrays<T> dst{};
     Bases base{};
     for (int k = 0; k < count; ++k) {
         dst.p[k] = (T*)items[k].dev;
         base.v[k] = items[k].base;
     }
-    return for_pieces(stream, cells, count, piece_cells(count, sizeof(double)), [&](long c0, long n, void* buffer, auto finish) {
+    return for_pieces(s, count, piece_cells(count, sizeof(double)), [&](long c0, long n, void* buffer, auto finish) {
         for (int k = 0; k < count; ++k)
             std::memcpy((double*)buffer + k * n, items[k].host + c0, n * sizeof(double));
-        hipLaunchKernelGGL(unpack_kernel<T>, piece_grid(n, count), dim3(256), 0, stream, dst, base, c0, (int)n,
+        hipLaunchKernelGGL(unpack_kernel<T>, piece_grid(n, count), dim3(256), 0, s->stream, dst, base, c0, (int)n,
                            (const double*)buffer);
         (void)finish();
     });
 }
 
 template <typename T>
-int put_state_typed(hipStream_t stream, const Fields<T>& f, double rho0, const double* rho, const double* const u[3],
-                    const double* q, long cells) {
+int put_state_typed(const lbm_solver* s, const Fields<T>& f, const double* rho, const double* const u[3],
+                    const double* q) {
+    const double rho0 = s->cfg.p.density;
     const double base = sizeof(T) == 4 ? rho0 : 0.0;
     const double* src[9];
     unsigned has = 0;
@@ -270,12 +273,12 @@ int put_state_typed(hipStream_t stream, const Fields<T>& f, double rho0, const d
         }
     if (q) {
         has |= 16;
-        for (int m = 0; m < 5; ++m) src[count++] = q + m * cells;
+        for (int m = 0; m < 5; ++m) src[count++] = q + m * s->V;
     }
-    return for_pieces(stream, cells, count, piece_cells(std::max(count, 1), sizeof(double)),
+    return for_pieces(s, count, piece_cells(std::max(count, 1), sizeof(double)),
                       [&](long c0, long n, void* buffer, auto finish) {
         for (int k = 0; k < count; ++k) std::memcpy((double*)buffer + k * n, src[k] + c0, n * sizeof(double));
-        hipLaunchKernelGGL(state_kernel<T>, piece_grid(n, 1), dim3(256), 0, stream, f, rho0, base, has, false, c0,
+        hipLaunchKernelGGL(state_kernel<T>, piece_grid(n, 1), dim3(256), 0, s->stream, f, rho0, base, has, false, c0,
                            (int)n, (const double*)buffer);
         (void)finish();
     });
@@ -299,17 +302,14 @@ int rest_typed(hipStream_t stream, const Fields<T>& f, double rho0, long cells) 
 
 int fetch_fields(lbm_solver* s, const FetchItem* items, int count) {
     if (count == 0) return LBM_OK;
-    return s->fp64 ? fetch_typed<double>(s->stream, items, count, s->V)
-                   : fetch_typed<float>(s->stream, items, count, s->V);
+    return s->fp64 ? fetch_typed<double>(s, items, count) : fetch_typed<float>(s, items, count);
 }
 int put_fields(lbm_solver* s, const PutItem* items, int count) {
     if (count == 0) return LBM_OK;
-    return s->fp64 ? put_typed<double>(s->stream, items, count, s->V) : put_typed<float>(s->stream, items, count, s->V);
+    return s->fp64 ? put_typed<double>(s, items, count) : put_typed<float>(s, items, count);
 }
 int put_state(lbm_solver* s, const double* rho, const double* const u[3], const double* q) {
-    const double rho0 = s->cfg.p.density;
-    return s->fp64 ? put_state_typed(s->stream, s->d64, rho0, rho, u, q, s->V)
-                   : put_state_typed(s->stream, s->d32, rho0, rho, u, q, s->V);
+    return s->fp64 ? put_state_typed(s, s->d64, rho, u, q) : put_state_typed(s, s->d32, rho, u, q);
 }
 int put_rest(lbm_solver* s) {
     const double rho0 = s->cfg.p.density;
@@ -317,7 +317,7 @@ int put_rest(lbm_solver* s) {
 }
 
 int fetch_order_director(lbm_solver* s, double* order, double* director) {
-    return for_pieces(s->stream, s->V, 4, piece_cells(4, sizeof(double)), [&](long c0, long n, void* buffer, auto finish) {
+    return for_pieces(s, 4, piece_cells(4, sizeof(double)), [&](long c0, long n, void* buffer, auto finish) {
         double* o = (double*)buffer;
         if (s->fp64) launch_order_director(s->d64, c0, n, o, o + n, s->stream);
         else launch_order_director(s->d32, c0, n, o, o + n, s->stream);

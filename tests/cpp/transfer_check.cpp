@@ -147,6 +147,7 @@ void expect(bool ok, const char* what) {
 void round_trip(int device, long cells, int count) {
     ihipStream_t stream{device};
     lbm_solver s;
+    s.device = device;
     s.stream = &stream;
     s.V = cells;
     std::vector<double> host(cells * count), dev(cells * count, -1.0), back(cells * count, -2.0);
@@ -181,6 +182,11 @@ int main(int argc, char** argv) {
             t_last = hipErrorOutOfMemory;
             round_trip(0, cells, 9);
         }
+    } else if (what == "other-device") {
+        // the handle's device is not the caller's current one
+        round_trip(1, kSmall, 9);
+        round_trip(1, kLarge, 9);
+        expect(t_device == 0, "the caller's device is current again");
     } else {
         std::printf("unknown scenario\n");
         return 2;
