@@ -117,12 +117,17 @@ int for_pieces(const lbm_solver* s, int arrays, long most, F&& work) {
     // in each of them would hold that many CPUs.
     if (threads > 1 && hipStreamSynchronize(stream) != hipSuccess)
         return fail(LBM_ERR_HIP, "field transfer: synchronize failed");
-    auto run = [&](bool own) {
-        if (own && hipSetDevice(s->device) != hipSuccess) error = (int)hipErrorInvalidDevice;
+    // A helper that cannot have the device, a buffer or an event leaves the
+    // pieces to the others; only the caller's own thread must have them.
+    auto run = [&](bool helper) {
+        if (helper && hipSetDevice(s->device) != hipSuccess) return;
         void* buffer = stage_acquire();
         hipEvent_t done = nullptr;
-        if (!buffer || hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess)
-            error = (int)hipErrorOutOfMemory;
+        if (!buffer || hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) {
+            stage_release(buffer);
+            if (!helper) error = (int)hipErrorOutOfMemory;
+            return;
+        }
         auto finish = [&]() -> bool {
             hipError_t e = hipGetLastError();
             if (e == hipSuccess) e = hipEventRecord(done, stream);
@@ -135,7 +140,7 @@ int for_pieces(const lbm_solver* s, int arrays, long most, F&& work) {
             work(i * piece, std::min(piece, cells - i * piece), buffer, finish);
         }
         if (error) (void)hipStreamSynchronize(stream);   // nothing may still use the buffer
-        if (done) (void)hipEventDestroy(done);
+        (void)hipEventDestroy(done);
         stage_release(buffer);
     };
     std::vector<std::thread> others;

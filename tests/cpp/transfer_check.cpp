@@ -28,6 +28,7 @@ namespace {
 thread_local int t_device = 0;
 thread_local hipError_t t_last = hipSuccess;
 thread_local bool t_helper = true;   // main() clears it
+std::atomic<int> g_refuse_helpers{0};   // 1: buffers, 2: events, 3: devices
 std::atomic<int> g_helpers{0}, g_launches{0};
 
 hipError_t status(hipError_t e) {
@@ -71,10 +72,12 @@ hipError_t hipGetDevice(int* d) {
 }
 hipError_t hipSetDevice(int d) {
     if (t_helper) ++g_helpers;
+    if (t_helper && g_refuse_helpers == 3) return status(hipErrorInvalidDevice);
     t_device = d;
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (t_helper && g_refuse_helpers == 1) return status(hipErrorOutOfMemory);
     *p = std::malloc(n);
     return hipSuccess;
 }
@@ -83,6 +86,7 @@ hipError_t hipHostFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    if (t_helper && g_refuse_helpers == 2) return status(hipErrorOutOfMemory);
     *e = new ihipEvent_t{t_device};
     return hipSuccess;
 }
@@ -187,6 +191,11 @@ int main(int argc, char** argv) {
         round_trip(1, kSmall, 9);
         round_trip(1, kLarge, 9);
         expect(t_device == 0, "the caller's device is current again");
+    } else if (what == "helper-buffer" || what == "helper-event" || what == "helper-device") {
+        // helpers without a buffer, event or device leave the work to the caller
+        g_refuse_helpers = what == "helper-buffer" ? 1 : (what == "helper-event" ? 2 : 3);
+        round_trip(0, kLarge, 9);
+        expect(g_helpers > 0, "helper threads were started");
     } else {
         std::printf("unknown scenario\n");
         return 2;
