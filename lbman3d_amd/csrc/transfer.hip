@@ -39,19 +39,17 @@ constexpr int kMaxThreads = 8;
 
 // ---- pinned buffers ------------------------------------------------------------
 // Shared by every handle of the process; at most kKeep are kept, and all are
-// freed with the last handle.
+// freed with the last handle. Giving one back allocates nothing: it happens at
+// the end of a helper thread, where an exception would end the process.
 std::mutex g_mu;
-std::vector<void*> g_free;
+void* g_free[kKeep];
+size_t g_kept = 0;
 int g_users = 0;
 
 void* stage_acquire() {
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        if (!g_free.empty()) {
-            void* p = g_free.back();
-            g_free.pop_back();
-            return p;
-        }
+        if (g_kept > 0) return g_free[--g_kept];
     }
     void* p = nullptr;
     return hipHostMalloc(&p, kStageBytes, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess ? p : nullptr;
@@ -60,8 +58,8 @@ void stage_release(void* p) {
     if (!p) return;
     {
         std::lock_guard<std::mutex> lock(g_mu);
-        if (g_users > 0 && g_free.size() < kKeep) {
-            g_free.push_back(p);
+        if (g_users > 0 && g_kept < kKeep) {
+            g_free[g_kept++] = p;
             return;
         }
     }
@@ -75,13 +73,14 @@ void staging_open() {
     ++g_users;
 }
 void staging_close() {
-    std::vector<void*> gone;
+    void* gone[kKeep];
+    size_t count = 0;
     {
         std::lock_guard<std::mutex> lock(g_mu);
         if (--g_users > 0) return;
-        gone.swap(g_free);
+        while (g_kept > 0) gone[count++] = g_free[--g_kept];
     }
-    for (void* p : gone) (void)hipHostFree(p);
+    while (count > 0) (void)hipHostFree(gone[--count]);
 }
 
 namespace {

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 
 #include "../../lbman3d_amd/csrc/transfer.hip"
 
@@ -27,7 +28,9 @@ struct ihipEvent_t {
 namespace {
 thread_local int t_device = 0;
 thread_local hipError_t t_last = hipSuccess;
-thread_local bool t_helper = true;   // main() clears it
+thread_local bool t_helper = true;        // main() clears it
+thread_local bool t_no_memory = false;    // operator new throws
+std::atomic<bool> g_no_memory_after_event{false};
 std::atomic<int> g_refuse_helpers{0};   // 1: buffers, 2: events, 3: devices
 std::atomic<int> g_helpers{0}, g_launches{0};
 
@@ -65,6 +68,14 @@ bool emulate(const void* fn, dim3 grid, void** args) {
 }
 }  // namespace
 
+void* operator new(size_t n) {
+    if (t_no_memory) throw std::bad_alloc();
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 extern "C" {
 hipError_t hipGetDevice(int* d) {
     *d = t_device;
@@ -92,6 +103,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 }
 hipError_t hipEventDestroy(hipEvent_t e) {
     delete e;
+    if (g_no_memory_after_event) t_no_memory = true;
     return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
@@ -196,6 +208,22 @@ int main(int argc, char** argv) {
         g_refuse_helpers = what == "helper-buffer" ? 1 : (what == "helper-event" ? 2 : 3);
         round_trip(0, kLarge, 9);
         expect(g_helpers > 0, "helper threads were started");
+    } else if (what == "host-memory") {
+        // a transfer that ends needs no host memory
+        g_no_memory_after_event = true;
+        ihipStream_t stream{0};
+        lbm_solver s;
+        s.stream = &stream;
+        s.V = kLarge;
+        std::vector<double> host(9 * kLarge, 1.0), dev(9 * kLarge);
+        PutItem put[9];
+        for (int k = 0; k < 9; ++k) put[k] = {&dev[k * kLarge], &host[k * kLarge], 0.0};
+        staging_open();
+        const int r = put_fields(&s, put, 9);
+        t_no_memory = false;
+        g_no_memory_after_event = false;
+        expect(r == LBM_OK && dev == host, "upload");
+        staging_close();
     } else {
         std::printf("unknown scenario\n");
         return 2;

@@ -25,7 +25,7 @@ def check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["plain", "earlier-error", "other-device", "helper-buffer", "helper-event",
-                                      "helper-device"])
+                                      "helper-device", "host-memory"])
 def test_transfer(check, scenario):
     r = subprocess.run([str(check), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
