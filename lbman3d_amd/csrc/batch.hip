@@ -21,6 +21,7 @@
 #define LBM_FUSED_BODY_ONLY
 #include "step_kernels.hpp"
 #include "fused_step.hpp"
+#include "batch_split.hpp"
 #include "solver_state.hpp"
 
 #include <algorithm>
@@ -98,12 +99,6 @@ batch_step_kernel(const SimDesc* __restrict__ descs, int nsims, int total, int p
         __syncthreads();
     }
 }
-
-// One work item of the third-pipeline kernel: planes [z0, z1) of column
-// tile txy (= tx + ty * ntx) of simulation sim.
-struct BatchItem {
-    int sim, txy, z0, z1;
-};
 
 // The work list on the third pipeline: block b runs the items
 // [ranges[b].x, ranges[b].y), which the host has cut so that every block has
@@ -219,7 +214,6 @@ struct lbm_batch {
     size_t items_cap = 0;          // bytes
     std::vector<BatchItem> items;  // host copies (the upload reads them asynchronously)
     std::vector<int2> ranges;
-    std::vector<int> order;        // simulations in the order in which their columns are cut
     hipStream_t stream = nullptr;
     int total = 0;
     int sq_total = 0;      // cells of the shell Q pass (simulations with walls)
@@ -290,80 +284,34 @@ int grid_for_tile(int tile, int total, int limit) {
     return limit > 0 ? std::min(grid, limit) : grid;
 }
 
-// Items and block ranges of the third-pipeline kernel. The columns of all
-// simulations, one after another, are cut into one range per resident block
-// so that the costliest range is the cheapest possible (by bisection over
-// its cost). Costs, in eighths of a periodic plane: a piece of n planes also
-// fills the pipeline, about two planes' time, and the wall-aware form takes
-// about an eighth more per plane. Before, blocks drew chunks of 16, 32 or 64
-// planes from a queue, longest first, so a sweep with fewer chunks than a few
-// rounds of blocks waited for the last ones: 6 boxes of 24 to 64 per side 95
-// -> 40 us, 20 boxes 127 -> 97 us, 64 boxes 335 -> 308 us, 80 boxes 377 ->
-// 357 us (with the tile shapes above and one loop body).
+// Items and block ranges of the third-pipeline kernel (batch_split.hpp): one
+// range of equal cost per resident block. Before, blocks drew chunks of 16, 32
+// or 64 planes from a queue, longest first, so a sweep with fewer chunks than
+// a few rounds of blocks waited for the last ones: 6 boxes of 24 to 64 per
+// side 95 -> 40 us, 20 boxes 127 -> 97 us, 64 boxes 335 -> 308 us, 80 boxes
+// 377 -> 357 us (with the tile shapes above and one loop body).
 // Simulations of one form are neighbours in the order, so that a compute
 // unit's blocks run the same body (18 boxes of 64^3, half of them slits: 256
 // -> 240 us), and neighbouring ranges run on the same XCD (block b runs on
 // XCD b mod 8), whose L2 then holds their shared halo columns.
-constexpr int kPlane = 8, kWallPlane = 9;
-constexpr int kPieceStart = 2 * kPlane;
-constexpr int kPieceMin = 4;   // planes; 6 boxes: 2 the same, 8: 45 -> 57 us
-
-struct BatchSplit {
-    std::vector<BatchItem> items;
-    std::vector<int> first;   // first item of each range
-};
-
-// Greedy cut with every range's cost at most `bound` (or one piece).
-void cut_columns(const lbm_batch* b, int zc, int bound, BatchSplit& out) {
-    out.items.clear();
-    out.first.assign(1, 0);
-    int load = 0;
-    for (int i : b->order) {
-        const SimDesc& d = b->desc[i];
-        const int nz = d.bc.n[2];
-        const int wp = d.walls ? kWallPlane : kPlane;
-        for (int txy = 0; txy < d.ntx * d.nty; ++txy)
-            for (int z = 0; z < nz;) {
-                const int left = nz - z;
-                const int room = (bound - load - kPieceStart) / wp;
-                if (room < std::min(kPieceMin, left) && load > 0) {
-                    out.first.push_back((int)out.items.size());
-                    load = 0;
-                    continue;
-                }
-                int n = std::min({left, zc, std::max(room, kPieceMin)});
-                if (left - n == 1 && left <= zc) n = left;   // one plane more, not a piece of one
-                out.items.push_back({(int)i, txy, z, z + n});
-                load += kPieceStart + n * wp;
-                z += n;
-            }
-    }
-    out.first.push_back((int)out.items.size());
-}
-
 int build_items(lbm_batch* b) {
     const int zc = kBatchTiles[b->tile].zc;
     int planes = 0;
     for (const SimDesc& d : b->desc) planes += d.ntx * d.nty * d.bc.n[2];
     const int slots = grid_for_tile(b->tile, planes, b->grid_limit);
-    b->order.resize(b->sims.size());
-    for (size_t i = 0; i < b->order.size(); ++i) b->order[i] = (int)i;
-    auto form = [&](int i) { return 4 * (b->desc[i].tile_x > 32) + 2 * b->desc[i].walls + (b->desc[i].k.advection != 0); };
-    std::stable_sort(b->order.begin(), b->order.end(), [&](int x, int y) { return form(x) < form(y); });
-    BatchSplit split;
-    int lo = kPieceStart + kPlane * kPieceMin, hi = lo;
-    auto fits = [&](int bound) {
-        cut_columns(b, zc, bound, split);
-        return (int)split.first.size() - 1 <= slots;
-    };
-    while (!fits(hi)) hi *= 2;
-    while (lo < hi) {
-        const int mid = (lo + hi) / 2;
-        if (fits(mid)) hi = mid;
-        else lo = mid + 1;
+    std::vector<BatchColumns> sims;
+    for (size_t i = 0; i < b->desc.size(); ++i) {
+        const SimDesc& d = b->desc[i];
+        sims.push_back({(int)i, d.ntx * d.nty, d.bc.n[2], d.walls != 0});
     }
-    cut_columns(b, zc, hi, split);
-    const int n = (int)split.first.size() - 1;
+    auto form = [&](const BatchColumns& c) {
+        const SimDesc& d = b->desc[c.sim];
+        return 4 * (d.tile_x > 32) + 2 * d.walls + (d.k.advection != 0);
+    };
+    std::stable_sort(sims.begin(), sims.end(),
+                     [&](const BatchColumns& x, const BatchColumns& y) { return form(x) < form(y); });
+    BatchSplit split = split_columns(sims, zc, slots);
+    const int n = split.ranges();
     b->items = std::move(split.items);
     b->ranges.resize(n);
     for (int r = 0, q = n / 8, m = n % 8; r < n; ++r) {
