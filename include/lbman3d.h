@@ -204,8 +204,10 @@ int lbm_profile_kernels(lbm_handle h, int32_t n, double* ms_out, int32_t max,
 /* Kernel schedule. 0 = automatic (autotuned on first use), 1 = two-kernel
  * split, 2.. = a fixed fused tile shape. FP32 tiles: lbm_tile_count /
  * lbm_tile_name. FP64: fully periodic domains, and domains with walls from 2^20
- * cells on, also have fused tiles, whose results equal the two-kernel split bit
- * for bit; other domains run the two-kernel split. */
+ * cells on, also have fused tiles (schedules 2 to 8: 32x8 and 16x16 columns,
+ * first with z chunks chosen by the grid, which tuning chooses from, then with
+ * fixed ones), whose results equal the two-kernel split bit for bit; other
+ * domains accept the same numbers and run the two-kernel split. */
 int lbm_set_schedule(lbm_handle h, int32_t schedule);
 int lbm_get_schedule(lbm_handle h, int32_t* schedule);
 int lbm_tile_count(void);
@@ -213,8 +215,8 @@ int lbm_tile_name(int32_t schedule, char* buf, size_t len);
 /* Name of a schedule of this handle's precision ("auto:...", "two-kernel",
  * "fused:..."). */
 int lbm_schedule_name(lbm_handle h, int32_t schedule, char* buf, size_t len);
-/* Time every schedule of the handle's precision for n steps from a snapshot
- * of the state (restored after each trial), then the three fastest again for
+/* Time every schedule of the handle's precision (in FP64 of the tiles those
+ * with z chunks chosen by the grid) for n steps from a snapshot of the state (restored after each trial), then the three fastest again for
  * 8n steps each, and keep the fastest of those for the automatic schedule;
  * results per schedule (1, 2, ...) in ms_out[count] (ms per step, the
  * longer trial's for the three). */

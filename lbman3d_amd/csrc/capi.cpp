@@ -1026,7 +1026,7 @@ int lbm_autotune(lbm_handle s, int32_t n, double* ms_out, int32_t max, int32_t* 
     std::vector<int> cands = {1};
     if (s->fp64) {
         if (s->fused64_ok)
-            for (int t = 0; t < fused64_tile_count(); ++t) cands.push_back(2 + t);
+            for (int t = 0; t < fused64_tuned_count(); ++t) cands.push_back(2 + t);
         return autotune_impl<double>(s, cands, n, ms_out, max, count);
     }
     if (s->fused_ok)

@@ -13,12 +13,24 @@ template void launch_diagnostics<double>(const Fields<double>&, const BCDesc<dou
                                          double*, double*, int, double*, hipStream_t);
 template void launch_order_director<double>(const Fields<double>&, long, long, double*, double*, hipStream_t);
 
-// FP64 tile catalogue of the fused step (fused64_kernel).
-constexpr const char* kTiles64[] = {"fp64:32x8", "fp64:16x16"};
+// FP64 tile catalogue of the fused step (fused64_kernel): the two column shapes
+// with chunk_planes' chunk length, which are what tuning chooses from, then the
+// same with a fixed length. Callers that hold a schedule number keep one: the
+// catalogue had seven entries before these shapes replaced the first pipeline's.
+struct Tile64 {
+    bool wide;     // 32x8 columns, else 16x16
+    int planes;    // length of the z chunks; 0: by chunk_planes
+    const char* name;
+};
+constexpr Tile64 kTiles64[] = {
+    {true, 0, "fp64:32x8"},       {false, 0, "fp64:16x16"},       {false, 64, "fp64:16x16x64"}, {false, 32, "fp64:16x16x32"},
+    {true, 64, "fp64:32x8x64"},   {true, 128, "fp64:32x8x128"},   {true, 32, "fp64:32x8x32"},
+};
 constexpr int kNumTiles64 = sizeof(kTiles64) / sizeof(kTiles64[0]);
 
 int fused64_tile_count() { return kNumTiles64; }
-const char* fused64_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles64) ? kTiles64[tile] : "?"; }
+int fused64_tuned_count() { return 2; }
+const char* fused64_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles64) ? kTiles64[tile].name : "?"; }
 
 // Length of the z chunks of a grid of `columns` column tiles: a chunk costs its
 // planes and two more, and the chunks run in rounds of two blocks per CU, so
@@ -47,10 +59,10 @@ static int chunk_planes(int columns, int nz) {
 }
 
 template <int TX, int TY>
-static void launch_tile64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int pull,
-                          int aux, hipStream_t s) {
+static void launch_tile64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int planes,
+                          int pull, int aux, hipStream_t s) {
     const int ntx = (bc.n[0] + TX - 1) / TX, nty = (bc.n[1] + TY - 1) / TY;
-    const int zc = chunk_planes(ntx * nty, bc.n[2]), nzc = (bc.n[2] + zc - 1) / zc;
+    const int zc = planes ? std::min(planes, bc.n[2]) : chunk_planes(ntx * nty, bc.n[2]), nzc = (bc.n[2] + zc - 1) / zc;
     const int grid = (ntx * nty * nzc + 7) / 8 * 8;
     bool walls = false;
     for (int face = 0; face < 6; ++face)
@@ -84,7 +96,8 @@ static void launch_tile64(const Fields<double>& f, const BCDesc<double>& bc, con
 
 void launch_fused_step_f64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int tile,
                            int pull, int aux, hipStream_t s) {
-    if (tile == 0) launch_tile64<32, 8>(f, bc, k, pull, aux, s);
-    else launch_tile64<16, 16>(f, bc, k, pull, aux, s);
+    const Tile64& t = kTiles64[tile];
+    if (t.wide) launch_tile64<32, 8>(f, bc, k, t.planes, pull, aux, s);
+    else launch_tile64<16, 16>(f, bc, k, t.planes, pull, aux, s);
 }
 }  // namespace lbm

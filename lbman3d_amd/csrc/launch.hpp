@@ -48,6 +48,7 @@ void launch_fused_step_f32(const Fields<float>& f, const BCDesc<float>& bc, cons
 // passes; its results are those of launch_qstep + launch_force_lbm bit for bit
 // (requires 15 * vs * 8 < 2^32).
 int fused64_tile_count();
+int fused64_tuned_count();   // of these, the first ones are what tuning times
 const char* fused64_tile_name(int tile);
 void launch_fused_step_f64(const Fields<double>& f, const BCDesc<double>& bc, const Phys<double>& k, int tile,
                            int pull, int store_aux, hipStream_t s);
