@@ -221,18 +221,18 @@ __device__ __forceinline__ void stage_a(const BCDesc<T>& bc, const Phys<T>& k,
         settle(r.advc[m]);
         if constexpr (sizeof(T) == 8) asm volatile("" ::: "memory");   // the next component's LDS reads stay below
     }
-    q_finish(k, Q, r, out.ta, fe, [&](int m, T qn, T sg) {
-        out.qn[m] = qn;
+    q_finish(k, Q, r, out.ta, fe, [&](int m, T rate, T sg) {
+        out.qn[m] = Q[m] + k.dt * rate;
         out.sg[m] = sg;
     });
 }
 
 // Register-lean form of the Q update for the FP32 fused kernels: the same
-// formulas as q_pointwise (src/model.h:102-342), evaluated component by
+// formulas as q_rates to q_finish (src/model.h:102-342), evaluated component by
 // component so that the 35 stencil derivatives are never live together.
-// Operand order inside each formula follows q_pointwise; the Ericksen force
+// Operand order inside each formula follows those; the Ericksen force
 // is accumulated per component (a different summation order, within FP32
-// rounding of q_pointwise).
+// rounding of theirs).
 // GH: 1 every face periodic (no ghosts), 0 the general ghost rules, 2 walls
 // on x and y faces only (Neumann Q; no-slip or specular velocity; z periodic).
 template <int GH, bool UPWIND, typename G>

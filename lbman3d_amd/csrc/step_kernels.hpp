@@ -181,7 +181,7 @@ __device__ __forceinline__ bool on_wall(const int pos[3], const int n[3], const 
 //
 // The stresses handed to the force kernel are Sigma and Tau in FP64. FP32
 // stores the eight independent components of the divergence form instead
-// (p_sets; zz = -xx - yy), in the same arrays: the force then needs 20
+// (stress_sets; zz = -xx - yy), in the same arrays: the force then needs 20
 // neighbour values rather than 52 and no Q^{n+1} (force kernel at 97x75x113:
 // 31.1 -> 26.3 us, at 256^3: 727 -> 557 us; FP64 keeps the reference's bits).
 //
@@ -241,12 +241,9 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
     }
     T ta[3], fe[3];
     if constexpr (sizeof(T) == 4) {
-        T qn[5], sg[5], pxy[6], pz[3];
-        q_finish(k, Q, r, ta, fe, [&](int c, T qc, T sc) {
-            qn[c] = qc;
-            sg[c] = sc;
-        });
-        p_sets(k.alpha, qn, sg, ta, pxy, pz);
+        T rate[5], pxy[6], pz[2];
+        q_finish(k, Q, r, ta, fe, [&](int c, T rc, T) { rate[c] = rc; });
+        stress_sets(k, Q, r.H, rate, pxy, pz);
 #pragma unroll
         for (int m = 0; m < 5; ++m) stn<NT>(f.sig[m], p.c, pxy[m]);
         stn<NT>(f.tau[0], p.c, pxy[5]);
@@ -254,12 +251,12 @@ __device__ __forceinline__ void qstep_cell(const Fields<T>& f, const BCDesc<T>& 
         stn<NT>(f.tau[2], p.c, pz[1]);
         if (own) {
 #pragma unroll
-            for (int m = 0; m < 5; ++m) stn<NT>(f.qn[m], p.c, qn[m]);
+            for (int m = 0; m < 5; ++m) stn<NT>(f.qn[m], p.c, Q[m] + k.dt * rate[m]);
         }
     } else {
-        q_finish(k, Q, r, ta, fe, [&](int c, T qc, T sc) {
+        q_finish(k, Q, r, ta, fe, [&](int c, T rate, T sc) {
             stn<NT>(f.sig[c], p.c, sc);
-            if (own) stn<NT>(f.qn[c], p.c, qc);
+            if (own) stn<NT>(f.qn[c], p.c, Q[c] + k.dt * rate);
         });
 #pragma unroll
         for (int m = 0; m < 3; ++m) stn<NT>(f.tau[m], p.c, ta[m]);
