@@ -195,13 +195,11 @@ BCDesc<T> make_bc(const lbm_config& c) {
     b.n[0] = c.nx;
     b.n[1] = c.ny;
     b.n[2] = c.nz;
-    b.all_periodic_u = 1;
     // FP32 runs store shifted populations and rho - rho0; FP64 stores rho.
     b.rho_base = sizeof(T) == 4 ? (T)c.p.density : T(0);
     for (int f = 0; f < 6; ++f) {
         b.qkind[f] = c.walls[f].qbc;
         b.ukind[f] = c.walls[f].ubc;
-        if (c.walls[f].ubc != LBM_U_PERIODIC) b.all_periodic_u = 0;
         double a[5];
         anchored_q_host(c.walls[f], a);
         for (int k = 0; k < 5; ++k) b.anchor[f][k] = (T)a[k];

@@ -95,7 +95,6 @@ struct BCDesc {
     int ukind[6];        // per face LBM_U_*
     T anchor[6][5];      // strong-anchoring Q per face (xx, xy, xz, yy, yz)
     T wall_u[6][3];      // wall velocity per face (MovingWall; zero otherwise)
-    int all_periodic_u;  // every velocity face periodic: no wall slots anywhere
     int q_ghosts;        // some axis has a wall whose ghost Q differs from what the stress stencil
                          // reads beyond it: anchoring, or a periodic high face opposite a wall
     int slots_xy;        // every reachable class has the slot row of its x, y

@@ -42,14 +42,14 @@ __device__ __forceinline__ void sto_hint(T* base, unsigned boff, T v) {
 }
 
 // Pull gather with 32-bit byte offsets (fused kernels; requires
-// 15 * vs * sizeof(T) < 2^32).
-template <bool PERIODIC, typename T>
-__device__ __forceinline__ void gather32(const Fields<T>& f, const BCDesc<T>& bc, int x, int y, int z,
-                                         unsigned c, int pull, T out[kQ]) {
-    constexpr unsigned E = sizeof(T);
+// 15 * vs * sizeof(float) < 2^32).
+template <bool PERIODIC>
+__device__ __forceinline__ void gather32(const Fields<float>& f, const BCDesc<float>& bc, int x, int y, int z,
+                                         unsigned c, int pull, float out[kQ]) {
+    constexpr unsigned E = sizeof(float);
     const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
     const unsigned vs4 = (unsigned)f.vs * E;
-    const T* g = f.g;
+    const float* g = f.g;
     if (!pull) {
 #pragma unroll
         for (int j = 0; j < kQ; ++j) out[j] = ldo(g, j * vs4 + c * E);
@@ -69,7 +69,7 @@ __device__ __forceinline__ void gather32(const Fields<T>& f, const BCDesc<T>& bc
         return;
     }
     const uint16_t* row = f.slots + cls * kSlotRow;
-    T rho_prev = T(0);
+    float rho_prev = 0.0f;
     bool have_rho = false;
 #pragma unroll
     for (int j = 0; j < kQ; ++j) {
@@ -86,9 +86,9 @@ __device__ __forceinline__ void gather32(const Fields<T>& f, const BCDesc<T>& bc
         } else {
             const int face = slot_face(e);
             if (!have_rho) { rho_prev = bc.rho_base + ldo(f.rho, c * E); have_rho = true; }
-            const T dot = T(cx(j)) * bc.wall_u[face][0] + T(cy(j)) * bc.wall_u[face][1]
-                        + T(cz(j)) * bc.wall_u[face][2];
-            out[j] = ldo(g, slot_src(e) * vs4 + c * E) + T(6.0) * rho_prev * T(wgt(j)) * dot;
+            const float dot = float(cx(j)) * bc.wall_u[face][0] + float(cy(j)) * bc.wall_u[face][1]
+                        + float(cz(j)) * bc.wall_u[face][2];
+            out[j] = ldo(g, slot_src(e) * vs4 + c * E) + 6.0f * rho_prev * float(wgt(j)) * dot;
         }
     }
 }
@@ -176,10 +176,9 @@ using StageA = StageAT<float>;
 constexpr int kNumIn = 8;    // Q (5) + u (3)
 constexpr int kNumA = 13;    // Q^{n+1} (5) + Sigma (5) + Tau (3)
 
-template <typename T>
-__device__ __forceinline__ void load_column(const Fields<T>& f, int qcol, int ucol_xy, unsigned qplane,
-                                            unsigned uplane, T v[kNumIn]) {
-    constexpr unsigned E = sizeof(T);
+__device__ __forceinline__ void load_column(const Fields<float>& f, int qcol, int ucol_xy, unsigned qplane,
+                                            unsigned uplane, float v[kNumIn]) {
+    constexpr unsigned E = sizeof(float);
     const unsigned qo = (qplane + (unsigned)qcol) * E, uo = (uplane + (unsigned)ucol_xy) * E;
 #pragma unroll
     for (int m = 0; m < 5; ++m) v[m] = ldo(f.q[m], qo);
@@ -426,13 +425,13 @@ __device__ __forceinline__ CellMask cell_mask(const BCDesc<T>& bc, int mode, int
 // column tile (tx, ty), writing the cells that `mode` selects. LDS buffers
 // come from the calling kernel so that a kernel instantiating several
 // variants does not allocate LDS per variant.
-template <int TX, int TY, int ZC, bool PERIODIC, typename T>
-__device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& bc, const Phys<T>& k,
+template <int TX, int TY, int ZC, bool PERIODIC>
+__device__ __forceinline__ void fused_body(const Fields<float>& f, const BCDesc<float>& bc, const Phys<float>& k,
                                            int pull, int aux, int tx, int ty, int tz,
-                                           T (*sIn)[TileGeom<TX, TY>::NI],
-                                           T (*sA)[kNumA][TileGeom<TX, TY>::NA],
-                                           T (*sRing)[kNumIn][TileGeom<TX, TY>::NR], int mode = 0) {
-    constexpr unsigned E = sizeof(T);
+                                           float (*sIn)[TileGeom<TX, TY>::NI],
+                                           float (*sA)[kNumA][TileGeom<TX, TY>::NA],
+                                           float (*sRing)[kNumIn][TileGeom<TX, TY>::NR], int mode = 0) {
+    constexpr unsigned E = sizeof(float);
     using G = TileGeom<TX, TY>;
     const int nx = bc.n[0], ny = bc.n[1], nz = bc.n[2];
     const int x0 = tx * TX, y0 = ty * TY;
@@ -487,12 +486,12 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     // Input history of the interior column in iteration pa: planes pa-1, pa,
     // pa+1 (registers); the next plane, pa + 2, is loaded one iteration ahead
     // of its use and joins the history at the start of the next iteration.
-    T hin[3][kNumIn], hnext[kNumIn];
+    float hin[3][kNumIn], hnext[kNumIn];
     load_column(f, qc0, uc0, qplane(z0 - 2), uplane(z0 - 2), hin[1]);
     load_column(f, qc0, uc0, qplane(z0 - 1), uplane(z0 - 1), hin[2]);
     load_column(f, qc0, uc0, qplane(z0), uplane(z0), hnext);
     if (has_ring) {
-        T v[kNumIn];
+        float v[kNumIn];
         load_column(f, qcr, ucr, qplane(z0 - 2), uplane(z0 - 2), v);
 #pragma unroll
         for (int m = 0; m < kNumIn; ++m) sRing[(z0 - 2 + 6) % 3][m][t] = v[m];
@@ -502,9 +501,9 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     }
     // Ring and outer-ring inputs are loaded one plane ahead of their LDS
     // store: ring plane pa + 1 and outer plane pa arrive in iteration pa.
-    T rnext[kNumIn], onext[kNumIn];
+    float rnext[kNumIn], onext[kNumIn];
     if (has_ring) load_column(f, qcr, ucr, qplane(z0), uplane(z0), rnext);
-    auto load_outer = [&](int z, T* v) {
+    auto load_outer = [&](int z, float* v) {
         const unsigned qo = (qplane(z) + (unsigned)oqc) * E, uo = (uplane(z) + (unsigned)ouc) * E;
 #pragma unroll
         for (int m = 0; m < 5; ++m) v[m] = ldo(f.q[m], qo);
@@ -516,10 +515,10 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     // z-difference values of the interior column's stage A at plane pa - 2
     // (the lower z neighbour of the plane finished in step 3), and the
     // Ericksen force of the interior column for planes pa - 1 and pa.
-    T dz_back[kNumDZ];
+    float dz_back[kNumDZ];
 #pragma unroll
-    for (int m = 0; m < kNumDZ; ++m) dz_back[m] = T(0);
-    T fe_prev[3] = {0, 0, 0}, fe_cur[3] = {0, 0, 0};
+    for (int m = 0; m < kNumDZ; ++m) dz_back[m] = 0.0f;
+    float fe_prev[3] = {0, 0, 0}, fe_cur[3] = {0, 0, 0};
 
     for (int pa = z0 - 1; pa <= z1; ++pa) {
         const int pb = pa - 1;
@@ -540,7 +539,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
         // update. (The moving-wall term reads rho of the own cell, which only
         // this thread writes, after the collision below.)
         const unsigned cpb = (unsigned)pb * plane + (unsigned)gy * nx + gx;
-        T pop[kQ];
+        float pop[kQ];
         if (do_b) gather32<PERIODIC>(f, bc, gx, gy, pb, cpb, pull, pop);
         {
             const int cc = (ib + 1) * G::IX + ia + 1;
@@ -568,7 +567,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
         // ---- step 2: Q update (stage A) at plane pa ----
         const int par = (pa + 2) & 1;
         const int zq = map_coord(pa, nz, ax[2].qlo, ax[2].qhi), zu = map_coord(pa, nz, ax[2].ulo, ax[2].uhi);
-        T dz_fwd[kNumDZ];
+        float dz_fwd[kNumDZ];
         fe_prev[0] = fe_cur[0];
         fe_prev[1] = fe_cur[1];
         fe_prev[2] = fe_cur[2];
@@ -577,7 +576,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
         // the Q-update code serves both.
 #pragma unroll 1
         for (int slot = 0; slot < (has_ring ? 2 : 1); ++slot) {
-            T zm[kNumIn], c[kNumIn], zp[kNumIn];
+            float zm[kNumIn], c[kNumIn], zp[kNumIn];
             int qpos[3], upos[3], ci, cj, acol;
             if (slot == 0) {
 #pragma unroll
@@ -600,8 +599,8 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
             }
             qpos[2] = zq;
             upos[2] = zu;
-            StageAT<T> a;
-            T fe[3];
+            StageA a;
+            float fe[3];
             stage_a<TX, TY, PERIODIC>(bc, k, sIn, (cj + 1) * G::IX + ci + 1, zm, c, zp, qpos, upos, a, fe);
 #pragma unroll
             for (int m = 0; m < kNumA; ++m) sA[par][m][acol] = stage_value(a, m);
@@ -617,7 +616,7 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
         __syncthreads();
 
         // ---- step 3: force + collide-stream at plane pb = pa - 1 ----
-        const T* A0 = &sA[(pb + 2) & 1][0][0];
+        const float* A0 = &sA[(pb + 2) & 1][0][0];
         auto A = [&](int m, int col) { return A0[m * G::NA + col]; };
         if (do_b) {
             // Neighbour columns with the reference's fetch rule: where a
@@ -628,34 +627,34 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
             const int lyp = (qy0 == ny - 1 && !ax[1].qhi) ? acell : acell + G::AX;
             const bool zm_self = (pb == 0 && !ax[2].qlo);
             const bool zp_self = (pb == nz - 1 && !ax[2].qhi);
-            auto zmv = [&](int m) -> T {
+            auto zmv = [&](int m) -> float {
                 const int sl = dz_slot(m);
                 return (zm_self || sl < 0) ? A(m, acell) : dz_back[sl];
             };
-            auto zpv = [&](int m) -> T {
+            auto zpv = [&](int m) -> float {
                 const int sl = dz_slot(m);
                 return (zp_self || sl < 0) ? A(m, acell) : dz_fwd[sl];
             };
             const int pos[3] = {qx0, qy0, pb};
-            T qc[5], dQ[5][3];
+            float qc[5], dQ[5][3];
 #pragma unroll
             for (int m = 0; m < 5; ++m) {
                 qc[m] = A(m, acell);
-                const Deriv<T> d = q_deriv<T, PERIODIC>(bc, m, pos, qc[m], A(m, lxm), A(m, lxp), A(m, lym), A(m, lyp),
+                const Deriv<float> d = q_deriv<float, PERIODIC>(bc, m, pos, qc[m], A(m, lxm), A(m, lxp), A(m, lym), A(m, lyp),
                                                zmv(m), zpv(m));
                 dQ[m][0] = d.d[0];
                 dQ[m][1] = d.d[1];
                 dQ[m][2] = d.d[2];
             }
-            T dS[8][3];
+            float dS[8][3];
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
-                dS[m][0] = (A(5 + m, lxp) - A(5 + m, lxm)) / T(2.0);
-                dS[m][1] = (A(5 + m, lyp) - A(5 + m, lym)) / T(2.0);
-                dS[m][2] = (zpv(5 + m) - zmv(5 + m)) / T(2.0);
+                dS[m][0] = (A(5 + m, lxp) - A(5 + m, lxm)) / 2.0f;
+                dS[m][1] = (A(5 + m, lyp) - A(5 + m, lym)) / 2.0f;
+                dS[m][2] = (zpv(5 + m) - zmv(5 + m)) / 2.0f;
             }
-            const T uo[3] = {hin[0][5], hin[0][6], hin[0][7]};   // u^{n-1} at (gx, gy, pb)
-            T F[3];
+            const float uo[3] = {hin[0][5], hin[0][6], hin[0][7]};   // u^{n-1} at (gx, gy, pb)
+            float F[3];
             if (k.force_full) {
                 body_force(k, dQ, dS, uo, fe_prev, F);
             } else {
@@ -663,11 +662,9 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
                 F[1] = fe_prev[1];
                 F[2] = fe_prev[2];
             }
-            // Density in its stored form: rho - rho0 for the shifted FP32
-            // populations, rho for FP64.
-            T drho, u[3];
-            if constexpr (sizeof(T) == 4) collide_shifted(k, pop, F, drho, u);
-            else collide_plain(k, pop, F, drho, u);
+            // Density in its stored form, rho - rho0.
+            float drho, u[3];
+            collide_shifted(k, pop, F, drho, u);
             const unsigned vs4 = (unsigned)f.vs * E, c4 = cpb * E;
             if (wmask.writes(pb)) {
 #pragma unroll
@@ -691,14 +688,14 @@ __device__ __forceinline__ void fused_body(const Fields<T>& f, const BCDesc<T>& 
     }
 }
 
-template <int TX, int TY, int ZC, bool PERIODIC, typename T = float>
+template <int TX, int TY, int ZC, bool PERIODIC>
 __global__ void __launch_bounds__(TX * TY)
-fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int ntx, int nty,
+fused_step_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull, int aux, int ntx, int nty,
                   int nzc, int mode) {
     using G = TileGeom<TX, TY>;
-    __shared__ T sIn[kNumIn][G::NI];          // input plane pa, extended region
-    __shared__ T sA[2][kNumA][G::NA];         // stage-A results, planes pa and pa - 1
-    __shared__ T sRing[3][kNumIn][G::NR];     // input history of the stage-A ring columns
+    __shared__ float sIn[kNumIn][G::NI];          // input plane pa, extended region
+    __shared__ float sA[2][kNumA][G::NA];         // stage-A results, planes pa and pa - 1
+    __shared__ float sRing[3][kNumIn][G::NR];     // input history of the stage-A ring columns
     // XCD-aware block order: hardware deals consecutive block ids round-robin
     // over the 8 XCDs; renumber so each XCD gets a contiguous run of tiles
     // (neighbouring tiles share halos in that XCD's L2).
@@ -707,7 +704,7 @@ fused_step_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, int pull, int aux, int n
     const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (L >= nblk) return;
     const int tx = L % ntx, ty = (L / ntx) % nty, tz = L / (ntx * nty);
-    fused_body<TX, TY, ZC, PERIODIC, T>(f, bc, k, pull, aux, tx, ty, tz, sIn, sA, sRing, mode);
+    fused_body<TX, TY, ZC, PERIODIC>(f, bc, k, pull, aux, tx, ty, tz, sIn, sA, sRing, mode);
 }
 
 // The FP64 step. The arithmetic is the unfused kernels' (stage_a, body_force,

@@ -45,7 +45,8 @@ __device__ __forceinline__ void q_pair(const BCDesc<T>& bc, int a, int c, int i,
 
 // QGradientAndLaplacian for one component from its seven stencil values
 // (src/boundary_handler.h:287-320).
-// NOGHOST: every face periodic, so the fetched neighbours are used as they are.
+// NOGHOST: the neighbours are used as they are passed (every face periodic, a
+// clamped value that is the ghost, or ghosts already in their place).
 template <typename T, bool NOGHOST = false>
 __device__ __forceinline__ Deriv<T> q_deriv(const BCDesc<T>& bc, int c, const int pos[3], T q0,
                                             T xm, T xp, T ym, T yp, T zm, T zp) {
