@@ -260,7 +260,14 @@ namespace {
 // 64 MiB apart and the 46 streams of the fused step ran 4-5% slower.)
 constexpr long kStagger = 64;
 
-// Cells from which a walled FP64 grid has the fused schedules.
+// Cells from which a walled FP64 grid has the fused schedules, which tuning
+// then times against the two-kernel step. The shell passes are a larger part
+// of a smaller grid, and the two-kernel step gains from the caches while an
+// array fits 9 MB. Two-kernel / 32x8 tiles with shells, us, walls in x and y and
+// then in z alone: 64^3 34.7/77 and 35/62, 96^3 127/159 and 127/121, 128x80x96
+// 139/165 and 141/129, 101^3 149/204 and 154/174, 128x100x90 169/191 and 169/153,
+// 128^3 300/301 and 301/228, 256x128x128 587/496 and 593/418. Below the line
+// only walls in z on rows of whole 64-byte pieces would gain, by up to 8 %.
 constexpr long kFused64Walls = 1L << 20;
 
 template <typename T>

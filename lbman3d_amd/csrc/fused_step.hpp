@@ -727,7 +727,7 @@ fused_step_kernel(Fields<float> f, BCDesc<float> bc, Phys<float> k, int pull, in
 // are stored for class-0 cells alone.
 //
 // 256^3 on 32x8 tiles: 2.14 ms for the first pipeline's best tile, 1.56 ms
-// here; 128^3 0.244 -> 0.213 ms. What it must not do is spill: with every halo
+// here; 128^3 0.244 -> 0.20 ms. What it must not do is spill: with every halo
 // load issued unconditionally (14 registers more) the prefetched values went
 // to scratch as they arrived and the step took 2.05 ms. NT: non-temporal
 // stores (see launch_tile64).

@@ -185,13 +185,15 @@ __device__ __forceinline__ bool on_wall(const int pos[3], const int n[3], const 
 // neighbour values rather than 52 and no Q^{n+1} (force kernel at 97x75x113:
 // 31.1 -> 26.3 us, at 256^3: 727 -> 557 us; FP64 keeps the reference's bits).
 //
-// Every load is issued before the first use, and the ghosts are selects: with
-// a branch per component and axis (uniform, but a branch) the loads of each
-// component waited for the arithmetic of the one before, eight memory
-// latencies in a row. Bound by latency on small grids and by the caches on
-// large ones. With force_lbm_cell, a step of the two kernels went from 23.7
-// to 14.4 us at 32^3 FP64, 48.6 to 36.4 us (FP64) and 30.7 to 19.0 us (FP32)
-// on a 20x100x100 channel, and 2.82 to 2.56 ms at 256^3 FP64.
+// Every load is issued before the first use, and the ghosts are patched after
+// the loads under a branch that only wavefronts with a cell on a wall take
+// (q_ghosts): with a branch per component and axis the loads of each component
+// waited for the arithmetic of the one before, eight memory latencies in a
+// row. Bound by latency on small grids and by the caches on large ones. With
+// force_lbm_cell and the block orders of CellGrid, a step of the two kernels
+// went from 23.7 to 9.9 us at 32^3 FP64, 48.6 to 29.7 us (FP64) and 30.6 to 14.9
+// us (FP32) on a 20x100x100 channel, 400 to 287 us on a 150x130x100 FP64 channel
+// and 2.82 to 2.41 ms at 256^3 FP64.
 template <typename T>
 __device__ __forceinline__ void settle(T& x) {
     if constexpr (sizeof(T) == 8) asm volatile("" : "+v"(x));
