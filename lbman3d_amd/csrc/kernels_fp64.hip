@@ -35,9 +35,11 @@ const char* fused64_tile_name(int tile) { return (tile >= 0 && tile < kNumTiles6
 // Length of the z chunks of a grid of `columns` column tiles: a chunk costs its
 // planes and two more, and the chunks run in rounds of two blocks per CU, so
 // that one block too many costs a whole round (150x130x100 on 32x8 tiles: 595
-// chunks of 16 planes in two rounds, 329 us; 510 of 17 in one, 270 us). Chunks
-// longer than 64 planes drift apart and share less in the L2 (256^3: 1.56 ms
-// with 64 planes, 1.64 ms with 128).
+// chunks of 16 planes in two rounds, 329 us; 510 of 17 in one, 270 us). Of 32,
+// 64 and 128 planes for every grid, no one comes within 5 % of this choice
+// everywhere (192^3: 664 us here, 741, 708 and 1262; 224x224x200: 942, 1072, 1357
+// and 1357). The limit of 64 costs up to 1 % where longer chunks would fill
+// their rounds as well (256^3: 1.555 ms with 64 planes, 1.54 with 128).
 static int chunk_planes(int columns, int nz) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess)
