@@ -289,9 +289,8 @@ __device__ __forceinline__ void p_sets(T alpha, const T q[5], const T sg[5], con
 // Relative to differences of Sigma, Tau and Q^{n+1} each rounded to 32 bits, the
 // force's L2 error is then 2 to 14 % smaller on smooth states and 2 to 17 % on
 // random directors; with sets summed in 32 bits it was up to 9 % larger on
-// smooth states. The Q kernel goes from 62..73 to 103..117 VGPRs for it: steps
-// of 97x75x113 43.1 -> 43.4 us, 20x100x100 14.6 -> 14.9, 256^3 1009 -> 1016 (held
-// to 79 VGPRs: 43.2, 14.7, 1017).
+// smooth states. Steps: 20x100x100 14.5 -> 14.7 us, 97x75x113 43.0 -> 43.1, 64^3
+// 15.0 -> 15.1, 256^3 1009 -> 1016.
 __device__ __forceinline__ void stress_sets(const Phys<float>& k, const float Qf[5], const float Hf[5],
                                             const float rate[5], float pxy[6], float pz[2]) {
     const double Qxx = Qf[0], Qxy = Qf[1], Qxz = Qf[2], Qyy = Qf[3], Qyz = Qf[4];

@@ -191,7 +191,7 @@ __device__ __forceinline__ bool on_wall(const int pos[3], const int n[3], const 
 // waited for the arithmetic of the one before, eight memory latencies in a
 // row. Bound by latency on small grids and by the caches on large ones. With
 // force_lbm_cell and the block orders of CellGrid, a step of the two kernels
-// went from 23.7 to 9.9 us at 32^3 FP64, 48.6 to 29.7 us (FP64) and 30.6 to 14.9
+// went from 23.7 to 9.9 us at 32^3 FP64, 48.6 to 29.7 us (FP64) and 30.6 to 14.7
 // us (FP32) on a 20x100x100 channel, 400 to 287 us on a 150x130x100 FP64 channel
 // and 2.82 to 2.41 ms at 256^3 FP64.
 template <typename T>
@@ -316,8 +316,13 @@ __device__ __forceinline__ Node<Off> node_at(const CellGrid& g, unsigned c) {
     return {(int)(r - y * g.nx), (int)y, (int)z, (Off)c};
 }
 
+// The FP32 form with walls on small arrays is held to five wavefronts per SIMD:
+// left alone, the 64-bit sums of stress_sets (and the wall constants) take it from
+// 79 to 117 registers, and 20x100x100 from 14.7 to 14.9 us a step, 64^3 from 15.7
+// to 16.0. The other forms are even or slower so (128^3 periodic 121.9 -> 122.4).
 template <typename T, bool WALLS, bool NT, int ADV, typename Off>
-__global__ void __launch_bounds__(kBlock) qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg) {
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 && WALLS && !NT ? 5 : 0)
+qstep_kernel(Fields<T> f, BCDesc<T> bc, Phys<T> k, CellGrid cg) {
     k.advection = ADV;
     const unsigned c = thread_cell(cg);
     if (c >= cg.cells) return;
